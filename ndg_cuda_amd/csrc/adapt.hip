@@ -637,11 +637,14 @@ __global__ void __launch_bounds__(kThreads) order_place_kernel(const int32_t *__
 // different orders when it is the lower-numbered element's; a periodic mortar side owns its own
 // faces against its partner's trace, one per face on the side (two on a larger side), as the
 // reference's periodic ghosts give each end of the period its own faces.
-__device__ void side_roles(const LogicalMesh &L, int64_t t, bool &mortar, int &owned) {
+// An oblique periodic side (see kKindTrace) of full length and equal orders has a record but no
+// mortar face.
+__device__ void side_roles(const LogicalMesh &L, int64_t t, bool &mortar, bool &oblique, int &owned) {
     const int64_t k = t / 4, l = L.link[t];
     const int hk = L.hang[t];
     const bool other = l >= 0 && L.order[l / 4] != L.order[k];
     mortar = hk != 0 || other;
+    oblique = !mortar && L.periodic[t] == kPeriodicOblique;
     if (L.periodic[t]) owned = mortar ? (hk == 2 ? chain_length(L, t) : 1) : 0;
     else owned = hk == 1 || (hk == 0 && other && l / 4 > k);
 }
@@ -652,19 +655,25 @@ __global__ void __launch_bounds__(kThreads) side_count_kernel(LogicalMesh L, int
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     unsigned long long pairs = 0, hfaces = 0, pfaces = 0;
     if (t < 4 * L.K) {
-        bool mortar;
+        bool mortar, oblique;
         int owned;
-        side_roles(L, t, mortar, owned);
+        side_roles(L, t, mortar, oblique, owned);
         const int64_t k = t / 4, l = L.link[t];
         const int N = L.order[k], hk = L.hang[t];
         const bool per = L.periodic[t] != 0;
         const int n_faces = hk == 2 ? chain_length(L, t) : 1;
-        cnt_rec[t] = mortar;
+        cnt_rec[t] = mortar || oblique;
         cnt_slot[t] = mortar ? 3 * (int64_t)(N + 1) * n_faces : 0;
         cnt_face[t] = owned;
         pairs = l >= 0 && hk == 0 && !per && l > t;
         hfaces = hk == 2 && !per ? n_faces : 0;
         pfaces = per ? n_faces : 0;
+        if ((owned && hk != 2) || oblique) {  // the other side writes its three traces if it has a record
+            bool m, o;
+            int own;
+            side_roles(L, l, m, o, own);
+            if (!m && !o && L.link[l] >= 0) atomicAdd(&c->bare_partner, 1ull);
+        }
         if (owned) {
             int Nr = L.order[l / 4];
             if (hk == 2) {
@@ -728,16 +737,25 @@ __global__ void __launch_bounds__(kThreads) side_fill_kernel(LogicalMesh L, Fill
     const int64_t local = dv - G.e_begin;
     if (s == 0)
         for (int i = 0; i < 8; ++i) A.verts[8 * dv + i] = L.verts[8 * k + i];
-    bool mortar;
+    bool mortar, oblique;
     int owned;
-    side_roles(L, t, mortar, owned);
+    side_roles(L, t, mortar, oblique, owned);
+    const v2 c0 = corner(L, k, s), c1 = corner(L, k, s + 1);
     int64_t code;
-    if (mortar) {
+    if (mortar || oblique) {
         code = -(1 + A.n_ghost + A.rec_idx[t]);
         BcSide rec{};
-        rec.kind = kKindMortar;
-        rec.slot = A.slot_off[t];
-        rec.n_faces = hk == 2 ? chain_length(L, t) : 1;
+        face_frame(c0, c1, c0, c1, rec.nx, rec.ny, rec.tx, rec.ty);
+        if (mortar) {
+            rec.kind = kKindMortar;
+            rec.slot = A.slot_off[t];
+            rec.n_faces = hk == 2 ? chain_length(L, t) : 1;
+        } else {
+            const int64_t local_r = L.dev_of[l / 4] - G.e_begin;
+            rec.kind = kKindTrace;
+            rec.slot = local_r * 12 * nf + (l % 4) * 3 * nf;
+            rec.partner = local_r * 4 + l % 4;
+        }
         A.bc[A.n_ghost + A.rec_idx[t]] = rec;
     } else if (l < 0) {
         code = l;
@@ -753,7 +771,6 @@ __global__ void __launch_bounds__(kThreads) side_fill_kernel(LogicalMesh L, Fill
         const GroupSpan &S = A.spans[n - 1];
         return S.tr_off + (L.dev_of[e] - S.e_begin) * 12 * n + (side % 4) * 3 * n;
     };
-    const v2 c0 = corner(L, k, s), c1 = corner(L, k, s + 1);
     const v2 PL[4] = {corner(L, k, 0), corner(L, k, 1), corner(L, k, 2), corner(L, k, 3)};
     const double sfL = side_scale(PL, s);
     if (L.periodic[t]) {

@@ -54,7 +54,8 @@ constexpr int kAdjSource = 16;  // add the receivers' misfit source to lambda' b
 template <int N>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 10 ? 3 : 2)))
 adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
-                     const double *__restrict__ tab, double *__restrict__ lam, double *__restrict__ mu,
+                     const BcSide *__restrict__ bc, const double *__restrict__ tab, double *__restrict__ lam,
+                     double *__restrict__ mu,
                      const double *__restrict__ chi_in, double *__restrict__ chi_out,
                      const double *__restrict__ qs, double *__restrict__ cpart, int64_t K, int flags,
                      double gs, double as, double gnext, double cw, const int64_t *__restrict__ rec_elem,
@@ -90,14 +91,14 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
         nbv[it][0] = nbv[it][1] = nbv[it][2] = 0.0;
         const int item = tid + it * T;
         if (apply && item < nel * 4 * NF) {
-            const int32_t cd = side_nb[(e0 + item / NF / 4) * 4 + (item / NF) % 4];
+            int32_t cd = side_nb[(e0 + item / NF / 4) * 4 + (item / NF) % 4];
             const int k = item % NF;
-            if (cd >= 0) {  // the host admits interior and periodic sides only
-                const double *nb = chi_in + (int64_t)(cd >> 2) * 12 * NF + (cd & 3) * 3 * NF + (N - k);
-                nbv[it][0] = nb[0];
-                nbv[it][1] = nb[NF];
-                nbv[it][2] = nb[2 * NF];
-            }
+            // the host admits interior and periodic sides only: a record is an oblique periodic side's
+            if (cd < 0) cd = (int32_t)bc[-1 - cd].partner;
+            const double *nb = chi_in + (int64_t)(cd >> 2) * 12 * NF + (cd & 3) * 3 * NF + (N - k);
+            nbv[it][0] = nb[0];
+            nbv[it][1] = nb[NF];
+            nbv[it][2] = nb[2 * NF];
         }
     }
     double mreg[QPT], lreg[QPT], qreg[QPT];
@@ -381,19 +382,20 @@ record_kernel(const double *__restrict__ q, const int64_t *__restrict__ elem, co
 }
 
 // record_kernel on the RK register in the stage kernel's tile order: element e is element
-// el = e mod epb of its tile of nel elements, node (i, j) of field 0 at ((j nel + el)(N+1) + i).
+// el = e mod epb of its tile, node (i, j) of field 0 in the tile's runs of its line indices j, two by two.
 __global__ void __launch_bounds__(64)
 record_rk_kernel(const double *__restrict__ g, const int64_t *__restrict__ elem, const double *__restrict__ w_t,
-                 int nf, int64_t K, int epb, double *__restrict__ out) {
+                 int nf, int epb, int run, double *__restrict__ out) {
     const int r = blockIdx.x, ne = nf * nf;
-    const int64_t e = elem[r], e0 = e - e % epb;
-    const int el = (int)(e - e0), nel = (int)min<int64_t>(epb, K - e0);
-    const double *tile = g + e0 * 3 * ne;
+    const int64_t e = elem[r], blk = e / epb;
+    const int el = (int)(e - blk * epb);
+    const double *tile = g + blk * 3 * nf * run;
     const double *wr = w_t + (int64_t)r * ne;
     double acc = 0.0;
     for (int k = threadIdx.x; k < ne; k += 64) {
         const int j = k / nf, i = k % nf;
-        acc += wr[k] * tile[(j * nel + el) * nf + i];
+        const int at = el * nf + i;
+        acc += wr[k] * (j + 1 < nf || nf % 2 == 0 ? tile[(j & ~1) * run + 2 * at + (j & 1)] : tile[j * run + at]);
     }
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
     if (threadIdx.x == 0) out[r] = acc;
@@ -451,7 +453,7 @@ static hipError_t adjoint_n(DeviceMesh &m, const AdjointArgs &A, hipStream_t s) 
     using S = LineShape<N>;
     const Group &G = m.groups[0];
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    hipLaunchKernelGGL(adjoint_stage_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts, m.side_nb, G.tab,
+    hipLaunchKernelGGL(adjoint_stage_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts, m.side_nb, m.bc, G.tab,
                        A.lam, A.mu, A.chi_in, A.chi_out, A.qs, A.cpart, G.K, A.flags, A.gs, A.as, A.gnext,
                        m.wave_speed, A.rec_elem, A.rec_w, A.rec_res, A.n_rec);
     return hipGetLastError();
@@ -496,8 +498,8 @@ hipError_t launch_record(const DeviceMesh &m, const int64_t *elem, const double 
 hipError_t launch_record_rk(const DeviceMesh &m, const int64_t *elem, const double *w_t, int n, double *out,
                             hipStream_t s) {
     const Group &G = m.groups[0];
-    hipLaunchKernelGGL(record_rk_kernel, dim3(n), dim3(64), 0, s, m.g, elem, w_t, G.N + 1, G.K, stage_tile_epb(G),
-                       out);
+    hipLaunchKernelGGL(record_rk_kernel, dim3(n), dim3(64), 0, s, m.g, elem, w_t, G.N + 1, stage_tile_epb(G),
+                       stage_tile_run(G), out);
     return hipGetLastError();
 }
 

@@ -31,14 +31,32 @@ struct BcSide {
     int32_t kind;
     int32_t n_faces = 1;
     int64_t slot;
+    int64_t partner = -1;  // kKindTrace: the partner side, nb*4+side
 };
 
-// Stage kernel flags: the step's first stage (the RK register is not read) and its last stage.
-constexpr int kRkFirst = 1, kRkLast = 2;
+// Stage kernel flags: the step's first stage (the RK register is not read), its last stage, the
+// three traces written for every side (see DeviceMesh::trace_all), and the state and RK register
+// streamed past the caches (where together they have more than kStreamBytes).
+constexpr int kRkFirst = 1, kRkLast = 2, kTraceAll = 4, kStream = 8;
+constexpr int64_t kStreamBytes = int64_t(160) << 20;
 
 // Element side whose face is non-conforming: its element flux trace is produced by the mortar
 // kernel (interpolation to the face, flux, L2 projection back) before the stage kernels run.
 constexpr int32_t kKindMortar = 100;
+
+// Periodic side whose partner side does not run parallel to it: the partner's outgoing
+// characteristic is not this side's incoming one, so its three traces are read (`slot`: their
+// offset in the group's slice of the trace buffer).
+constexpr int32_t kKindTrace = 101;
+// Values of LogicalMesh::periodic (and the host topology's): no, yes, and such a side.
+constexpr int8_t kPeriodic = 1, kPeriodicOblique = 2;
+// Whether the side a0 -> a1 runs against the side b0 -> b1 (their normals are opposite) to rounding:
+// coordinates of size X carry errors of about 1e-16 X, so an edge of length len has a direction
+// good to 1e-16 X / len.
+__host__ __device__ inline bool opposite_sides(double ax, double ay, double bx, double by) {
+    const double la = sqrt(ax * ax + ay * ay), lb = sqrt(bx * bx + by * by);
+    return fabs(ax / la + bx / lb) <= 1e-12 && fabs(ay / la + by / lb) <= 1e-12;
+}
 
 // One non-conforming face (src/meshes/Mesh2D_t.cpp:3803-4006). L is the element
 // that created the face in the reference's face building, R the other element (or, for a periodic
@@ -94,11 +112,18 @@ __host__ __device__ inline int64_t mortar_matrix_key(int Ne, int Nf, int side, i
 constexpr int64_t kMortarMatrixKeys = (int64_t)(kMaxOrder + 1) * (kMaxOrder + 1) * 4 * kMortarClasses;
 
 // Per-order constant tables in device memory, packed as Dhat[Nf*Nf], l(-1)[Nf], l(+1)[Nf], w[Nf],
-// x[Nf], 1/w[Nf], then the modal matrix poly[Nf*Nf] used by the estimator and the transpose
-// Dhat^T[Nf*Nf] used by the adjoint (its columns as contiguous rows).
+// x[Nf], 1/w[Nf], then the modal matrix poly[Nf*Nf] used by the estimator, the transpose
+// Dhat^T[Nf*Nf] used by the adjoint (its columns as contiguous rows), and for the stage kernel
+// l(+1)/w[Nf] and the even and odd parts of Dhat (see contract in kernels.hip).
+__host__ __device__ constexpr int even_odd_len(int nf) {
+    return (nf / 2) * (2 * (nf / 2) + nf % 2) + (nf % 2) * (nf / 2);
+}
 inline int64_t table_pack_len(int N) {
     const int nf = N + 1;
-    return (int64_t)nf * nf * 3 + 5 * nf;
+    return (int64_t)nf * nf * 3 + 6 * nf + even_odd_len(nf);
+}
+__host__ __device__ constexpr int64_t table_stage_offset(int N) {
+    return (int64_t)(N + 1) * (N + 1) * 3 + 5 * (N + 1);
 }
 inline int64_t table_dhat_t_offset(int N) {
     const int nf = N + 1;
@@ -138,7 +163,7 @@ void arena_free(Arena &a);
 // The buffers of one device mesh. A mesh keeps two: the current one, and the one an adaptation
 // builds the next mesh into (the state is transferred from the first to the second).
 struct DeviceStore {
-    Arena verts, side_nb, bc, faces, side_flux, side_flux32, q, g, tr[2], rhs, scratch, qh, gl32, tr32[2];
+    Arena verts, side_nb, bc, faces, side_flux, side_flux32, q, g, tr[2], wave[2], rhs, scratch, qh, gl32, tr32[2];
     Arena spans;  // GroupSpan[kMaxOrder + 1] of the layout
 };
 void store_free(DeviceStore &s);
@@ -163,7 +188,9 @@ struct Group {
     int64_t K = 0;
     int64_t e_begin = 0;     // first element (device order)
     int64_t q_off = 0;       // offset (values) into q / g: 3 (N+1)^2 per element
-    int64_t tr_off = 0;      // offset (values) into the trace buffers: 12 (N+1) per element
+    int64_t tr_off = 0;      // offset (values) into the trace buffers: 12 (N+1) per element (a third
+                             // of it into the characteristics: 4 (N+1) per element)
+    int64_t g_off = 0;       // offset (values) into g: stage_rk_values(N, K)
     double *tab = nullptr;   // packed tables for N
     float *tab32 = nullptr;
     // Launch shape of the group's stage kernel per precision (index NDG_PRECISION_*): elements
@@ -181,10 +208,12 @@ struct DeviceMesh {
     int64_t K = 0;
     int N_min = 0, N_max = 0;
     int64_t n_q = 0, n_tr = 0;   // values per state buffer / trace buffer
+    int64_t n_g = 0;             // values of the RK register
     double *verts = nullptr;     // [K][4][2], device order
     int32_t *side_nb = nullptr;  // [K][4]: group-local nb*4+side (>=0) or -(1+bc index)
     BcSide *bc = nullptr;        // [n_bc]
     int64_t n_bc = 0;
+    int64_t n_ghost = 0;         // of these, the boundary ghosts (the others are mortar and oblique sides)
     MortarFace *faces = nullptr; // [n_faces]
     int64_t n_faces = 0;
     int mortar_nodes = 0;        // largest N + 1 over the faces' NL, NR and Nf (sizes the mortar LDS)
@@ -196,10 +225,14 @@ struct DeviceMesh {
     double *q = nullptr;
     double *g = nullptr;         // RK register (alive within a step; the stage kernel's tile order)
     double *trace[2] = {nullptr, nullptr};
+    double *wave[2] = {nullptr, nullptr};  // outgoing characteristics, [K][4][N+1]
+    // The stage kernels write the three traces of the sides with a record (boundary, mortar); of
+    // every side when a mortar face or an oblique periodic side reads a side without one.
+    bool trace_all = false;
     double *rhs = nullptr;       // compute_rhs only (allocated on demand)
     double *scratch = nullptr;   // reductions
     int64_t scratch_len = 0;
-    int cur = 0;                 // trace buffer holding the traces of the current state
+    int cur = 0;                 // trace and wave buffers holding those of the current state
     double *clock = nullptr;     // [4]: step start time, then the 3 stage times
     double *q_out = nullptr;     // when set, FP64 stage kernels write the new state here (not in q)
     bool has_inflow = false;     // the stage time is read only by inflow ghosts
@@ -260,6 +293,7 @@ struct AdaptCounts {
     unsigned long long conforming_pairs, mortar_nodes, bad_face;
     unsigned long long periodic_faces;           // faces of periodic sides (one per face on the side)
     unsigned long long hanging_faces;            // faces of interior larger sides
+    unsigned long long bare_partner;             // sides without a record whose three traces are read
 };
 // refused bits: a raised order beyond the tables, a face smaller than 1 / 2^kMaxSpanLevel of its side
 constexpr unsigned kRefuseOrder = 1, kRefuseSpan = 4;
@@ -361,8 +395,11 @@ hipError_t launch_record(const DeviceMesh &m, const int64_t *elem, const double 
 // tile order; w_t holds the weights in transposed node order (k = j (N+1) + i for node (i, j)).
 hipError_t launch_record_rk(const DeviceMesh &m, const int64_t *elem, const double *w_t, int n, double *out,
                             hipStream_t s);
-// Elements per workgroup tile of the FP64 stage kernel for group G (the RK register's tile order).
+// Elements per workgroup tile of the FP64 stage kernel for group G (the RK register's tile order),
+// the values of one (field, line index) run of a tile, and the register's size for K elements.
 int stage_tile_epb(const Group &G);
+int stage_tile_run(const Group &G);
+int64_t stage_rk_values(int N, int64_t K);
 hipError_t launch_source(double *lam, const DeviceMesh &m, const int64_t *elem, const double *w,
                          const double *res, int n, hipStream_t s);
 

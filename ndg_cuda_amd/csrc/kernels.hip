@@ -4,21 +4,25 @@
 //   q      [K][3][(N+1)^2]   state (p, u, v), reference node order i*(N+1)+j
 //   g      [K][3][(N+1)^2]   RK register, alive within a step only; the stage kernel's own order
 //                            within each workgroup tile (see stage_kernel)
-//   trace  [K][4][3][N+1]    element traces of the current state (two buffers, ping-pong)
+//   wave   [K][4][N+1]       outgoing characteristics at the side points of the current state (two
+//                            buffers, ping-pong)
+//   trace  [K][4][3][N+1]    element traces of the current state (two buffers), of the sides that
+//                            need all three (see stage_kernel)
 //   verts  [K][4][2]         element vertices (metrics are recomputed from them per node)
 //   side_nb[K][4]            neighbour element*4+side, or -(1+index) into the BcSide records
 //
 // One fused stage kernel replaces the reference's per-phase kernels of one stage
 // (include/solvers/Solver2D_t.tcu:45-52): a workgroup stages the (N+1)^2 tiles of EPB elements in
-// LDS, computes the upwind flux on its 4 sides from its own traces (recomputed from the LDS tile)
-// and the neighbours' traces (one HBM read), applies volume + lift, the RK update, and writes the
-// traces of the updated state for the next stage. Per element and stage HBM traffic is the state
-// and RK register (read + write), one read of the neighbours' traces and one write of its own.
+// LDS, computes the upwind flux on its 4 sides from its own and the neighbours' outgoing
+// characteristics, applies volume + lift, the RK update, and writes the characteristics of the
+// updated state for the next stage. Per element and stage HBM traffic is the state and RK register
+// (read + write), and the characteristics of its sides (one value a point, read and written).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "device.hpp"
 #include "internal.hpp"
@@ -42,6 +46,29 @@ __device__ __forceinline__ void plane_wave(double x, double y, double t, double 
     p = exp(-a * a / (d * d));
     u = p * kx;  // the reference's p k / c at c = 1 (and the plane wave of the speed-c system)
     v = p * ky;
+}
+
+// Outward normal of the edge P_s -> P_s+1 of vertices V; returns its Jacobian (src/entities/
+// Element2D_t.cpp:756-769), constant along a side of a bilinear element and half its length.
+__device__ __forceinline__ double side_geometry(const double *V, int s, double &nx, double &ny) {
+    const int s1 = (s + 1) & 3;
+    const double ex = V[2 * s1] - V[2 * s], ey = V[2 * s1 + 1] - V[2 * s + 1];
+    const double len = sqrt(ex * ex + ey * ey);
+    nx = ey / len;
+    ny = -(ex / len);
+    return len / 2;
+}
+
+// The outward normal that the characteristic of side s of element e is formed with: its record's,
+// where it has one.
+__device__ __forceinline__ void side_normal(const double *verts, const int32_t *side_nb, const BcSide *bc, int64_t e,
+                                            int s, double &nx, double &ny) {
+    side_geometry(verts + e * 8, s, nx, ny);
+    const int32_t cd = side_nb[e * 4 + s];
+    if (cd < 0) {
+        nx = bc[-1 - cd].nx;
+        ny = bc[-1 - cd].ny;
+    }
 }
 
 // Trace k of side s of one element tile (src/entities/Element2D_t.cpp:86-125): sides 2 and 3
@@ -68,30 +95,39 @@ __device__ __forceinline__ double side_trace(const double *tile, const double *l
 }
 
 // ---------------------------------------------------------------------------------------------
-// Traces of the current state (used after the state is set; the stage kernel writes them
-// afterwards).
+// Traces and outgoing characteristics (see stage_kernel) of the current state, used after the state
+// is set; the stage kernel writes them afterwards.
 template <int N>
 __global__ void __launch_bounds__(Shape<N>::THREADS)
-traces_kernel(const double *__restrict__ tab, const double *__restrict__ q,
-              double *__restrict__ tr, int64_t K) {
+traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb, const BcSide *__restrict__ bc,
+              const double *__restrict__ tab, const double *__restrict__ q, double *__restrict__ tr,
+              double *__restrict__ w, int64_t K) {
     using S = Shape<N>;
     constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::THREADS;
     __shared__ double s_lm[NF], s_lp[NF];
     __shared__ double s_q[EPB * 3 * NE];
+    __shared__ double s_n[EPB * 8];  // outward normal per side
     const int tid = threadIdx.x;
     const int64_t e0 = (int64_t)blockIdx.x * EPB;
     const int nel = (int)min<int64_t>(EPB, K - e0);
-    for (int r = tid; r < NF; r += T) {
-        s_lm[r] = tab[NF * NF + r];
+    for (int r = tid; r < NF; r += T) {  // l(-1) is the reverse of l(+1), as in the stage kernel
+        s_lm[r] = tab[NF * NF + NF + N - r];
         s_lp[r] = tab[NF * NF + NF + r];
     }
     const double *qg = q + e0 * 3 * NE;
     for (int r = tid; r < nel * 3 * NE; r += T) s_q[r] = qg[r];
+    for (int r = tid; r < nel * 4; r += T) side_normal(verts, side_nb, bc, e0 + r / 4, r % 4, s_n[2 * r], s_n[2 * r + 1]);
     __syncthreads();
-    for (int r = tid; r < nel * 12 * NF; r += T) {
-        const int el = r / (12 * NF), rs = r % (12 * NF);
-        const int s = rs / (3 * NF), f = (rs / NF) % 3, k = rs % NF;
-        tr[(e0 + el) * 12 * NF + rs] = side_trace<N>(s_q + el * 3 * NE + f * NE, s_lm, s_lp, s, k);
+    for (int r = tid; r < nel * 4 * NF; r += T) {
+        const int el = r / (4 * NF), s = (r / NF) % 4, k = r % NF;
+        const double *qe = s_q + el * 3 * NE;
+        const double p = side_trace<N>(qe, s_lm, s_lp, s, k), u = side_trace<N>(qe + NE, s_lm, s_lp, s, k),
+                     v = side_trace<N>(qe + 2 * NE, s_lm, s_lp, s, k);
+        double *to = tr + (e0 + el) * 12 * NF + s * 3 * NF + k;
+        to[0] = p;
+        to[NF] = u;
+        to[2 * NF] = v;
+        w[e0 * 4 * NF + r] = p + kWaveSpeed * (u * s_n[8 * el + 2 * s] + v * s_n[8 * el + 2 * s + 1]);
     }
 }
 
@@ -99,20 +135,46 @@ traces_kernel(const double *__restrict__ tab, const double *__restrict__ q,
 // One fused RK stage. A workgroup is three waves, one per field (p, u, v); lane (element e, line l)
 // of the wave for field f handles one (N+1)-point line of that field for EPB = floor(64/(N+1))
 // elements. Every field-dependent branch is therefore wave-uniform (a scalar branch, no masked
-// lanes), the D^ contractions run in registers with the D^ rows as wave-uniform scalar loads, and
-// LDS carries the element tiles:
+// lanes), the D^ contractions run in registers, and LDS carries the element tiles:
 //   P0  every HBM read of the tile is issued before any is waited on: state tile -> LDS, the
-//       thread's RK-register line and the neighbour traces of its flux points -> registers
-//   P1  the element's own traces (row l and column l of field f); wave 0 the metric lines along
-//       xi, wave 1 along eta, wave 2 the side normals and edge Jacobians
-//   P2  upwind flux at the 4(N+1) side points, times the edge Jacobian
-//       (boundary_conditions / project_to_faces / calculate_wave_fluxes / project_to_elements,
-//       Mesh2D_t.cpp:3731-3935, Solver2D_t.cpp:48-63)
-//   P3  xi lines: D^ (y_eta f - x_eta g) + lift (Solver2D_t.cpp:71-100)
-//   P4  eta lines: D^ (-y_xi f + x_xi g) + lift, G = (-d_xi - d_eta)/J (:104-133), RK update
-//       (Solver2D_t.cpp:138-172)
-//   P5  coalesced stores of q and g, traces of the updated state for the next stage.
-// RHS_ONLY writes G (the compute_dg_wave_derivative output) and leaves the state alone. rk_flags:
+//       thread's RK-register line, and for each side point the outgoing characteristics of the
+//       element and of its neighbour -> registers
+//   P1  D^ (y_eta f - x_eta g) along the thread's xi line (Solver2D_t.cpp:71-100) and
+//       D^ (-y_xi f + x_xi g) along its eta line (:104-133), both from the state tile; then the upwind
+//       flux of the side points (boundary_conditions / project_to_faces / calculate_wave_fluxes /
+//       project_to_elements, Mesh2D_t.cpp:3731-3935, Solver2D_t.cpp:48-63) and, by wave 2, the side
+//       normals and edge Jacobians
+//   P2  the lifts; d_xi to LDS
+//   P3  eta lines: G = (-d_xi - d_eta)/J, RK update (Solver2D_t.cpp:138-172), the new state to LDS,
+//       its traces on sides 0 and 2 from the line in registers
+//   P4  coalesced store of q, traces on sides 1 and 3 from the new tile's columns
+//   P5  the new outgoing characteristic of every side point, for the next stage.
+//
+// The upwind flux of a side point needs from the other element only the characteristic that leaves
+// it, w = p + u.n with its own outward normal n: on a side shared by two elements the normals are
+// opposite, so this is p - u.n in the receiver's normal. One value a point is exchanged instead of
+// the three traces: 4 (N+1) values an element are written once and read twice (the element's own
+// from the same tile) instead of 12 (N+1) written and read, 7,200 instead of 8,290 bytes an element
+// and stage at N = 8. Sides where that is not enough carry a record (code < 0): boundary ghosts are
+// built from the element's own traces, formed from the state tile; a mortar side's flux comes from
+// the mortar kernel; a periodic side whose partner does not run parallel to it reads the partner's
+// three traces. Elements write the three traces of the sides with a record (and with kTraceAll of
+// every side) for these.
+//
+// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 324 us a
+// launch, 5.8 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches 5.3 to 5.8
+// here); 421 us and 2.18 GB with the traces exchanged. 512 x 512, N = 4: 116 us (164 us before). 128 x
+// 128, N = 8 (in the last-level cache): 24.9 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
+// us from launch to launch, 7.0 us before. What made the difference, at N = 8:
+//  - the state and the RK register are streamed past the caches (non-temporal, in 16-byte words on
+//    whole 128-byte lines) where they are larger than these (stage_flags): 401 -> 324 us at 512 x 512;
+//  - D^ out of the scalar loads (LaneTable) and by even and odd parts (contract): 24.9 us instead of
+//    28 us at 128 x 128;
+//  - no branch inside the line loops and no wait among the loads (a condition on the field in a loop
+//    kept each LDS read from overlapping the next: 3,700 cycles for the update of a line, 1,700 now);
+//  - five barriers instead of six, LDS for five workgroups a CU instead of four.
+//
+// RHS_ONLY writes G (the compute_dg_wave_derivative output) and leaves the state alone. flags:
 // kRkFirst, the step's first stage (a = 0: the RK register is not read); kRkLast, the step's last
 // stage, whose RK register no one reads (the next step's first stage overwrites it), so it is not
 // stored.
@@ -121,40 +183,253 @@ traces_kernel(const double *__restrict__ tab, const double *__restrict__ q,
 // A workgroup takes epb <= EPB consecutive elements (fewer gives more workgroups for a small
 // order group); remap != 0 applies the XCD-contiguous block order. t_ptr points at the stage time
 // in device memory (the inflow ghost reads it), so that a captured step can be replayed.
+//
+// LDS at N = 8 is 31,920 bytes, which the 1,280-byte allocation steps still let fit five times into
+// a CU's 160 KB.
 
+// Values per (field, line index) of a workgroup tile in the RK register: whole 128-byte lines for
+// the full tiles, whole 16-byte words for the tuner's smaller ones.
+template <int N>
+__host__ __device__ constexpr int rk_run(int epb) {
+    return epb == LineShape<N>::EPB ? (LineShape<N>::EPB * (N + 1) + 15) / 16 * 16 : (epb * (N + 1) + 1) / 2 * 2;
+}
+
+// The state tile in LDS: [element][f][i][j] with the row stride padded to an odd number of values,
+// so that lanes on consecutive rows fall on different banks (at even N + 1 the unpadded rows of a
+// column of lanes share a few banks).
+template <int N>
+struct StageTile {
+    using S = LineShape<N>;
+    static constexpr int NFP = S::NF | 1;                       // padded row stride
+    static constexpr int NEP = S::NF * NFP;                     // one field of one element
+    static constexpr int kFlux = S::EPB * 8 * S::NF;            // (w_L - w_R)/2 and (w_L + w_R)/2 per side point
+    static constexpr int QPT = (S::EPB * 3 * S::NE + 15 + 2 * S::T - 1) / (2 * S::T);  // pairs per thread
+    // LDS index of value r of a tile in the state's order
+    __device__ static __forceinline__ int at(int r) { return NFP == S::NF ? r : r + (int)((unsigned)r / S::NF); }
+};
+
+// n values from p with the hardware's bounds check: a load outside [0, n) gives 0, a store outside it
+// is dropped, so a tile's loads and stores need no branch for its remainder.
+struct Buffer {
+    static constexpr int kNonTemporal = 2;  // the instruction's nt bit
+    __amdgpu_buffer_rsrc_t rsrc;
+    __device__ __forceinline__ Buffer(const double *p, int n)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc((void *)p, 0, n * 8, 0x00027000)) {}
+    __device__ __forceinline__ double load(int i) const {
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, i * 8, 0, 0));
+    }
+    // values i and i + 1, p + i on a 16-byte boundary; past the caches with kNonTemporal
+    template <int kHow>
+    __device__ __forceinline__ double2 load2(int i) const {
+        return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rsrc, i * 8, 0, kHow));
+    }
+    __device__ __forceinline__ void store(int i, double v) const {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Words2, v), rsrc, i * 8, 0, 0);
+    }
+    template <int kHow>
+    __device__ __forceinline__ void store2(int i, double2 v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(Words4, v), rsrc, i * 8, 0, kHow);
+    }
+    typedef unsigned int Words2 __attribute__((ext_vector_type(2)));
+    typedef unsigned int Words4 __attribute__((ext_vector_type(4)));
+};
+
+// A table of L values held across the lanes of each row of 16 (value e in lane e mod 16 of register
+// e / 16), so that a wave-uniform entry is one cross-lane move (DPP row broadcast) away: the stage
+// kernel's D^ entries as scalar loads came a few at a time (81 doubles are more than the scalar
+// registers hold), each batch a wait of some 300 cycles that the contraction of the line could
+// not hide: 3,650 cycles for the 81 multiply-adds of a line at N = 8.
+template <int L>
+struct LaneTable {
+    double v[(L + 15) / 16];
+    __device__ __forceinline__ void load(const double *t) {
+        const int m = threadIdx.x & 15;
+#pragma unroll
+        for (int p = 0; p < (L + 15) / 16; ++p) v[p] = t[min(p * 16 + m, L - 1)];
+    }
+    template <int E>
+    __device__ __forceinline__ double get() const {
+        const long long b = __builtin_bit_cast(long long, v[E / 16]);
+        return __builtin_bit_cast(double, (long long)__builtin_amdgcn_update_dpp(0ll, b, 0x150 + E % 16, 0xf, 0xf, true));
+    }
+};
+
+// D^ F of a line by even and odd parts: the Gauss nodes are symmetric, so D^[N-i][N-k] = -D^[i][k], and with
+// s_k = F[k] + F[N-k], d_k = F[k] - F[N-k] (k < h = (N+1)/2) and the middle node m of an even order
+//   Q_i = sum_k A[i][k] s_k + D^[i][m] F[m],  P_i = sum_k B[i][k] d_k,  A, B = (D^[i][k] +- D^[i][N-k])/2,
+//   (D^ F)[i] = P_i + Q_i,  (D^ F)[N-i] = P_i - Q_i,  (D^ F)[m] = P_m,
+// about half the multiply-adds and entries of D^. The table holds row by row A[i][.], D^[i][m], B[i][.],
+// then B[m][.].
+template <int NF, int E = 0>
+__device__ __forceinline__ void even_odd_entries(const LaneTable<even_odd_len(NF)> &D, const double *F, double *a) {
+    constexpr int h = NF / 2, odd = NF & 1, per = 2 * h + odd;
+    constexpr bool mid = E >= h * per;
+    constexpr int i = mid ? h : E / per, c = mid ? h + odd + E - h * per : E % per;
+    // entry c of a row multiplies F[c]: s in [0, h), F[m] at h, then d
+    constexpr int out = c < h + odd ? NF - 1 - i : i;  // Q_i is summed in place N - i, P_i in place i
+    const double d = D.template get<E>();
+    a[out] = c == 0 || c == h + odd ? d * F[c] : fma(d, F[c], a[out]);
+    // finished here, a row at a time: the compiler would keep the moved entries and move the sums on
+    if constexpr (c == per - 1) {
+        asm volatile("" : "+v"(a[i]));
+        if constexpr (!mid) asm volatile("" : "+v"(a[NF - 1 - i]));
+    }
+    if constexpr (E + 1 < even_odd_len(NF)) even_odd_entries<NF, E + 1>(D, F, a);
+}
+
+// a = D^ F (F is overwritten).
+template <int NF>
+__device__ __forceinline__ void contract(const LaneTable<even_odd_len(NF)> &D, double *F, double *a) {
+    constexpr int h = NF / 2, odd = NF & 1;
+    double t[NF];
+#pragma unroll
+    for (int k = 0; k < h; ++k) {
+        t[k] = F[k] + F[NF - 1 - k];
+        t[h + odd + k] = F[k] - F[NF - 1 - k];
+    }
+    if (odd) t[h] = F[h];
+    even_odd_entries<NF>(D, t, a);
+#pragma unroll
+    for (int i = 0; i < h; ++i) {
+        const double P = a[i], Q = a[NF - 1 - i];
+        a[i] = P + Q;
+        a[NF - 1 - i] = P - Q;
+    }
+}
+
+// tid, opaque to the compiler, so that indices formed from it are formed again rather than kept in
+// registers since an earlier phase.
+__device__ __forceinline__ int fresh(int tid) {
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+
+// Values from a tile's first value down to the 128-byte line it starts in: the tile's loads and
+// stores start there (the values before the tile masked), so that each wave instruction covers
+// whole lines.
+__device__ __forceinline__ int line_lead(const double *p) { return (int)(((uintptr_t)p >> 3) & 15); }
+
+// What the flux of a side point with a record needs of it (an inflow ghost reads its nodes too).
+struct SideRecord {
+    double nx, ny, tx, ty, sf;
+    int64_t slot;
+    int32_t kind, n_faces;
+    __device__ __forceinline__ void load(const BcSide *r) {
+        nx = r->nx;
+        ny = r->ny;
+        tx = r->tx;
+        ty = r->ty;
+        sf = r->sf;
+        slot = r->slot;
+        kind = r->kind;
+        n_faces = r->n_faces;
+    }
+};
+
+// (w_L - w_R)/2 and (w_L + w_R)/2 of point k of side s with a record: a boundary ghost (Mesh2D_t.cpp:
+// 4298-4730), a mortar side (the projected flux, already times the edge Jacobian: the side's scale
+// is 1 then) or a periodic side of another direction. The normal is the record's; tq is the
+// element's state in LDS, whose traces are summed in the order of the line's nodes.
+template <int N>
+__device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide *bc, const double *tq, const double *lm,
+                                            const double *lp, const double *x, const double *tr_in,
+                                            const double *side_flux, int s, int k, const double *t_ptr, double cw,
+                                            double &fa, double &fb) {
+    constexpr int NF = N + 1, NFP = StageTile<N>::NFP, NEP = StageTile<N>::NEP;
+    constexpr double c = kWaveSpeed;
+    if (rec.kind == kKindMortar) {  // projected by the mortar kernel (already x sf)
+        const double *sfl = side_flux + rec.slot + k;
+        double f0 = sfl[0], f1 = sfl[NF], f2 = sfl[2 * NF];
+        for (int m = 1; m < rec.n_faces; ++m) {  // a side covered by several faces
+            const double *s2 = sfl + m * 3 * NF;
+            f0 += s2[0];
+            f1 += s2[NF];
+            f2 += s2[2 * NF];
+        }
+        fa = f0;
+        fb = f1 * rec.nx + f2 * rec.ny;
+        return;
+    }
+    double pL = 0.0, uL = 0.0, vL = 0.0;
+    {
+        const bool low = s == 0 || s == 3;
+        const int m = s < 2 ? k : N - k, stride = (s & 1) ? NFP : 1;
+        const double *line = tq + ((s & 1) ? m : m * NFP);
+        constexpr int kUnroll = NF <= 6 ? NF : 3;
+#pragma unroll kUnroll
+        for (int j = 0; j < NF; ++j) {
+            const double lj = low ? lm[j] : lp[j];
+            pL += lj * line[j * stride];
+            uL += lj * line[NEP + j * stride];
+            vL += lj * line[2 * NEP + j * stride];
+        }
+    }
+    double pR = 0.0, uR = 0.0, vR = 0.0;
+    if (rec.kind == NDG_BC_WALL || rec.kind == NDG_BC_SYMMETRY) {
+        // ghost = sf * own trace, normal velocity reversed (Mesh2D_t.cpp:4377-4433)
+        pR = pL * rec.sf;
+        const double ux = uL * rec.sf, uy = vL * rec.sf;
+        const double l0 = -(ux * rec.nx + uy * rec.ny);
+        const double l1 = ux * rec.tx + uy * rec.ty;
+        uR = rec.nx * l0 + rec.tx * l1;
+        vR = rec.ny * l0 + rec.ty * l1;
+    } else if (rec.kind == NDG_BC_OUTFLOW) {
+        pR = pL * rec.sf;
+        uR = uL * rec.sf;
+        vR = vL * rec.sf;
+    } else if (rec.kind == NDG_BC_INFLOW) {
+        // ghost trace = g(x, t) at the ghost's nodes, seen reversed (Mesh2D_t.cpp:4575-4599)
+        const double interp = (x[N - k] + 1) / 2;
+        const double X = bc->bx * interp + bc->ax * (1 - interp);
+        const double Y = bc->by * interp + bc->ay * (1 - interp);
+        plane_wave(X, Y, *t_ptr, cw, pR, uR, vR);
+    } else if (rec.kind == kKindTrace) {
+        const double *nb = tr_in + rec.slot + (N - k);
+        pR = nb[0];
+        uR = nb[NF];
+        vR = nb[2 * NF];
+    }
+    const double wL = pL + c * (uL * rec.nx + vL * rec.ny);
+    const double wR = pR - c * (uR * rec.nx + vR * rec.ny);
+    fa = c * (wL - wR) / 2;
+    fb = (wL + wR) / 2;
+}
 
 template <int N, bool RHS_ONLY>
-__global__ void __launch_bounds__(192)
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 4 : N <= 12 ? 3 : 2)))
 stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
              const BcSide *__restrict__ bc, const double *__restrict__ tab,
-             const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ tr_in,
-             double *__restrict__ tr_out, double *__restrict__ rhs, const double *__restrict__ side_flux,
-             int64_t K, int rk_flags, double a, double gdt, const double *__restrict__ t_ptr, int epb,
-             int remap, double cw) {
-    const bool first = rk_flags & kRkFirst, store_g = !(rk_flags & kRkLast);
+             const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ w_in,
+             double *__restrict__ w_out, const double *__restrict__ tr_in, double *__restrict__ tr_out,
+             double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
+             double gdt, const double *__restrict__ t_ptr, int epb, int remap, double cw) {
+    const bool first = flags & kRkFirst, store_g = !(flags & kRkLast), once = flags & kStream;
     using S = LineShape<N>;
-    constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT;
+    using L = StageTile<N>;
+    constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT, NFP = L::NFP, NEP = L::NEP;
     constexpr double c = kWaveSpeed;
-    __shared__ double s_q[EPB * 3 * NE];
-    __shared__ double s_d[EPB * 3 * NE];
-    __shared__ double s_tr[EPB * 12 * NF];
-    __shared__ double s_met[EPB * 4 * NF];
-    __shared__ double s_side[EPB * 4 * 3];  // outward normal and edge Jacobian per side
-    __shared__ double s_v[EPB * 8];
-    const double *Dh = tab;
+    __shared__ double s_q[EPB * 3 * NEP];
+    __shared__ double s_d[EPB * 3 * NEP];  // vertices, then d_xi, then the new traces on sides 1 and 3
+    __shared__ double s_f[L::kFlux];       // fluxes, then the new traces on sides 0 and 2
+    __shared__ double s_side[EPB * 4 * 3]; // outward normal and edge Jacobian per side
+    double *const s_v = s_d;
+    static_assert(EPB * 8 <= EPB * 3 * NEP, "the vertices fit the tile they share");
     const double *lm = tab + NF * NF;
     const double *lp = lm + NF;
     const double *x = lp + 2 * NF;
-    const double *winv = x + NF;
+    const double *lpw = tab + table_stage_offset(N);  // l(+1) / w; that of l(-1) is its reverse
 
     const int tid = threadIdx.x;
     const int f = __builtin_amdgcn_readfirstlane(tid >> 6);  // field of this wave
     const int lane = tid & 63;
-    const int el = lane / NF, l = lane % NF;
     const int64_t blk = remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
     const int64_t e0 = blk * epb;
     const int nel = (int)min<int64_t>(epb, K - e0);
-    const bool active = el < nel;
+    const int n_val = nel * 3 * NE, n_pt = nel * 4 * NF;
+    const bool active = lane < nel * NF;
+    // lanes past the tile's lines work on line 0 of its first element, so that every lane takes part
+    // in the D^ broadcasts, and store nothing
+    const int el = active ? lane / NF : 0, l = active ? lane % NF : 0;
 
     __builtin_amdgcn_s_setprio(3);  // issue this workgroup's loads ahead of other waves' math
     // P0
@@ -162,275 +437,295 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
         const int item = tid + it * T;
-        code[it] = item < nel * 4 * NF ? side_nb[(e0 + item / NF / 4) * 4 + (item / NF) % 4] : INT32_MIN;
+        code[it] = item < n_pt ? side_nb[e0 * 4 + item / NF] : INT32_MIN;
     }
-    double qreg[S::QPT];
-    const double *qg = q + e0 * 3 * NE;
+    int32_t tile_code[(EPB * 4 + 63) / 64];  // all the tile's codes, over the lanes of each wave
 #pragma unroll
-    for (int it = 0; it < S::QPT; ++it) {
-        const int r = tid + it * T;
-        qreg[it] = r < nel * 3 * NE ? qg[r] : 0.0;
-    }
-    double vreg[S::VPT];
-#pragma unroll
-    for (int it = 0; it < S::VPT; ++it) {
-        const int r = tid + it * T;
-        vreg[it] = r < nel * 8 ? verts[e0 * 8 + r] : 0.0;
-    }
+    for (int it = 0; it < (EPB * 4 + 63) / 64; ++it)
+        tile_code[it] = side_nb[e0 * 4 + min(lane + 64 * it, nel * 4 - 1)];
     // The RK register lives only within a step (the first stage writes it without reading it), so
-    // its layout is the kernel's own: within the workgroup's tile of nel elements it is stored as
-    // [f][j][el][i], so that the row owners of all the tile's elements read and write one line
-    // index j with consecutive lanes on consecutive addresses (one contiguous run per wave
-    // instruction instead of one short run per element).
-    double g_old[NF];
-    if (!RHS_ONLY && !first && active) {
-        const double *gg = g + e0 * 3 * NE + ((int64_t)f * NF * nel + el) * NF + l;
+    // its layout is the kernel's own: within the workgroup's tile it is stored as [f][j / 2][el][i][j % 2]
+    // (an odd last j by itself), so that the row owners of all the tile's elements read and write two
+    // line indices j with consecutive lanes on consecutive 16-byte words, each such run starting on a
+    // 128-byte line.
+    const int run = rk_run<N>(epb);
+    const Buffer g_buf(RHS_ONLY ? nullptr : g + (blk * 3 + f) * NF * run, RHS_ONLY ? 0 : NF * run);
+    const double *qg = q + e0 * 3 * NE;
+    const int lead = line_lead(qg), q_last = lead + n_val - 1;
+    const Buffer q_buf(qg - lead, lead + n_val), v_buf(verts + e0 * 8, nel * 8), w_buf(w_in + e0 * 4 * NF, n_pt);
+    double2 qreg[L::QPT], g_old[NF / 2];
+    double vreg[S::VPT], own[FPT], g_odd = 0.0;
+    LaneTable<even_odd_len(NF)> Dh;
+    auto load_tile = [&](auto how) {
+        constexpr int kHow = decltype(how)::value;
 #pragma unroll
-        for (int j = 0; j < NF; ++j) g_old[j] = gg[j * nel * NF];
-    } else {
+        for (int it = 0; it < L::QPT; ++it) {
+            const int i = 2 * (tid + it * T);
+            qreg[it] = q_buf.load2<kHow>(i == q_last ? i - 1 : i);  // the last value as the second of a pair
+        }
 #pragma unroll
-        for (int j = 0; j < NF; ++j) g_old[j] = 0.0;
-    }
-    double nbv[FPT][3];
+        for (int it = 0; it < S::VPT; ++it) vreg[it] = v_buf.load(tid + it * T);
+        Dh.load(lpw + NF);
+#pragma unroll
+        for (int it = 0; it < FPT; ++it) own[it] = w_buf.load(tid + it * T);
+        if (!RHS_ONLY && !first) {
+#pragma unroll
+            for (int j = 0; j < NF / 2; ++j) g_old[j] = g_buf.load2<kHow>(2 * j * run + 2 * lane);
+            if (NF % 2) g_odd = g_buf.load(NF / 2 * 2 * run + lane);
+        }
+    };
+    if (once) load_tile(std::integral_constant<int, Buffer::kNonTemporal>());
+    else load_tile(std::integral_constant<int, 0>());
+    SideRecord rec[FPT];
+#pragma unroll
+    for (int it = 0; it < FPT; ++it)
+        if (code[it] < 0 && code[it] != INT32_MIN) rec[it].load(bc + (-1 - code[it]));
+    double ext[FPT];
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
-        nbv[it][0] = nbv[it][1] = nbv[it][2] = 0.0;
-        const int32_t cd = code[it];
-        if (cd >= 0) {
-            const int k = (tid + it * T) % NF;
-            const double *nb = tr_in + (int64_t)(cd >> 2) * 12 * NF + (cd & 3) * 3 * NF + (N - k);
-            nbv[it][0] = nb[0];
-            nbv[it][1] = nb[NF];
-            nbv[it][2] = nb[2 * NF];
-        }
+        const int32_t cd = max(code[it], 0);  // side 0 of the group for sides with a record
+        const int k = (tid + it * T) % NF;
+        ext[it] = w_in[(int64_t)cd * NF + (N - k)];
     }
     __builtin_amdgcn_s_setprio(0);
+    // in the order of the loads; the whole of the LDS tiles is written, with zeros past the last
+    // element; the own characteristics wait in the flux array
+#pragma unroll
+    for (int it = 0; it < L::QPT; ++it) {
+        const int r = 2 * (tid + it * T) - lead;
+        const bool inside = 2 * (it + 1) * T <= EPB * 3 * NE;
+        if (r + lead == q_last) qreg[it] = make_double2(qreg[it].y, 0.0);
+        if ((it > 0 || r >= 0) && (inside || r < EPB * 3 * NE)) s_q[L::at(r)] = qreg[it].x;
+        if ((it > 0 || r >= -1) && (inside || r + 1 < EPB * 3 * NE)) s_q[L::at(r + 1)] = qreg[it].y;
+    }
 #pragma unroll
     for (int it = 0; it < S::VPT; ++it) {
         const int r = tid + it * T;
-        if (r < nel * 8) s_v[r] = vreg[it];
+        if ((it + 1) * T <= EPB * 8 || r < EPB * 8) s_v[r] = vreg[it];
     }
-#pragma unroll
-    for (int it = 0; it < S::QPT; ++it) {
-        const int r = tid + it * T;
-        if (r < nel * 3 * NE) s_q[r] = qreg[it];
-    }
-    __syncthreads();
-
-    // P1
-    if (active) {
-        const double *P = s_v + el * 8;
-        double *met = s_met + el * 4 * NF;
-        if (f == 0) {  // x_eta, y_eta depend on xi only (include/functions/quad_metrics.tpp:3-8)
-            const double xi = x[l];
-            met[l] = ((1 - xi) * (P[6] - P[0]) + (1 + xi) * (P[4] - P[2])) / 4;
-            met[NF + l] = ((1 - xi) * (P[7] - P[1]) + (1 + xi) * (P[5] - P[3])) / 4;
-        } else if (f == 1) {  // x_xi, y_xi depend on eta only
-            const double eta = x[l];
-            met[2 * NF + l] = ((1 - eta) * (P[2] - P[0]) + (1 + eta) * (P[4] - P[6])) / 4;
-            met[3 * NF + l] = ((1 - eta) * (P[3] - P[1]) + (1 + eta) * (P[5] - P[7])) / 4;
-        } else {  // sides l, l + N + 1, ...: outward normal of the edge P_s -> P_s+1 and its Jacobian
-            for (int s = l; s < 4; s += NF) {
-                const int s1 = (s + 1) & 3;
-                const double ex = P[2 * s1] - P[2 * s], ey = P[2 * s1 + 1] - P[2 * s + 1];
-                const double len = sqrt(ex * ex + ey * ey);
-                double *sd = s_side + (el * 4 + s) * 3;
-                sd[0] = ey / len;
-                sd[1] = -(ex / len);
-                sd[2] = side_scale(P, s, x[0]);
-            }
-        }
-        const double *tq = s_q + el * 3 * NE + f * NE;
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
-#pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            const double row = tq[l * NF + j], col = tq[j * NF + l];
-            t0 += lm[j] * row;
-            t2 += lp[j] * row;
-            t1 += lp[j] * col;
-            t3 += lm[j] * col;
-        }
-        double *tr = s_tr + el * 12 * NF + f * NF;
-        tr[l] = t0;
-        tr[6 * NF + (N - l)] = t2;
-        tr[3 * NF + l] = t1;
-        tr[9 * NF + (N - l)] = t3;
-    }
-    __syncthreads();
-
-    // P2
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
         const int item = tid + it * T;
-        if (item < nel * 4 * NF) {
-            const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
-            double *tr = s_tr + fe * 12 * NF + s * 3 * NF + k;
-            const double pL = tr[0], uL = tr[NF], vL = tr[2 * NF];
-            const double *sd = s_side + (fe * 4 + s) * 3;
-            double nx = sd[0], ny = sd[1];
-            const double sf = sd[2];
-            double pR, uR, vR;
-            const int32_t cd = code[it];
-            if (cd >= 0) {
-                pR = nbv[it][0];
-                uR = nbv[it][1];
-                vR = nbv[it][2];
-            } else {
-                const BcSide rec = bc[-1 - cd];
-                if (rec.kind == kKindMortar) {  // projected by the mortar kernel (already x sf)
-                    const double *sfl = side_flux + rec.slot + k;
-                    double f0 = sfl[0], f1 = sfl[NF], f2 = sfl[2 * NF];
-                    for (int m = 1; m < rec.n_faces; ++m) {  // a side covered by several faces
-                        const double *s2 = sfl + m * 3 * NF;
-                        f0 += s2[0];
-                        f1 += s2[NF];
-                        f2 += s2[2 * NF];
-                    }
-                    tr[0] = f0;
-                    tr[NF] = f1;
-                    tr[2 * NF] = f2;
-                    continue;
-                }
-                nx = rec.nx;
-                ny = rec.ny;
-                if (rec.kind == NDG_BC_WALL || rec.kind == NDG_BC_SYMMETRY) {
-                    // ghost = sf * own trace, normal velocity reversed (Mesh2D_t.cpp:4377-4433)
-                    pR = pL * rec.sf;
-                    const double ux = uL * rec.sf, uy = vL * rec.sf;
-                    const double l0 = -(ux * rec.nx + uy * rec.ny);
-                    const double l1 = ux * rec.tx + uy * rec.ty;
-                    uR = rec.nx * l0 + rec.tx * l1;
-                    vR = rec.ny * l0 + rec.ty * l1;
-                } else if (rec.kind == NDG_BC_OUTFLOW) {
-                    pR = pL * rec.sf;
-                    uR = uL * rec.sf;
-                    vR = vL * rec.sf;
-                } else if (rec.kind == NDG_BC_INFLOW) {
-                    // ghost trace = g(x, t) at the ghost's nodes, seen reversed (Mesh2D_t.cpp:4575-4599)
-                    const double interp = (x[N - k] + 1) / 2;
-                    const double X = rec.bx * interp + rec.ax * (1 - interp);
-                    const double Y = rec.by * interp + rec.ay * (1 - interp);
-                    plane_wave(X, Y, *t_ptr, cw, pR, uR, vR);
-                } else {
-                    pR = 0.0;
-                    uR = 0.0;
-                    vR = 0.0;
-                }
-            }
-            const double wL = pL + c * (uL * nx + vL * ny);
-            const double wR = pR - c * (uR * nx + vR * ny);
-            tr[0] = (c * (wL - wR) / 2) * sf;
-            tr[NF] = (nx * (wL + wR) / 2) * sf;
-            tr[2 * NF] = (ny * (wL + wR) / 2) * sf;
-        }
+        if ((it + 1) * T <= EPB * 4 * NF || item < EPB * 4 * NF) s_f[item] = own[it];
     }
     __syncthreads();
 
-    const double *tq = s_q + el * 3 * NE;
-    const double *met = s_met + el * 4 * NF;
-    const double *fs = s_tr + el * 12 * NF + f * NF;
-    // P3: thread owns xi-line j = l of field f
-    if (active) {
-        const int j = l;
-        double F[NF];
+    // the points of sides with a record, from the state tile (before the contractions, whose sums
+    // would be live beside it)
+    bool has_record = false;
 #pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            const int node = k * NF + j;
-            const double xeta = met[k], yeta = met[NF + k];
-            if (f == 0) F[k] = yeta * (c * tq[NE + node]) - xeta * (c * tq[2 * NE + node]);
-            else if (f == 1) F[k] = yeta * tq[node];
-            else F[k] = -(xeta * tq[node]);
+    for (int it = 0; it < (EPB * 4 + 63) / 64; ++it) has_record = has_record || tile_code[it] < 0;
+    const bool recorded = __any(has_record);  // the same in every wave
+    if (recorded) {
+#pragma unroll
+        for (int it = 0; it < FPT; ++it) {
+            const int item = tid + it * T;
+            if (code[it] >= 0 || code[it] == INT32_MIN) continue;
+            const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
+            record_flux<N>(rec[it], bc + (-1 - code[it]), s_q + fe * 3 * NEP, lm, lp, x, tr_in, side_flux, s, k, t_ptr,
+                           cw, s_f[item], s_f[EPB * 4 * NF + item]);
         }
-        const double Fr = fs[3 * NF + j], Fl = fs[9 * NF + (N - j)];
-        double *d = s_d + el * 3 * NE + f * NE + j;
+    }
+
+    // P1. Metric lines from the vertices (include/functions/quad_metrics.tpp:3-8): x_eta, y_eta
+    // are linear in xi, x_xi, y_xi in eta.
+    const double *tq = s_q + el * 3 * NEP;
+    const double *P = s_v + el * 8;
+    double vx[NF], ve[NF];
+    {
+        double F[NF];
+        // a line's value at coordinate t is m + d t, from its values P_a -> P_b at t = -1 and at t = +1
+        auto mean = [&](int a0, int a1, int b0, int b1) { return ((P[b1] - P[b0]) + (P[a1] - P[a0])) / 4; };
+        auto slope = [&](int a0, int a1, int b0, int b1) { return ((P[b1] - P[b0]) - (P[a1] - P[a0])) / 4; };
+        const double *col = tq + l, *row = tq + l * NFP;  // node (k, l) at col[k * NFP], (l, k) at row[k]
+        if (f == 0) {
+            const double xe_m = mean(0, 6, 2, 4), xe_d = slope(0, 6, 2, 4), ye_m = mean(1, 7, 3, 5), ye_d = slope(1, 7, 3, 5);
+#pragma unroll
+            for (int k = 0; k < NF; ++k)
+                F[k] = (ye_m + ye_d * x[k]) * col[NEP + k * NFP] - (xe_m + xe_d * x[k]) * col[2 * NEP + k * NFP];
+        } else {  // y_eta p, -x_eta p
+            const int o = f == 1 ? 1 : 0;
+            const double m = mean(o, 6 + o, 2 + o, 4 + o), d = slope(o, 6 + o, 2 + o, 4 + o), sign = f == 1 ? 1.0 : -1.0;
+#pragma unroll
+            for (int k = 0; k < NF; ++k) F[k] = (sign * m + sign * d * x[k]) * col[k * NFP];
+        }
+        contract<NF>(Dh, F, vx);
+        __builtin_amdgcn_sched_barrier(0);  // one line's operands in registers at a time
+        if (f == 0) {
+            const double xx_m = mean(0, 2, 6, 4), xx_d = slope(0, 2, 6, 4), yx_m = mean(1, 3, 7, 5), yx_d = slope(1, 3, 7, 5);
+#pragma unroll
+            for (int k = 0; k < NF; ++k)
+                F[k] = (xx_m + xx_d * x[k]) * row[2 * NEP + k] - (yx_m + yx_d * x[k]) * row[NEP + k];
+        } else {  // -y_xi p, x_xi p
+            const int o = f == 1 ? 1 : 0;
+            const double m = mean(o, 2 + o, 6 + o, 4 + o), d = slope(o, 2 + o, 6 + o, 4 + o), sign = f == 1 ? -1.0 : 1.0;
+#pragma unroll
+            for (int k = 0; k < NF; ++k) F[k] = (sign * m + sign * d * x[k]) * row[k];
+        }
+        contract<NF>(Dh, F, ve);
+    }
+    // the Jacobian of a bilinear element is linear in eta along the thread's eta line: jac_m + jac_d eta
+    double jac_m, jac_d;
+    {
+        const double x_l = x[fresh(l)];
+        const double xeta = ((P[6] - P[0]) + (P[4] - P[2]) + ((P[4] - P[2]) - (P[6] - P[0])) * x_l) / 4;
+        const double yeta = ((P[7] - P[1]) + (P[5] - P[3]) + ((P[5] - P[3]) - (P[7] - P[1])) * x_l) / 4;
+        jac_m = (((P[4] - P[6]) + (P[2] - P[0])) * yeta - xeta * ((P[5] - P[7]) + (P[3] - P[1]))) / 4;
+        jac_d = (((P[4] - P[6]) - (P[2] - P[0])) * yeta - xeta * ((P[5] - P[7]) - (P[3] - P[1]))) / 4;
+    }
+    // fluxes of the side points, side geometry (sides l, l + N + 1, ... of the wave's elements)
+    const int t1 = fresh(tid);
+#pragma unroll
+    for (int it = 0; it < FPT; ++it) {
+        const int item = t1 + it * T;
+        if (item < n_pt && !(recorded && side_nb[e0 * 4 + item / NF] < 0)) {
+            const double w = s_f[item];
+            s_f[item] = c * (w - ext[it]) / 2;
+            s_f[EPB * 4 * NF + item] = (w + ext[it]) / 2;
+        }
+    }
+    if (f == 2 && active)
+        for (int s = l; s < 4; s += NF) {
+            double *sd = s_side + (el * 4 + s) * 3;
+            sd[2] = side_geometry(P, s, sd[0], sd[1]);
+            if (const int32_t cd = side_nb[(e0 + el) * 4 + s]; cd < 0) {
+                const BcSide &rec = bc[-1 - cd];
+                sd[0] = rec.nx;
+                sd[1] = rec.ny;
+                if (rec.kind == kKindMortar) sd[2] = 1.0;
+            }
+        }
+    __syncthreads();
+
+    // P2. Lifts: the thread's column j = l of d_xi and row i = l of d_eta. The flux of field f at a
+    // side point is (w_L - w_R)/2 (p) or the normal's component times (w_L + w_R)/2 (u, v), times
+    // the edge Jacobian.
+    {
+        const double *side = s_side + el * 12;
+        const double *fl = s_f + (f == 0 ? 0 : EPB * 4 * NF) + el * 4 * NF;
+        const double v1 = fl[NF + l], v3 = fl[3 * NF + N - l], v2 = fl[2 * NF + N - l], v0 = fl[l];
+        const double *n = side + (f == 2 ? 1 : 0);
+        const double n0 = f ? n[0] : 1.0, n1 = f ? n[3] : 1.0, n2 = f ? n[6] : 1.0, n3 = f ? n[9] : 1.0;
+        const double Fr = (n1 * v1) * side[5], Fl = (n3 * v3) * side[11], Ft = (n2 * v2) * side[8],
+                     Fb = (n0 * v0) * side[2];
+        double *d = s_d + el * 3 * NEP + f * NEP + l;
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
-            double acc = 0.0;
-#pragma unroll
-            for (int k = 0; k < NF; ++k) acc += Dh[i * NF + k] * F[k];
-            acc += (Fr * lp[i] + Fl * lm[i]) * winv[i];
-            d[i * NF] = acc;
+            vx[i] += Fr * lpw[i] + Fl * lpw[N - i];
+            ve[i] += Ft * lpw[i] + Fb * lpw[N - i];
         }
+        if (active)
+#pragma unroll
+            for (int i = 0; i < NF; ++i) d[i * NFP] = vx[i];
     }
     __syncthreads();
 
-    // P4: thread owns eta-line i = l of field f. The new RK register goes straight to HBM (tile
-    // layout, coalesced); the new state waits for the barrier.
-    double qn[NF];
-    if (active) {
-        const int i = l;
-        double Gt[NF];
+    // P3. The thread's eta line i = l of field f: the right-hand side replaces ve, then the new RK
+    // register line, which goes straight to HBM, and the new state line, which replaces the old
+    // one in the tile (no one else reads it until the barrier). One loop an operation, so that the
+    // nodes' chains overlap.
+    double *qrow = s_q + el * 3 * NEP + f * NEP + l * NFP;
+    {
+        double *d = s_d + el * 3 * NEP + f * NEP + l * NFP;
 #pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            const int node = i * NF + k;
-            const double xxi = met[2 * NF + k], yxi = met[3 * NF + k];
-            if (f == 0) Gt[k] = -yxi * (c * tq[NE + node]) + xxi * (c * tq[2 * NE + node]);
-            else if (f == 1) Gt[k] = -yxi * tq[node];
-            else Gt[k] = xxi * tq[node];
-        }
-        const double Ft = fs[6 * NF + (N - i)], Fb = fs[i];
-        const double xeta_i = met[i], yeta_i = met[NF + i];
-        double *d = s_d + el * 3 * NE + f * NE + i * NF;
-        const double *qrow = tq + f * NE + i * NF;
+        for (int j = 0; j < NF; ++j) ve[j] = (d[j] + ve[j]) * (-cw * recip(jac_m + jac_d * x[j]));
+        if (RHS_ONLY) {
+            if (active)
 #pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            double acc = 0.0;
+                for (int j = 0; j < NF; ++j) d[j] = ve[j];
+        } else if (!first) {
 #pragma unroll
-            for (int k = 0; k < NF; ++k) acc += Dh[j * NF + k] * Gt[k];
-            acc += (Ft * lp[j] + Fb * lm[j]) * winv[j];
-            const double jac = met[2 * NF + j] * yeta_i - xeta_i * met[3 * NF + j];
-            const double Gv = cw * ((-d[j] - acc) * recip(jac));
-            if (RHS_ONLY) {
-                d[j] = Gv;
-            } else {
-                const double gn = first ? Gv : a * g_old[j] + Gv;
-                if (store_g) g[e0 * 3 * NE + ((f * NF + j) * nel + el) * NF + i] = gn;
-                qn[j] = qrow[j] + gdt * gn;
+            for (int j = 0; j < NF / 2; ++j) {
+                ve[2 * j] = a * g_old[j].x + ve[2 * j];
+                ve[2 * j + 1] = a * g_old[j].y + ve[2 * j + 1];
             }
+            if (NF % 2) ve[NF - 1] = a * g_odd + ve[NF - 1];
         }
     }
-    __syncthreads();
     if (!RHS_ONLY && active) {
-        double *qw = s_q + el * 3 * NE + f * NE + l * NF;
+        if (store_g) {
+            auto store_lines = [&](auto how) {
 #pragma unroll
-        for (int j = 0; j < NF; ++j) qw[j] = qn[j];
+                for (int j = 0; j < NF / 2; ++j)
+                    g_buf.store2<decltype(how)::value>(2 * j * run + 2 * lane, make_double2(ve[2 * j], ve[2 * j + 1]));
+            };
+            if (once) store_lines(std::integral_constant<int, Buffer::kNonTemporal>());
+            else store_lines(std::integral_constant<int, 0>());
+            if (NF % 2) g_buf.store(NF / 2 * 2 * run + lane, ve[NF - 1]);
+        }
+        double t0 = 0.0, t2 = 0.0;
+#pragma unroll
+        for (int j = 0; j < NF; ++j) ve[j] = qrow[j] + gdt * ve[j];
+#pragma unroll
+        for (int j = 0; j < NF; ++j) {
+            qrow[j] = ve[j];
+            t0 += lp[N - j] * ve[j];
+            t2 += lp[j] * ve[j];
+        }
+        double *tr = s_f + (el * 3 + f) * 2 * NF;
+        tr[l] = t0;
+        tr[NF + (N - l)] = t2;
+    }
+    __syncthreads();
+
+    // P4
+    if (RHS_ONLY) {
+        double *rg = rhs + e0 * 3 * NE;
+        for (int r = tid; r < n_val; r += T) rg[r] = s_d[L::at(r)];
+        return;
+    }
+    if (active) {
+        const double *col = s_q + el * 3 * NEP + f * NEP + l;
+        double t1 = 0.0, t3 = 0.0;
+#pragma unroll
+        for (int j = 0; j < NF; ++j) {
+            const double v = col[j * NFP];
+            t1 += lp[j] * v;
+            t3 += lp[N - j] * v;
+        }
+        double *tr = s_d + (el * 3 + f) * 2 * NF;
+        tr[l] = t1;
+        tr[NF + (N - l)] = t3;
+    }
+    {
+        // pairs wholly inside the tile; its first and last value alone where a pair straddles an end
+        double *qw = q_out + e0 * 3 * NE;
+        const int t4 = fresh(tid);
+        const int lead_out = line_lead(qw), end = lead_out + n_val;
+        const Buffer out_buf(qw - lead_out, end & ~1);
+        auto value = [&](int r) { return s_q[min(max(L::at(r), 0), EPB * 3 * NEP - 1)]; };
+        auto store_tile = [&](auto how) {
+#pragma unroll
+            for (int it = 0; it < L::QPT; ++it) {
+                const int i = 2 * (t4 + it * T), r = i - lead_out;
+                const double2 v = make_double2(value(r), value(r + 1));
+                if (it > 0 || r >= 0) out_buf.store2<decltype(how)::value>(i, v);
+            }
+        };
+        if (once) store_tile(std::integral_constant<int, Buffer::kNonTemporal>());
+        else store_tile(std::integral_constant<int, 0>());
+        if ((lead_out & 1) && tid == 0) qw[0] = s_q[0];
+        if ((end & 1) && tid == 64) qw[n_val - 1] = s_q[L::at(n_val - 1)];
     }
     __syncthreads();
 
     // P5
-    if (RHS_ONLY) {
-        double *rg = rhs + e0 * 3 * NE;
+    const int t5 = fresh(tid);
 #pragma unroll
-        for (int it = 0; it < S::QPT; ++it) {
-            const int r = tid + it * T;
-            if (r < nel * 3 * NE) rg[r] = s_d[r];
+    for (int it = 0; it < FPT; ++it) {
+        const int item = t5 + it * T;
+        if (item >= n_pt) continue;
+        const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
+        const double *tr = ((s & 1) ? s_d : s_f) + fe * 6 * NF + (s >> 1) * NF + k;
+        const double *sd = s_side + (fe * 4 + s) * 3;
+        const double p = tr[0], u = tr[2 * NF], v = tr[4 * NF];
+        w_out[e0 * 4 * NF + item] = p + c * (u * sd[0] + v * sd[1]);
+        if ((recorded && side_nb[e0 * 4 + item / NF] < 0) || (flags & kTraceAll)) {
+            double *to = tr_out + (e0 + fe) * 12 * NF + s * 3 * NF + k;
+            to[0] = p;
+            to[NF] = u;
+            to[2 * NF] = v;
         }
-        return;
-    }
-    {
-        double *qw = q_out + e0 * 3 * NE;
-#pragma unroll
-        for (int it = 0; it < S::QPT; ++it) {
-            const int r = tid + it * T;
-            if (r < nel * 3 * NE) qw[r] = s_q[r];
-        }
-    }
-    if (active) {
-        const double *tqf = s_q + el * 3 * NE + f * NE;
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
-#pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            const double row = tqf[l * NF + j], col = tqf[j * NF + l];
-            t0 += lm[j] * row;
-            t2 += lp[j] * row;
-            t1 += lp[j] * col;
-            t3 += lm[j] * col;
-        }
-        double *to = tr_out + (e0 + el) * 12 * NF + f * NF;
-        to[l] = t0;
-        to[6 * NF + (N - l)] = t2;
-        to[3 * NF + l] = t1;
-        to[9 * NF + (N - l)] = t3;
     }
 }
 
@@ -465,8 +760,8 @@ __device__ __forceinline__ int64_t c32_tile_index(int64_t e, int f, int i, int j
 // q and qh are in reference node order; gl32 (RK register in x, low state word in y) is in the
 // FP32 stage kernel's tile order. Thread r writes one float2. The RK register carries no value
 // from one step to the next, so g is copied word for word whatever its order.
-__global__ void to_c32_kernel(const double *__restrict__ q, const double *__restrict__ g,
-                              float *__restrict__ qh, float2 *__restrict__ gl32, int64_t n, int nf, int epb) {
+__global__ void to_c32_kernel(const double *__restrict__ q, float *__restrict__ qh, float2 *__restrict__ gl32,
+                              int64_t n, int nf, int epb) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const int ne = nf * nf, node = (int)(r % ne), i = node / nf, j = node % nf;
@@ -475,11 +770,11 @@ __global__ void to_c32_kernel(const double *__restrict__ q, const double *__rest
     const double v = q[r];
     const float h = (float)v;
     qh[r] = h;
-    gl32[c32_tile_index(e, f, i, j, nf, epb, n / (3 * ne))] = make_float2((float)g[r], (float)(v - (double)h));
+    gl32[c32_tile_index(e, f, i, j, nf, epb, n / (3 * ne))] = make_float2(0.f, (float)(v - (double)h));
 }
 
 __global__ void from_c32_kernel(const float *__restrict__ qh, const float2 *__restrict__ gl32,
-                                double *__restrict__ q, double *__restrict__ g, int64_t n, int nf, int epb) {
+                                double *__restrict__ q, int64_t n, int nf, int epb) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const int ne = nf * nf, node = (int)(r % ne), i = node / nf, j = node % nf;
@@ -487,7 +782,6 @@ __global__ void from_c32_kernel(const float *__restrict__ qh, const float2 *__re
     const int f = (int)((r / ne) % 3);
     const float2 w = gl32[c32_tile_index(e, f, i, j, nf, epb, n / (3 * ne))];
     q[r] = (double)qh[r] + (double)w.y;
-    g[r] = (double)w.x;
 }
 
 template <int N>
@@ -695,7 +989,12 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
                 nx = (float)rec.nx;
                 ny = (float)rec.ny;
                 const float tx = (float)rec.tx, ty = (float)rec.ty, gs = (float)rec.sf;
-                if (rec.kind == NDG_BC_WALL || rec.kind == NDG_BC_SYMMETRY) {
+                if (rec.kind == kKindTrace) {
+                    const float *nb = tr_in + rec.slot + (N - k);
+                    pR = nb[0];
+                    uR = nb[NF];
+                    vR = nb[2 * NF];
+                } else if (rec.kind == NDG_BC_WALL || rec.kind == NDG_BC_SYMMETRY) {
                     pR = pL * gs;
                     const float ux = uL * gs, uy = vL * gs;
                     const float l0 = -(ux * nx + uy * ny);
@@ -1247,8 +1546,9 @@ template <int N>
 static hipError_t traces_n(const DeviceMesh &m, const Group &G, hipStream_t s) {
     using S = Shape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    hipLaunchKernelGGL(traces_kernel<N>, dim3((unsigned)blocks), dim3(S::THREADS), 0, s, G.tab, m.q + G.q_off,
-                       m.trace[m.cur] + G.tr_off, G.K);
+    hipLaunchKernelGGL(traces_kernel<N>, dim3((unsigned)blocks), dim3(S::THREADS), 0, s, m.verts + G.e_begin * 8,
+                       m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.trace[m.cur] + G.tr_off,
+                       m.wave[m.cur] + G.tr_off / 3, G.K);
     return hipGetLastError();
 }
 
@@ -1270,14 +1570,45 @@ int stage_tile_epb(const Group &G) {
 }
 
 template <int N>
+static int stage_run_n(int epb) { return rk_run<N>(epb); }
+
+int stage_tile_run(const Group &G) {
+    const int epb = stage_tile_epb(G);
+    switch (G.N) { CASES_1(stage_run_n, epb) }
+    return 0;
+}
+
+template <int N>
+static int64_t rk_values_n(int64_t K) {
+    constexpr int EPB = LineShape<N>::EPB;
+    return 3 * (N + 1) * std::max((K + EPB - 1) / EPB * rk_run<N>(EPB), K * (N + 2));
+}
+
+int64_t stage_rk_values(int N, int64_t K) {
+    switch (N) { CASES_1(rk_values_n, K) }
+    return 0;
+}
+
+// The state and the RK register go past the caches when they are far larger than these (the
+// last-level cache holds 256 MB), so that they leave room for what is read again. At N = 8, past and
+// through the caches: 512 x 512 (1 GB) 324 and 401 us a launch, 256 x 256 (255 MB) 85.8 and 91.1,
+// 192 x 192 (143 MB) 51.2 and 45.2, 160 x 160 (100 MB) 37.3 and 33.8.
+static int stage_flags(const DeviceMesh &m) {
+    return (m.trace_all ? kTraceAll : 0) | (16 * m.n_q > kStreamBytes ? kStream : 0);
+}
+
+template <int N>
 static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, hipStream_t s) {
     using S = LineShape<N>;
     const int epb = group_epb<N>(G, NDG_PRECISION_FP64);
     const int64_t blocks = (G.K + epb - 1) / epb;
     hipLaunchKernelGGL((stage_kernel<N, false>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, (m.q_out ? m.q_out : m.q) + G.q_off,
-                       m.g + G.q_off, m.trace[m.cur] + G.tr_off, m.trace[1 - m.cur] + G.tr_off, nullptr, m.side_flux,
-                       G.K, (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0), a, gdt,
+                       m.g + G.g_off, m.wave[m.cur] + G.tr_off / 3, m.wave[1 - m.cur] + G.tr_off / 3,
+                       m.trace[m.cur] + G.tr_off,
+                       m.trace[1 - m.cur] + G.tr_off, nullptr, m.side_flux, G.K,
+                       (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0) |
+                           stage_flags(m), a, gdt,
                        m.clock + 1 + stage, epb, G.tune[NDG_PRECISION_FP64].remap,
                        m.wave_speed);
     return hipGetLastError();
@@ -1288,8 +1619,9 @@ static hipError_t rhs_n(DeviceMesh &m, const Group &G, hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
     hipLaunchKernelGGL((stage_kernel<N, true>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
-                       m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.q + G.q_off, m.g + G.q_off,
-                       m.trace[m.cur] + G.tr_off, nullptr, m.rhs + G.q_off, m.side_flux, G.K, 1, 0.0, 0.0,
+                       m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.q + G.q_off, nullptr,
+                       m.wave[m.cur] + G.tr_off / 3, nullptr, m.trace[m.cur] + G.tr_off, nullptr, m.rhs + G.q_off, m.side_flux,
+                       G.K, stage_flags(m), 0.0, 0.0,
                        m.clock + 1, S::EPB, 1, m.wave_speed);
     return hipGetLastError();
 }
@@ -1444,7 +1776,7 @@ hipError_t launch_to_c32(DeviceMesh &m, hipStream_t s) {
     return for_groups(m, [&](const Group &G) -> hipError_t {
         const int64_t n = G.K * 3 * (int64_t)(G.N + 1) * (G.N + 1);
         hipLaunchKernelGGL(to_c32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m.q + G.q_off,
-                           m.g + G.q_off, m.qh + G.q_off, m.gl32 + G.q_off, n, G.N + 1, stage_max_epb(G.N));
+                           m.qh + G.q_off, m.gl32 + G.q_off, n, G.N + 1, stage_max_epb(G.N));
         return hipGetLastError();
     });
 }
@@ -1453,7 +1785,7 @@ hipError_t launch_from_c32(DeviceMesh &m, hipStream_t s) {
     return for_groups(m, [&](const Group &G) -> hipError_t {
         const int64_t n = G.K * 3 * (int64_t)(G.N + 1) * (G.N + 1);
         hipLaunchKernelGGL(from_c32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m.qh + G.q_off,
-                           m.gl32 + G.q_off, m.q + G.q_off, m.g + G.q_off, n, G.N + 1, stage_max_epb(G.N));
+                           m.gl32 + G.q_off, m.q + G.q_off, n, G.N + 1, stage_max_epb(G.N));
         return hipGetLastError();
     });
 }

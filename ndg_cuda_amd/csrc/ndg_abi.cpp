@@ -78,7 +78,7 @@ void ndg::arena_free(Arena &a) {
 
 void ndg::store_free(DeviceStore &s) {
     for (Arena *a : {&s.verts, &s.side_nb, &s.bc, &s.faces, &s.side_flux, &s.side_flux32, &s.q, &s.g, &s.tr[0],
-                     &s.tr[1], &s.rhs, &s.scratch, &s.qh, &s.gl32, &s.tr32[0], &s.tr32[1]})
+                     &s.tr[1], &s.wave[0], &s.wave[1], &s.rhs, &s.scratch, &s.qh, &s.gl32, &s.tr32[0], &s.tr32[1]})
         arena_free(*a);
 }
 
@@ -535,6 +535,7 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
             if (!d.groups.empty()) {
                 const Group &H = d.groups.back();
                 G.q_off = H.q_off + 3 * (int64_t)(H.N + 1) * (H.N + 1) * H.K;
+                G.g_off = H.g_off + stage_rk_values(H.N, H.K);
                 G.tr_off = H.tr_off + 12 * (int64_t)(H.N + 1) * H.K;
             }
             group_of_N[N] = (int)d.groups.size();
@@ -546,6 +547,7 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
         const Group &H = d.groups.back();
         d.n_q = H.q_off + 3 * (int64_t)(H.N + 1) * (H.N + 1) * H.K;
         d.n_tr = H.tr_off + 12 * (int64_t)(H.N + 1) * H.K;
+        d.n_g = H.g_off + stage_rk_values(H.N, H.K);
     }
     d.N_min = d.groups.front().N;
     d.N_max = d.groups.back().N;
@@ -578,6 +580,7 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
     std::vector<BcSide> bcs = m->bc_base;
     for (size_t b = 0; b < bcs.size(); ++b)
         if (m->bar_zero[(size_t)m->bc_bar[b]]) bcs[b].sf = 0.0;
+    d.n_ghost = (int64_t)bcs.size();
     for (const BcSide &b : bcs) d.has_inflow = d.has_inflow || b.kind == NDG_BC_INFLOW;
 
     // Device connectivity. Sides whose exterior state has another order are non-conforming: they
@@ -586,14 +589,22 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
     std::vector<int32_t> side_nb((size_t)(4 * K));
     std::vector<MortarFace> faces;
     std::vector<int64_t> mortar_rec((size_t)(4 * K), -1);
+    std::vector<int64_t> partners;  // sides whose three traces are read
     int64_t n_slot = 0;
-    auto add_mortar_side = [&](int64_t es) {
+    auto add_record = [&](int64_t es, int32_t kind) -> BcSide & {
         BcSide rec{};
-        rec.kind = kKindMortar;
-        rec.slot = n_slot;
-        n_slot += 3 * (int64_t)(order[es / 4] + 1);
+        rec.kind = kind;
+        rec.slot = -1;
+        const v2 f0 = corner(es / 4, (int)(es % 4)), f1 = corner(es / 4, (int)(es % 4) + 1);
+        face_frame(f0, f1, f0, f1, rec.nx, rec.ny, rec.tx, rec.ty);
         mortar_rec[es] = (int64_t)bcs.size();
         bcs.push_back(rec);
+        return bcs.back();
+    };
+    auto add_mortar_side = [&](int64_t es) {
+        BcSide &rec = add_record(es, kKindMortar);
+        rec.slot = n_slot;
+        n_slot += 3 * (int64_t)(order[es / 4] + 1);
         return rec.slot;
     };
     // A larger hanging side sums the projected fluxes of its faces, one block per small side
@@ -640,10 +651,18 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
                     fc.slotL = slot + h * 3 * (int64_t)(order[e] + 1);
                     fc.slotR = -1;
                     faces.push_back(fc);
+                    partners.push_back(c);
                 }
                 continue;
             }
             if (hk == 2) continue;  // built from its small sides
+            if (l >= 0 && hk == 0 && order[l / 4] == order[e] && periodic_link[es] == kPeriodicOblique) {
+                BcSide &rec = add_record(es, kKindTrace);
+                rec.slot = trace_at(l / 4, (int)(l % 4)) - group_of(l / 4).tr_off;
+                rec.partner = local_of(l / 4) * 4 + l % 4;
+                partners.push_back(l);
+                continue;
+            }
             if (l < 0 || (hk == 0 && order[l / 4] == order[e])) continue;
             const int64_t r = l / 4;
             const int rs = (int)(l % 4);
@@ -683,7 +702,9 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
                 fc.slotR = add_mortar_side(l);
             }
             faces.push_back(fc);
+            partners.push_back(l);
         }
+    for (int64_t p : partners) d.trace_all = d.trace_all || (mortar_rec[p] < 0 && link[p] >= 0);
     ndg_status st;
     if ((st = ensure_shared_tables(m)) != NDG_OK) return st;
     for (MortarFace &fc : faces)
@@ -730,7 +751,9 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
         G.tab = m->tab64[G.N];
     }
     if ((st = fit_view(store.q, &d.q, d.n_q, "hipMalloc q")) != NDG_OK) return st;
-    if ((st = fit_view(store.g, &d.g, d.n_q, "hipMalloc g")) != NDG_OK) return st;
+    if ((st = fit_view(store.g, &d.g, d.n_g, "hipMalloc g")) != NDG_OK) return st;
+    for (int k = 0; k < 2; ++k)
+        if ((st = fit_view(store.wave[k], &d.wave[k], d.n_tr / 3, "hipMalloc characteristics")) != NDG_OK) return st;
     if ((st = fit_view(store.tr[0], &d.trace[0], d.n_tr, "hipMalloc traces")) != NDG_OK) return st;
     if ((st = fit_view(store.tr[1], &d.trace[1], d.n_tr, "hipMalloc traces")) != NDG_OK) return st;
     d.scratch_len = 1024;
@@ -1037,7 +1060,7 @@ ndg_status build_topology(const HostMesh &h, Topology &t) {
             // unchanged (and takes the donor element's order), so the side couples to the donor
             // element side directly.
             link[es] = bar_side[d];
-            periodic_link[es] = 1;
+            periodic_link[es] = kPeriodic;
             continue;
         }
         if (kind < NDG_BC_NONE || kind > NDG_BC_OUTFLOW) return fail(NDG_ERR_INVALID, "mesh topology: unknown boundary kind");
@@ -1193,6 +1216,11 @@ ndg_status build_topology(const HostMesh &h, Topology &t) {
     for (int64_t es = 0; es < 4 * K; ++es)
         if (link[es] == INT64_MIN)
             return fail(NDG_ERR_INVALID, "mesh topology: element side has neither a neighbour nor a boundary bar");
+    for (int64_t es = 0; es < 4 * K; ++es) {
+        if (!periodic_link[es]) continue;
+        const v2 a0 = P(h.quads[es]), a1 = P(end_node(es)), b0 = P(h.quads[link[es]]), b1 = P(end_node(link[es]));
+        if (!opposite_sides(a1.x - a0.x, a1.y - a0.y, b1.x - b0.x, b1.y - b0.y)) periodic_link[es] = kPeriodicOblique;
+    }
     return NDG_OK;
 }
 
@@ -1274,7 +1302,6 @@ extern "C" ndg_status ndg_mesh_create(const ndg_mesh_desc *desc, const ndg_table
     if (st != NDG_OK) return st;
     DeviceMesh &d = m->d;
     HIP_TRY(hipMemsetAsync(d.q, 0, sizeof(double) * d.n_q, m->stream), "hipMemset q");
-    HIP_TRY(hipMemsetAsync(d.g, 0, sizeof(double) * d.n_q, m->stream), "hipMemset g");
     HIP_TRY(launch_traces(d, m->stream), "traces kernel");
     HIP_TRY(hipStreamSynchronize(m->stream), "mesh create sync");
     *out = m.release();
@@ -1421,7 +1448,6 @@ extern "C" ndg_status ndg_set_ic(ndg_mesh *mesh, const ndg_ic_desc *ic) {
     mesh->ic_pulses.assign(ic->pulses, ic->pulses + 4 * np);
     mesh->ic_period[0] = ic->period_x;
     mesh->ic_period[1] = ic->period_y;
-    HIP_TRY(hipMemsetAsync(d.g, 0, sizeof(double) * d.n_q, mesh->stream), "hipMemset g");
     HIP_TRY(launch_traces(d, mesh->stream), "traces kernel");
     ndg_status st = refresh_c32(mesh);
     if (st != NDG_OK) return st;
@@ -1437,7 +1463,6 @@ extern "C" ndg_status ndg_set_state(ndg_mesh *mesh, const double *p, const doubl
     double *const ins[3] = {const_cast<double *>(p), const_cast<double *>(u), const_cast<double *>(v)};
     ndg_status st = copy_state(mesh, d.q, ins, false, "upload state");
     if (st != NDG_OK) return st;
-    HIP_TRY(hipMemsetAsync(d.g, 0, sizeof(double) * d.n_q, mesh->stream), "hipMemset g");
     HIP_TRY(launch_traces(d, mesh->stream), "traces kernel");
     if ((st = refresh_c32(mesh)) != NDG_OK) return st;
     HIP_TRY(hipStreamSynchronize(mesh->stream), "ndg_set_state sync");
@@ -1577,6 +1602,8 @@ extern "C" ndg_status ndg_get_traces(ndg_mesh *mesh, double *out) {
     ndg_status st = refresh_fp64(mesh);
     if (st != NDG_OK) return st;
     const DeviceMesh &d = mesh->d;
+    // the steps keep the three traces of the sides that need them only
+    if (d.precision == NDG_PRECISION_FP64) HIP_TRY(launch_traces(d, mesh->stream), "traces kernel");
     mesh->staging.resize((size_t)d.n_tr);
     HIP_TRY(hipMemcpyAsync(mesh->staging.data(), d.trace[d.cur], sizeof(double) * d.n_tr, hipMemcpyDeviceToHost,
                            mesh->stream), "download traces");
@@ -2185,7 +2212,6 @@ ndg_status adapt_split(ndg_mesh *mesh, const std::vector<int32_t> &ref, const st
         for (int64_t k = 0; k < Knew; ++k) keep[(size_t)k] = !child[(size_t)k] && !raise[(size_t)parent[(size_t)k]];
         carry_estimates(mesh, (size_t)K, parent, keep);
     }
-    HIP_TRY(hipMemsetAsync(d.g, 0, sizeof(double) * d.n_q, mesh->stream), "hipMemset g");
     HIP_TRY(launch_traces(d, mesh->stream), "traces kernel");
     if (precision == NDG_PRECISION_FP32_COMPENSATED) {
         if ((st = ndg_mesh_set_precision(mesh, precision)) != NDG_OK) return st;
@@ -2255,7 +2281,7 @@ ndg_status adapt_on_device(ndg_mesh *mesh, int32_t N_max, int32_t max_split_leve
     // the device mesh of the new layout, in the spare store
     DeviceMesh nd;
     nd.K = Kn;
-    int64_t e_begin = 0, q_off = 0, tr_off = 0;
+    int64_t e_begin = 0, q_off = 0, tr_off = 0, g_off = 0;
     for (int n = 0; n <= kMaxOrder; ++n) {
         const int64_t Kg = (int64_t)c.order_count[n];
         if (Kg == 0) continue;
@@ -2266,17 +2292,22 @@ ndg_status adapt_on_device(ndg_mesh *mesh, int32_t N_max, int32_t max_split_leve
         G.e_begin = e_begin;
         G.q_off = q_off;
         G.tr_off = tr_off;
+        G.g_off = g_off;
         G.tab = mesh->tab64[n];
         nd.groups.push_back(G);
         e_begin += Kg;
         q_off += 3 * (int64_t)(n + 1) * (n + 1) * Kg;
         tr_off += 12 * (int64_t)(n + 1) * Kg;
+        g_off += stage_rk_values(n, Kg);
     }
     nd.n_q = q_off;
     nd.n_tr = tr_off;
+    nd.n_g = g_off;
     nd.N_min = nd.groups.front().N;
     nd.N_max = nd.groups.back().N;
     nd.n_bc = Gn + (int64_t)c.n_rec;
+    nd.n_ghost = Gn;
+    nd.trace_all = c.bare_partner != 0;
     nd.n_faces = (int64_t)c.n_face;
     nd.n_side_flux = (int64_t)c.n_slot;
     nd.mortar_nodes = (int)c.mortar_nodes;
@@ -2285,7 +2316,9 @@ ndg_status adapt_on_device(ndg_mesh *mesh, int32_t N_max, int32_t max_split_leve
         (st = fit_view(ns.bc, &nd.bc, nd.n_bc, "hipMalloc boundary records")) != NDG_OK ||
         (st = fit_view(ns.faces, &nd.faces, nd.n_faces, "hipMalloc mortar faces")) != NDG_OK ||
         (st = fit_view(ns.q, &nd.q, nd.n_q, "hipMalloc q")) != NDG_OK ||
-        (st = fit_view(ns.g, &nd.g, nd.n_q, "hipMalloc g")) != NDG_OK ||
+        (st = fit_view(ns.g, &nd.g, nd.n_g, "hipMalloc g")) != NDG_OK ||
+        (st = fit_view(ns.wave[0], &nd.wave[0], nd.n_tr / 3, "hipMalloc characteristics")) != NDG_OK ||
+        (st = fit_view(ns.wave[1], &nd.wave[1], nd.n_tr / 3, "hipMalloc characteristics")) != NDG_OK ||
         (st = fit_view(ns.tr[0], &nd.trace[0], nd.n_tr, "hipMalloc traces")) != NDG_OK ||
         (st = fit_view(ns.tr[1], &nd.trace[1], nd.n_tr, "hipMalloc traces")) != NDG_OK)
         return restore(st);
@@ -2307,7 +2340,6 @@ ndg_status adapt_on_device(ndg_mesh *mesh, int32_t N_max, int32_t max_split_leve
     if ((he = adapt_transfer(L, (const GroupSpan *)mesh->store[mesh->active].spans.p, d.q, Ln, spans_new, nd.q,
                              mesh->tab1d, w, s)) != hipSuccess)
         return hip_restore(he, "transfer kernel");
-    if ((he = hipMemsetAsync(nd.g, 0, sizeof(double) * nd.n_q, s)) != hipSuccess) return hip_restore(he, "hipMemset g");
     if ((he = launch_traces(nd, s)) != hipSuccess) return hip_restore(he, "traces kernel");
     AdaptCounts c2;
     if ((he = hipMemcpyAsync(&c2, w.counts.p, sizeof c2, hipMemcpyDeviceToHost, s)) != hipSuccess ||
@@ -2440,7 +2472,6 @@ extern "C" ndg_status ndg_adapt(ndg_mesh *mesh, int32_t N_max, int32_t max_split
         }
         carry_estimates(mesh, (size_t)K, same, keep);
     }
-    HIP_TRY(hipMemsetAsync(d.g, 0, sizeof(double) * d.n_q, mesh->stream), "hipMemset g");
     HIP_TRY(launch_traces(d, mesh->stream), "traces kernel");
     if (precision == NDG_PRECISION_FP32_COMPENSATED) {
         if ((st = ndg_mesh_set_precision(mesh, precision)) != NDG_OK) return st;
@@ -2481,7 +2512,7 @@ extern "C" ndg_status ndg_mesh_sides(ndg_mesh *mesh, int64_t *link, int8_t *hang
         if (link) link[i] = mesh->link[i];
         if (hang) hang[i] = (int8_t)mesh->hang_kind[i];
         if (next_small) next_small[i] = mesh->hang_second[i];
-        if (periodic) periodic[i] = (int8_t)mesh->periodic_link[i];
+        if (periodic) periodic[i] = (int8_t)(mesh->periodic_link[i] != 0);
         if (span) span[i] = mesh->span[i];
     }
     return NDG_OK;
@@ -2717,7 +2748,7 @@ void lagrange_at(const Tables &t, int N, double xi, std::vector<double> &out) {
 // The adjoint and the receivers need one order group, no boundary records and no mortar faces.
 ndg_status check_adjoint_mesh(const ndg_mesh *m, const char *who) {
     const DeviceMesh &d = m->d;
-    if (d.groups.size() != 1 || d.n_bc != 0 || d.n_faces != 0)
+    if (d.groups.size() != 1 || d.n_ghost != 0 || d.n_faces != 0)
         return fail(NDG_ERR_UNSUPPORTED, std::string(who) + ": needs a single-order mesh whose sides are all interior "
                                                             "or periodic");
     if (d.precision != NDG_PRECISION_FP64) return fail(NDG_ERR_UNSUPPORTED, std::string(who) + ": FP64 precision only");
@@ -3146,7 +3177,6 @@ extern "C" ndg_status ndg_adjoint_gradient(ndg_mesh *mesh, const ndg_receivers *
     double dc = 0.0;
     for (double v : hc) dc += v;
     HIP_TRY(hipMemcpyAsync(d.q, ckp(0), qb, hipMemcpyDeviceToDevice, s), "restore state");
-    HIP_TRY(hipMemsetAsync(d.g, 0, qb, s), "hipMemset g");
     HIP_TRY(launch_traces(d, s), "traces kernel");
     HIP_TRY(hipStreamSynchronize(s), "ndg_adjoint_gradient sync");
     if (J) *J = Jv;

@@ -171,6 +171,16 @@ std::vector<double> pack_tables(const Tables &t, int N) {
     out.insert(out.end(), M.begin(), M.end());
     for (int a = 0; a < nf; ++a)
         for (int i = 0; i < nf; ++i) out.push_back(Dh[i * nf + a]);
+    for (int i = 0; i < nf; ++i) out.push_back(t.tab[NDG_TABLE_LAGRANGE_RIGHT][N][i] / t.tab[NDG_TABLE_WEIGHTS][N][i]);
+    const int h = nf / 2;
+    for (int i = 0; i < h + nf % 2; ++i) {
+        const double *row = Dh.data() + i * nf;
+        if (i < h) {
+            for (int k = 0; k < h; ++k) out.push_back((row[k] + row[N - k]) / 2);
+            if (nf % 2) out.push_back(row[h]);
+        }
+        for (int k = 0; k < h; ++k) out.push_back((row[k] - row[N - k]) / 2);
+    }
     return out;
 }
 
