@@ -38,6 +38,7 @@ struct BcSide {
 // three traces written for every side (see DeviceMesh::trace_all), and the state and RK register
 // streamed past the caches (where together they have more than kStreamBytes).
 constexpr int kRkFirst = 1, kRkLast = 2, kTraceAll = 4, kStream = 8;
+constexpr int kRhsClock = 2;
 constexpr int64_t kStreamBytes = int64_t(160) << 20;
 
 // Element side whose face is non-conforming: its element flux trace is produced by the mortar
@@ -233,7 +234,9 @@ struct DeviceMesh {
     double *scratch = nullptr;   // reductions
     int64_t scratch_len = 0;
     int cur = 0;                 // trace and wave buffers holding those of the current state
-    double *clock = nullptr;     // [4]: step start time, then the 3 stage times
+    // [4]: the start time of a step that begins with trace buffer 0 and with 1 (see StageClock), and the
+    // time of a right-hand side outside the steps (kRhsClock)
+    double *clock = nullptr;
     double *q_out = nullptr;     // when set, FP64 stage kernels write the new state here (not in q)
     bool has_inflow = false;     // the stage time is read only by inflow ghosts
     // Wave speed c of the symmetric system p_t + c div(u, v) = 0, (u, v)_t + c grad p = 0: the
@@ -333,8 +336,8 @@ hipError_t adapt_copy_estimate(const LogicalMesh &L, const double *est, hipStrea
 // Kernel launchers (kernels.hip). All return hipSuccess or the first launch error.
 hipError_t launch_traces(const DeviceMesh &m, hipStream_t s);
 // Stage s of the RK step (mortar faces, then every order group, in the mesh's precision); the
-// stage time is read from clock[1 + s] (see launch_clock_begin). Flips `cur`.
-hipError_t launch_stage(DeviceMesh &m, int stage, double a, double gdt, hipStream_t s);
+// stage time comes from the device clock and dt. Flips `cur`.
+hipError_t launch_stage(DeviceMesh &m, int stage, double a, double gdt, double dt, hipStream_t s);
 hipError_t launch_rhs(DeviceMesh &m, double t, hipStream_t s);
 // FP32 compensated form: conversions between the FP64 state (q, g) and (qh, ql, g32), traces of
 // qh, and the stage.
@@ -342,13 +345,10 @@ hipError_t launch_to_c32(DeviceMesh &m, hipStream_t s);
 hipError_t launch_from_c32(DeviceMesh &m, hipStream_t s);
 hipError_t launch_traces_c32(const DeviceMesh &m, hipStream_t s);
 // One order group's stage kernel (of the mesh's precision); does not flip `cur`.
-hipError_t launch_group_stage(DeviceMesh &m, int group, int stage, double a, double gdt, hipStream_t s);
-// Device clock: begin writes the 3 stage times of a step starting at t (set != 0) or at clock[0];
-// end advances clock[0] by dt. Both are single-thread kernels, so a captured step replays with
-// the time advancing on the device. Meshes without inflow ghosts never read the time, and the
-// clock kernels are skipped for them.
-hipError_t launch_clock_begin(DeviceMesh &m, double t, int set, double dt, hipStream_t s);
-hipError_t launch_clock_end(DeviceMesh &m, double dt, hipStream_t s);
+hipError_t launch_group_stage(DeviceMesh &m, int group, int stage, double a, double gdt, double dt, hipStream_t s);
+// The start time of the next step (from the current trace buffer); the steps then advance it. Meshes
+// without inflow ghosts never read the time, and nothing is launched for them.
+hipError_t launch_clock_set(DeviceMesh &m, double t, hipStream_t s);
 // Autotuning: the largest elements-per-workgroup of the stage kernel for order N, and one launch
 // of group g's stage kernel that leaves the state and the current traces unchanged.
 int stage_max_epb(int N);

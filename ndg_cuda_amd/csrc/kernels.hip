@@ -37,6 +37,20 @@ struct Shape {
     static constexpr int THREADS = ((EPB * NE + 63) / 64) * 64;
 };
 
+// The stage's time, which the inflow ghost reads: the step's start time in device memory (so that a
+// captured step replays with the time advancing) plus the stage's part of the step; the step's last
+// stage leaves the next step's start time. One workgroup of one order group is given `next`.
+struct StageClock {
+    const double *start;
+    double part;   // b_s dt (include/solvers/Solver2D_t.tpp:16, :45-63), rounded on the host
+    double *next;  // null but in the step's last stage
+    double dt;
+    __device__ __forceinline__ double time() const { return *start + part; }
+    __device__ __forceinline__ void advance() const {
+        if (next && blockIdx.x == 0 && threadIdx.x == 0) *next = *start + dt;
+    }
+};
+
 // The reference plane wave g(x, t) (include/functions/analytical_solution.tpp:5-11).
 __device__ __forceinline__ void plane_wave(double x, double y, double t, double cw, double &p, double &u,
                                            double &v) {
@@ -181,8 +195,7 @@ traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side
 // The new state goes to q_out, which is q for the in-place step (q and q_out are therefore not
 // restrict; every value of q a workgroup reads precedes, through barriers, its writes).
 // A workgroup takes epb <= EPB consecutive elements (fewer gives more workgroups for a small
-// order group); remap != 0 applies the XCD-contiguous block order. t_ptr points at the stage time
-// in device memory (the inflow ghost reads it), so that a captured step can be replayed.
+// order group); remap != 0 applies the XCD-contiguous block order.
 //
 // LDS at N = 8 is 31,920 bytes, which the 1,280-byte allocation steps still let fit five times into
 // a CU's 160 KB.
@@ -333,7 +346,7 @@ struct SideRecord {
 template <int N>
 __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide *bc, const double *tq, const double *lm,
                                             const double *lp, const double *x, const double *tr_in,
-                                            const double *side_flux, int s, int k, const double *t_ptr, double cw,
+                                            const double *side_flux, int s, int k, const StageClock &clock, double cw,
                                             double &fa, double &fb) {
     constexpr int NF = N + 1, NFP = StageTile<N>::NFP, NEP = StageTile<N>::NEP;
     constexpr double c = kWaveSpeed;
@@ -382,7 +395,7 @@ __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide 
         const double interp = (x[N - k] + 1) / 2;
         const double X = bc->bx * interp + bc->ax * (1 - interp);
         const double Y = bc->by * interp + bc->ay * (1 - interp);
-        plane_wave(X, Y, *t_ptr, cw, pR, uR, vR);
+        plane_wave(X, Y, clock.time(), cw, pR, uR, vR);
     } else if (rec.kind == kKindTrace) {
         const double *nb = tr_in + rec.slot + (N - k);
         pR = nb[0];
@@ -402,7 +415,7 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
              const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ w_in,
              double *__restrict__ w_out, const double *__restrict__ tr_in, double *__restrict__ tr_out,
              double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
-             double gdt, const double *__restrict__ t_ptr, int epb, int remap, double cw) {
+             double gdt, StageClock clock, int epb, int remap, double cw) {
     const bool first = flags & kRkFirst, store_g = !(flags & kRkLast), once = flags & kStream;
     using S = LineShape<N>;
     using L = StageTile<N>;
@@ -430,6 +443,8 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
     // lanes past the tile's lines work on line 0 of its first element, so that every lane takes part
     // in the D^ broadcasts, and store nothing
     const int el = active ? lane / NF : 0, l = active ? lane % NF : 0;
+
+    clock.advance();
 
     __builtin_amdgcn_s_setprio(3);  // issue this workgroup's loads ahead of other waves' math
     // P0
@@ -522,7 +537,7 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
             const int item = tid + it * T;
             if (code[it] >= 0 || code[it] == INT32_MIN) continue;
             const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
-            record_flux<N>(rec[it], bc + (-1 - code[it]), s_q + fe * 3 * NEP, lm, lp, x, tr_in, side_flux, s, k, t_ptr,
+            record_flux<N>(rec[it], bc + (-1 - code[it]), s_q + fe * 3 * NEP, lm, lp, x, tr_in, side_flux, s, k, clock,
                            cw, s_f[item], s_f[EPB * 4 * NF + item]);
         }
     }
@@ -824,7 +839,7 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
                  const float *__restrict__ tab, float *__restrict__ qh, float2 *__restrict__ gl,
                  const float *__restrict__ tr_in, float *__restrict__ tr_out,
                  const float *__restrict__ side_flux, int64_t K, int first, float a, float gdt,
-                 const double *__restrict__ t_ptr, int epb, int remap, double cw) {
+                 StageClock clock, int epb, int remap, double cw) {
     using S = LineShape<N>;
     constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT;
     __shared__ float s_q[EPB * 3 * NE];
@@ -847,6 +862,8 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
     const int64_t e0 = blk * epb;
     const int nel = (int)min<int64_t>(epb, K - e0);
     const bool active = el < nel;
+
+    clock.advance();
 
     __builtin_amdgcn_s_setprio(3);  // issue this workgroup's loads ahead of other waves' math
     // P0
@@ -1010,7 +1027,7 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
                     const double X = rec.bx * interp + rec.ax * (1 - interp);
                     const double Y = rec.by * interp + rec.ay * (1 - interp);
                     double p64, u64, v64;
-                    plane_wave(X, Y, *t_ptr, cw, p64, u64, v64);
+                    plane_wave(X, Y, clock.time(), cw, p64, u64, v64);
                     pR = (float)p64;
                     uR = (float)u64;
                     vR = (float)v64;
@@ -1266,22 +1283,9 @@ estimate_kernel(const double *__restrict__ tab, const double *__restrict__ q, in
 }
 
 // ---------------------------------------------------------------------------------------------
-// Device clock of a step: clock[0] is the time at the start of the step, clock[1 + s] the time of
-// stage s, t + b_s dt (include/solvers/Solver2D_t.tpp:16, :45-63), rounded as the host loop does
-// (no contraction). set != 0 starts from t, else from clock[0]; clock_end advances clock[0] by dt.
-__global__ void clock_begin_kernel(double *clock, double t, int set, double dt) {
-#pragma clang fp contract(off)
-    if (threadIdx.x != 0) return;
-    const double t0 = set ? t : clock[0];
-    clock[0] = t0;
-    clock[1] = t0 + 0.0 * dt;
-    clock[2] = t0 + (1.0 / 3.0) * dt;
-    clock[3] = t0 + 0.75 * dt;
-}
-
-__global__ void clock_end_kernel(double *clock, double dt) {
-#pragma clang fp contract(off)
-    if (threadIdx.x == 0) clock[0] = clock[0] + dt;
+// Sets a value of the device clock (DeviceMesh::clock).
+__global__ void clock_set_kernel(double *clock, double t) {
+    if (threadIdx.x == 0) *clock = t;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1597,8 +1601,17 @@ static int stage_flags(const DeviceMesh &m) {
     return (m.trace_all ? kTraceAll : 0) | (16 * m.n_q > kStreamBytes ? kStream : 0);
 }
 
+// The clock has a start time for each trace buffer that a step can begin with: three stages flip it
+// three times, so the next step begins with the other one.
+static StageClock stage_clock(const DeviceMesh &m, const Group &G, int stage, double dt) {
+    constexpr double kB[3] = {0.0, 1.0 / 3.0, 0.75};
+    const int begin = m.cur ^ (stage & 1);
+    double *next = stage == 2 && m.has_inflow && &G == &m.groups[0] ? m.clock + (1 - begin) : nullptr;
+    return StageClock{m.clock + begin, kB[stage] * dt, next, dt};
+}
+
 template <int N>
-static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, hipStream_t s) {
+static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, double dt, hipStream_t s) {
     using S = LineShape<N>;
     const int epb = group_epb<N>(G, NDG_PRECISION_FP64);
     const int64_t blocks = (G.K + epb - 1) / epb;
@@ -1609,8 +1622,7 @@ static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, do
                        m.trace[1 - m.cur] + G.tr_off, nullptr, m.side_flux, G.K,
                        (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0) |
                            stage_flags(m), a, gdt,
-                       m.clock + 1 + stage, epb, G.tune[NDG_PRECISION_FP64].remap,
-                       m.wave_speed);
+                       stage_clock(m, G, stage, dt), epb, G.tune[NDG_PRECISION_FP64].remap, m.wave_speed);
     return hipGetLastError();
 }
 
@@ -1622,7 +1634,7 @@ static hipError_t rhs_n(DeviceMesh &m, const Group &G, hipStream_t s) {
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.q + G.q_off, nullptr,
                        m.wave[m.cur] + G.tr_off / 3, nullptr, m.trace[m.cur] + G.tr_off, nullptr, m.rhs + G.q_off, m.side_flux,
                        G.K, stage_flags(m), 0.0, 0.0,
-                       m.clock + 1, S::EPB, 1, m.wave_speed);
+                       StageClock{m.clock + kRhsClock, 0.0, nullptr, 0.0}, S::EPB, 1, m.wave_speed);
     return hipGetLastError();
 }
 
@@ -1653,14 +1665,16 @@ static hipError_t traces_c32_n(const DeviceMesh &m, const Group &G, hipStream_t 
 }
 
 template <int N>
-static hipError_t stage_c32_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, hipStream_t s) {
+static hipError_t stage_c32_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, double dt,
+                              hipStream_t s) {
     using S = LineShape<N>;
     const int epb = S::EPB;  // the low state words are kept in the full tiles' order
     const int64_t blocks = (G.K + epb - 1) / epb;
     hipLaunchKernelGGL(stage_c32_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, G.tab32, m.qh + G.q_off, m.gl32 + G.q_off,
                        m.trace32[m.cur] + G.tr_off, m.trace32[1 - m.cur] + G.tr_off,
-                       m.side_flux32, G.K, stage == 0 ? 1 : 0, (float)a, (float)gdt, m.clock + 1 + stage, epb,
+                       m.side_flux32, G.K, stage == 0 ? 1 : 0, (float)a, (float)gdt,
+                       stage_clock(m, G, stage, dt), epb,
                        G.tune[NDG_PRECISION_FP32_COMPENSATED].remap, m.wave_speed);
     return hipGetLastError();
 }
@@ -1673,12 +1687,12 @@ int stage_max_epb(int N) {
     return 0;
 }
 
-hipError_t launch_group_stage(DeviceMesh &m, int group, int stage, double a, double gdt, hipStream_t s) {
+hipError_t launch_group_stage(DeviceMesh &m, int group, int stage, double a, double gdt, double dt, hipStream_t s) {
     const Group &G = m.groups[group];
     if (m.precision == NDG_PRECISION_FP32_COMPENSATED) {
-        switch (G.N) { CASES_1(stage_c32_n, m, G, stage, a, gdt, s) }
+        switch (G.N) { CASES_1(stage_c32_n, m, G, stage, a, gdt, dt, s) }
     } else {
-        switch (G.N) { CASES_1(stage_n, m, G, stage, a, gdt, s) }
+        switch (G.N) { CASES_1(stage_n, m, G, stage, a, gdt, dt, s) }
     }
     return hipErrorInvalidValue;
 }
@@ -1686,7 +1700,7 @@ hipError_t launch_group_stage(DeviceMesh &m, int group, int stage, double a, dou
 // Autotuning probe: stage 0 form with a = 0 and gdt = 0, so that the state and the current traces
 // are left as they are.
 hipError_t launch_group_probe(DeviceMesh &m, int group, hipStream_t s) {
-    return launch_group_stage(m, group, 0, 0.0, 0.0, s);
+    return launch_group_stage(m, group, 0, 0.0, 0.0, 0.0, s);
 }
 
 
@@ -1728,17 +1742,18 @@ hipError_t launch_mortar(DeviceMesh &m, hipStream_t s) {
     return mortar_m<kMaxOrder + 1>(m, s);
 }
 
-hipError_t launch_stage(DeviceMesh &m, int stage, double a, double gdt, hipStream_t s) {
+hipError_t launch_stage(DeviceMesh &m, int stage, double a, double gdt, double dt, hipStream_t s) {
     hipError_t e = launch_mortar(m, s);
     if (e != hipSuccess) return e;
     for (int g = 0; g < (int)m.groups.size(); ++g)
-        if ((e = launch_group_stage(m, g, stage, a, gdt, s)) != hipSuccess) return e;
+        if ((e = launch_group_stage(m, g, stage, a, gdt, dt, s)) != hipSuccess) return e;
     m.cur = 1 - m.cur;
     return hipSuccess;
 }
 
 hipError_t launch_rhs(DeviceMesh &m, double t, hipStream_t s) {
-    hipError_t e = launch_clock_begin(m, t, 1, 0.0, s);
+    if (m.has_inflow) hipLaunchKernelGGL(clock_set_kernel, dim3(1), dim3(64), 0, s, m.clock + kRhsClock, t);
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if ((e = launch_mortar(m, s)) != hipSuccess) return e;
     return for_groups(m, [&](const Group &G) -> hipError_t {
@@ -1807,15 +1822,9 @@ hipError_t launch_delta_t(const DeviceMesh &m, double cfl, double *dt_dev, hipSt
     return hipGetLastError();
 }
 
-hipError_t launch_clock_begin(DeviceMesh &m, double t, int set, double dt, hipStream_t s) {
+hipError_t launch_clock_set(DeviceMesh &m, double t, hipStream_t s) {
     if (!m.has_inflow) return hipSuccess;  // nothing reads the stage time
-    hipLaunchKernelGGL(clock_begin_kernel, dim3(1), dim3(64), 0, s, m.clock, t, set, dt);
-    return hipGetLastError();
-}
-
-hipError_t launch_clock_end(DeviceMesh &m, double dt, hipStream_t s) {
-    if (!m.has_inflow) return hipSuccess;
-    hipLaunchKernelGGL(clock_end_kernel, dim3(1), dim3(64), 0, s, m.clock, dt);
+    hipLaunchKernelGGL(clock_set_kernel, dim3(1), dim3(64), 0, s, m.clock + m.cur, t);
     return hipGetLastError();
 }
 

@@ -1480,20 +1480,6 @@ extern "C" ndg_status ndg_get_state(ndg_mesh *mesh, double *p, double *u, double
 
 namespace {
 
-// The right-hand side at time t without disturbing a running solve: launch_rhs sets the device
-// clock (which the next step of ndg_solve continues from) to t, so its 4 values are saved before
-// and put back after.
-ndg_status rhs_keeping_clock(ndg_mesh *mesh, double t) {
-    DeviceMesh &d = mesh->d;
-    double saved[4];
-    HIP_TRY(hipMemcpyAsync(saved, d.clock, sizeof saved, hipMemcpyDeviceToHost, mesh->stream), "save clock");
-    HIP_TRY(hipStreamSynchronize(mesh->stream), "save clock sync");
-    HIP_TRY(launch_rhs(d, t, mesh->stream), "rhs kernel");
-    HIP_TRY(hipMemcpyAsync(d.clock, saved, sizeof saved, hipMemcpyHostToDevice, mesh->stream), "restore clock");
-    HIP_TRY(hipStreamSynchronize(mesh->stream), "restore clock sync");
-    return NDG_OK;
-}
-
 // The uniform-grid output of get_solution (5 planes: x, y, p, u, v) or, with `complete`, of
 // get_complete_solution (11 planes: also dq/dt of the current state at `time` and the plane-wave
 // errors), each plane [K][n][n] in the caller's element order; a null plane pointer is skipped.
@@ -1511,7 +1497,7 @@ ndg_status interpolated_output(ndg_mesh *mesh, const char *who, bool complete, d
             const ndg_status rs = fit_view(mesh->store[mesh->active].rhs, &d.rhs, d.n_q, "hipMalloc rhs");
             if (rs != NDG_OK) return rs;
         }
-        if ((st = rhs_keeping_clock(mesh, time)) != NDG_OK) return st;
+        HIP_TRY(launch_rhs(d, time, mesh->stream), "rhs kernel");
     }
     const int64_t K = d.K, nn = n * n;
     const int n_planes = complete ? 11 : 5;
@@ -1633,7 +1619,7 @@ extern "C" ndg_status ndg_compute_rhs(ndg_mesh *mesh, double t, double *Gp, doub
         const ndg_status rs = fit_view(mesh->store[mesh->active].rhs, &d.rhs, d.n_q, "hipMalloc rhs");
         if (rs != NDG_OK) return rs;
     }
-    if ((st = rhs_keeping_clock(mesh, t)) != NDG_OK) return st;
+    HIP_TRY(launch_rhs(d, t, mesh->stream), "rhs kernel");
     double *const outs[3] = {Gp, Gu, Gv};
     return copy_state(mesh, d.rhs, outs, true, "download rhs");
 }
@@ -1658,11 +1644,10 @@ void drop_graphs(ndg_mesh *m) {
     m->graph_precision = -1;
 }
 
-// One RK step from the device clock (clock_begin with set = 0), launched on s; with `parallel`
+// One RK step from the device clock, launched on s; with `parallel`
 // the order groups of each stage are forked onto side streams and joined (graph branches).
 ndg_status launch_step_body(ndg_mesh *m, double dt, bool parallel, hipStream_t s) {
     DeviceMesh &d = m->d;
-    HIP_TRY(launch_clock_begin(d, 0.0, 0, dt, s), "clock kernel");
     const int ng = (int)d.groups.size();
     for (int st = 0; st < 3; ++st) {
         HIP_TRY(launch_mortar(d, s), "mortar kernel");
@@ -1679,17 +1664,16 @@ ndg_status launch_step_body(ndg_mesh *m, double dt, bool parallel, hipStream_t s
             HIP_TRY(hipEventRecord(m->side_events[0], s), "fork");
             for (int g : gorder) {
                 HIP_TRY(hipStreamWaitEvent(m->side_streams[g], m->side_events[0], 0), "fork wait");
-                HIP_TRY(launch_group_stage(d, g, st, kAm[st], kGm[st] * dt, m->side_streams[g]), "stage kernel");
+                HIP_TRY(launch_group_stage(d, g, st, kAm[st], kGm[st] * dt, dt, m->side_streams[g]), "stage kernel");
                 HIP_TRY(hipEventRecord(m->side_events[1 + g], m->side_streams[g]), "join");
                 HIP_TRY(hipStreamWaitEvent(s, m->side_events[1 + g], 0), "join wait");
             }
         } else {
             for (int g = 0; g < ng; ++g)
-                HIP_TRY(launch_group_stage(d, g, st, kAm[st], kGm[st] * dt, s), "stage kernel");
+                HIP_TRY(launch_group_stage(d, g, st, kAm[st], kGm[st] * dt, dt, s), "stage kernel");
         }
         d.cur = 1 - d.cur;
     }
-    HIP_TRY(launch_clock_end(d, dt, s), "clock kernel");
     return NDG_OK;
 }
 
@@ -1766,7 +1750,7 @@ ndg_status step_from_clock(ndg_mesh *m, double dt) {
 
 extern "C" ndg_status ndg_step(ndg_mesh *mesh, double t, double dt) {
     if (!mesh) return fail(NDG_ERR_INVALID, "ndg_step: null mesh");
-    HIP_TRY(launch_clock_begin(mesh->d, t, 1, dt, mesh->stream), "clock kernel");
+    HIP_TRY(launch_clock_set(mesh->d, t, mesh->stream), "clock kernel");
     return step_from_clock(mesh, dt);
 }
 
@@ -2204,6 +2188,7 @@ ndg_status adapt_split(ndg_mesh *mesh, const std::vector<int32_t> &ref, const st
     if (coords_dev) (void)hipFree(coords_dev);
     if (st != NDG_OK) return restore(st);
     nd.wave_speed = d.wave_speed;
+    nd.cur = d.cur;  // the clock's start time goes with the trace buffer
     carry_tuning(d, nd);
     d = nd;
     mesh->active ^= 1;
@@ -2333,7 +2318,7 @@ ndg_status adapt_on_device(ndg_mesh *mesh, int32_t N_max, int32_t max_split_leve
     nd.clock = mesh->clock;
     nd.has_inflow = d.has_inflow;
     nd.wave_speed = d.wave_speed;
-    nd.cur = 0;
+    nd.cur = d.cur;  // the clock's start time goes with the trace buffer
     carry_tuning(d, nd);
     if ((he = adapt_layout_fill(Ln, spans_new, mesh->mortar_key_dev, nd, w, s)) != hipSuccess)
         return hip_restore(he, "adaptation layout");
@@ -2459,7 +2444,7 @@ extern "C" ndg_status ndg_adapt(ndg_mesh *mesh, int32_t N_max, int32_t max_split
     if (recs_dev) (void)hipFree(recs_dev);
     if (st != NDG_OK) return restore(st);
     nd.wave_speed = d.wave_speed;
-    nd.cur = 0;
+    nd.cur = d.cur;  // the clock's start time goes with the trace buffer
     carry_tuning(d, nd);
     d = nd;
     mesh->active ^= 1;
@@ -2547,7 +2532,7 @@ ndg_status solve_impl(ndg_mesh *mesh, double cfl, const double *times, int64_t n
     if (fn)
         for (int64_t k = 0; k < n_times; ++k)
             if (time >= times[k] && time < times[k] + dt && (st = output()) != NDG_OK) return st;
-    HIP_TRY(launch_clock_begin(mesh->d, time, 1, dt0, mesh->stream), "clock kernel");
+    HIP_TRY(launch_clock_set(mesh->d, time, mesh->stream), "clock kernel");
     while (time < t_end) {
         ++steps;
         dt = dt0;
@@ -2571,7 +2556,7 @@ ndg_status solve_impl(ndg_mesh *mesh, double cfl, const double *times, int64_t n
             if ((st = ndg_adapt(mesh, mesh->tables->t.N_max, mesh->max_split_level, &raised)) != NDG_OK) return st;
             if (raised > 0) {
                 if ((st = ndg_get_delta_t(mesh, cfl, &dt0)) != NDG_OK) return st;
-                HIP_TRY(launch_clock_begin(mesh->d, time, 1, dt0, mesh->stream), "clock kernel");
+                HIP_TRY(launch_clock_set(mesh->d, time, mesh->stream), "clock kernel");
             }
         }
     }
@@ -2643,7 +2628,7 @@ extern "C" ndg_status ndg_run_steps(ndg_mesh *mesh, double cfl, int64_t n_steps,
     ndg_status st = ndg_get_delta_t(mesh, cfl, &dt);
     if (st != NDG_OK) return st;
     double time = time_io ? *time_io : 0.0;
-    HIP_TRY(launch_clock_begin(mesh->d, time, 1, dt, mesh->stream), "clock kernel");
+    HIP_TRY(launch_clock_set(mesh->d, time, mesh->stream), "clock kernel");
     for (int64_t k = 0; k < n_steps; ++k) {
         if ((st = step_from_clock(mesh, dt)) != NDG_OK) return st;
         time += dt;
@@ -2824,7 +2809,7 @@ extern "C" ndg_status ndg_record_receivers(ndg_mesh *mesh, const ndg_receivers *
     if (n_steps == 0) return NDG_OK;
     if ((st = dev_alloc(out, sizeof(double) * R.n * n_steps, "hipMalloc records")) != NDG_OK) return st;
     DeviceMesh &d = mesh->d;
-    HIP_TRY(launch_clock_begin(d, 0.0, 1, dt, mesh->stream), "clock kernel");
+    HIP_TRY(launch_clock_set(d, 0.0, mesh->stream), "clock kernel");
     for (int64_t n = 0; n < n_steps; ++n) {
         if ((st = step_from_clock(mesh, dt)) != NDG_OK) return st;
         HIP_TRY(launch_record(d, R.elem.as<int64_t>(), R.w.as<double>(), R.n, out.as<double>() + n * R.n,
@@ -2864,7 +2849,7 @@ extern "C" ndg_status ndg_record_receivers_noalloc(ndg_mesh *mesh, const ndg_rec
     HIP_TRY(hipMemcpyAsync(elem_dev, elem.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice, s), "upload receivers");
     HIP_TRY(hipMemcpyAsync(w_dev, w.data(), sizeof(double) * n * ne, hipMemcpyHostToDevice, s), "upload receivers");
     // direct launches (a captured step graph would be instantiated on first use)
-    HIP_TRY(launch_clock_begin(d, 0.0, 1, dt, s), "clock kernel");
+    HIP_TRY(launch_clock_set(d, 0.0, s), "clock kernel");
     for (int64_t k = 0; k < n_steps; ++k) {
         if ((st = launch_step_body(mesh, dt, false, s)) != NDG_OK) return st;
         HIP_TRY(launch_record(d, elem_dev, w_dev, (int)n, rec_dev + k * n, s), "record kernel");
@@ -3002,7 +2987,7 @@ extern "C" ndg_status ndg_adjoint_gradient(ndg_mesh *mesh, const ndg_receivers *
                 double *out = stage < 2 ? stp(k, j - n0, stage + 1) : (j + 1 < n1 ? stp(k, j + 1 - n0, 0) : q_main);
                 dm.q = in;
                 dm.q_out = out;
-                HIP_TRY(launch_stage(dm, stage, kAm[stage], kGm[stage] * dt, st_), "stage kernel");
+                HIP_TRY(launch_stage(dm, stage, kAm[stage], kGm[stage] * dt, dt, st_), "stage kernel");
                 if (stage == 2 && record) {
                     dm.q = out;
                     HIP_TRY(launch_record(dm, R.elem.as<int64_t>(), R.w.as<double>(), R.n,
@@ -3019,7 +3004,7 @@ extern "C" ndg_status ndg_adjoint_gradient(ndg_mesh *mesh, const ndg_receivers *
 
     // Forward pass: checkpoints; the kept segments keep their stage inputs right away. With stage
     // records: the RK register's pressure at the receivers after every stage as well.
-    HIP_TRY(launch_clock_begin(d, 0.0, 1, dt, s), "clock kernel");
+    HIP_TRY(launch_clock_set(d, 0.0, s), "clock kernel");
     if (records) {
         HIP_TRY(hipMemcpyAsync(ckp(0), d.q, qb, hipMemcpyDeviceToDevice, s), "checkpoint");
         // the RK register is recorded after every stage, the last included
@@ -3030,7 +3015,7 @@ extern "C" ndg_status ndg_adjoint_gradient(ndg_mesh *mesh, const ndg_receivers *
         } keep_last_rk{d};
         for (int64_t n = 0; n < n_steps; ++n) {
             for (int stage = 0; stage < 3; ++stage) {
-                HIP_TRY(launch_stage(d, stage, kAm[stage], kGm[stage] * dt, s), "stage kernel");
+                HIP_TRY(launch_stage(d, stage, kAm[stage], kGm[stage] * dt, dt, s), "stage kernel");
                 HIP_TRY(launch_record_rk(d, R.elem.as<int64_t>(), R.w_t.as<double>(), R.n,
                                          recs_g.as<double>() + (n * 3 + stage) * R.n, s),
                         "record kernel");
