@@ -164,7 +164,7 @@ void arena_free(Arena &a);
 // The buffers of one device mesh. A mesh keeps two: the current one, and the one an adaptation
 // builds the next mesh into (the state is transferred from the first to the second).
 struct DeviceStore {
-    Arena verts, side_nb, bc, faces, side_flux, side_flux32, q, g, tr[2], wave[2], rhs, scratch, qh, gl32, tr32[2];
+    Arena verts, side_nb, bc, faces, side_flux, side_flux32, q, g, tr[2], wave[2], rhs, scratch, qh, gl32, tr32[2], wave32[2];
     Arena spans;  // GroupSpan[kMaxOrder + 1] of the layout
 };
 void store_free(DeviceStore &s);
@@ -250,10 +250,11 @@ struct DeviceMesh {
     // every stage); otherwise that store is skipped, no later stage reading it.
     bool keep_last_rk = false;
     float *qh = nullptr;
-    // RK register (x) and low state word (y) of each value, interleaved so that a line owner
-    // reads and writes both with one 8-byte access; transposed within each (element, field) block
+    // RK register (x) and low state word (y) of each value, interleaved, in the tile order of the RK
+    // register (n_g values)
     float2 *gl32 = nullptr;
     float *trace32[2] = {nullptr, nullptr};
+    float *wave32[2] = {nullptr, nullptr};
 };
 
 // Position of the order-N group in the device layout (one per order 0..kMaxOrder; K = 0 when the

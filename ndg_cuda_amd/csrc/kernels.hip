@@ -764,19 +764,19 @@ __device__ __forceinline__ void two_sum_add(float &hi, float &lo, float d) {
     hi = h;
 }
 
-// Position in the FP32 form's gl32 (tile order [f][j][el][i] of tiles of epb elements, the last
-// tile of K - tile start elements) of value (element e, field f, node (i, j)); nf = N + 1.
-__device__ __forceinline__ int64_t c32_tile_index(int64_t e, int f, int i, int j, int nf, int epb, int64_t K) {
-    const int64_t e0 = e - e % epb;
-    const int nel = (int)min<int64_t>(epb, K - e0), el = (int)(e - e0);
-    return e0 * 3 * nf * nf + ((int64_t)(f * nf + j) * nel + el) * nf + i;
+// Position in the FP32 form's gl32 (the RK register's order in tiles of epb elements and runs of `run`
+// values, see stage_kernel) of value (element e, field f, node (i, j)); nf = N + 1.
+__device__ __forceinline__ int64_t c32_tile_index(int64_t e, int f, int i, int j, int nf, int epb, int run) {
+    const int64_t blk = e / epb, base = (blk * 3 + f) * nf * run;
+    const int at = (int)(e - blk * epb) * nf + i;
+    return j < nf / 2 * 2 ? base + (j & ~1) * run + 2 * at + (j & 1) : base + j * run + at;
 }
 
 // q and qh are in reference node order; gl32 (RK register in x, low state word in y) is in the
 // FP32 stage kernel's tile order. Thread r writes one float2. The RK register carries no value
 // from one step to the next, so g is copied word for word whatever its order.
 __global__ void to_c32_kernel(const double *__restrict__ q, float *__restrict__ qh, float2 *__restrict__ gl32,
-                              int64_t n, int nf, int epb) {
+                              int64_t n, int nf, int epb, int run) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const int ne = nf * nf, node = (int)(r % ne), i = node / nf, j = node % nf;
@@ -785,27 +785,34 @@ __global__ void to_c32_kernel(const double *__restrict__ q, float *__restrict__ 
     const double v = q[r];
     const float h = (float)v;
     qh[r] = h;
-    gl32[c32_tile_index(e, f, i, j, nf, epb, n / (3 * ne))] = make_float2(0.f, (float)(v - (double)h));
+    gl32[c32_tile_index(e, f, i, j, nf, epb, run)] = make_float2(0.f, (float)(v - (double)h));
 }
 
 __global__ void from_c32_kernel(const float *__restrict__ qh, const float2 *__restrict__ gl32,
-                                double *__restrict__ q, int64_t n, int nf, int epb) {
+                                double *__restrict__ q, int64_t n, int nf, int epb, int run) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const int ne = nf * nf, node = (int)(r % ne), i = node / nf, j = node % nf;
     const int64_t e = r / (3 * ne);
     const int f = (int)((r / ne) % 3);
-    const float2 w = gl32[c32_tile_index(e, f, i, j, nf, epb, n / (3 * ne))];
+    const float2 w = gl32[c32_tile_index(e, f, i, j, nf, epb, run)];
     q[r] = (double)qh[r] + (double)w.y;
+}
+
+// p + u.n with one fused product, as every place must round it (left to the compiler, a pair of products
+// becomes a vector of two here and there and loses it).
+__device__ __forceinline__ float characteristic32(float p, float u, float v, float nx, float ny) {
+    return p + fmaf(v, ny, u * nx);
 }
 
 template <int N>
 __global__ void __launch_bounds__(192)
-traces_c32_kernel(const float *__restrict__ tab, const float *__restrict__ qh, float *__restrict__ tr,
-                  int64_t K) {
+traces_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb, const BcSide *__restrict__ bc,
+                  const float *__restrict__ tab, const float *__restrict__ qh, float *__restrict__ tr,
+                  float *__restrict__ w, int64_t K) {
     using S = LineShape<N>;
     constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T;
-    __shared__ float s_q[EPB * 3 * NE];
+    __shared__ float s_q[EPB * 3 * NE], s_tr[EPB * 12 * NF];
     const float *lm = tab + NF * NF;
     const float *lp = lm + NF;
     const int tid = threadIdx.x;
@@ -824,31 +831,200 @@ traces_c32_kernel(const float *__restrict__ tab, const float *__restrict__ qh, f
             t1 += lp[j] * col;
             t3 += lm[j] * col;
         }
-        float *to = tr + (e0 + el) * 12 * NF + f * NF;
+        float *to = s_tr + el * 12 * NF + f * NF;
         to[l] = t0;
         to[6 * NF + (N - l)] = t2;
         to[3 * NF + l] = t1;
         to[9 * NF + (N - l)] = t3;
     }
+    __syncthreads();
+    for (int r = tid; r < nel * 12 * NF; r += T) tr[e0 * 12 * NF + r] = s_tr[r];
+    for (int r = tid; r < nel * 4 * NF; r += T) {
+        const int fe = r / (4 * NF), s = (r / NF) % 4, k = r % NF;
+        double nx, ny;
+        side_normal(verts, side_nb, bc, e0 + fe, s, nx, ny);
+        const float *t = s_tr + fe * 12 * NF + s * 3 * NF + k;
+        w[e0 * 4 * NF + r] = characteristic32(t[0], t[NF], t[2 * NF], (float)nx, (float)ny);
+    }
 }
 
+// n floats from p, in 16-byte words, bounds-checked as Buffer's values are.
+struct Buffer32 {
+    __amdgpu_buffer_rsrc_t rsrc;
+    __device__ __forceinline__ Buffer32(const float *p, int n)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc((void *)p, 0, n * 4, 0x00027000)) {}
+    __device__ __forceinline__ float load(int i) const {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, i * 4, 0, 0));
+    }
+    template <int kHow>
+    __device__ __forceinline__ float2 load2(int i) const {
+        return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, i * 4, 0, kHow));
+    }
+    template <int kHow>
+    __device__ __forceinline__ float4 load4(int i) const {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, i * 4, 0, kHow));
+    }
+    __device__ __forceinline__ void store(int i, float v) const {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc, i * 4, 0, 0);
+    }
+    template <int kHow>
+    __device__ __forceinline__ void store2(int i, float2 v) const {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Buffer::Words2, v), rsrc, i * 4, 0, kHow);
+    }
+    template <int kHow>
+    __device__ __forceinline__ void store4(int i, float4 v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(Buffer::Words4, v), rsrc, i * 4, 0, kHow);
+    }
+};
+
+// LaneTable of floats.
+template <int L>
+struct LaneTable32 {
+    float v[(L + 15) / 16];
+    __device__ __forceinline__ void load(const float *t) {
+        const int m = threadIdx.x & 15;
+#pragma unroll
+        for (int p = 0; p < (L + 15) / 16; ++p) v[p] = t[min(p * 16 + m, L - 1)];
+    }
+};
+
+// a[i S] (+)= D(entry E + i Step) F for the R rows i, a column of D^ at a time: the entry is a DPP operand of the
+// multiply-add (the compiler moves it to a register first, with a wait: three issues instead of
+// one). A block first waits out the two cycles that a register written just before it takes to reach
+// a DPP instruction, and within one every row is another register.
+template <bool kSet, int E, int Step, int R, int L>
+__device__ __forceinline__ void rows32(const LaneTable32<L> &D, float F, float *a) {
+#define NDG_MAC32(o, d, f, e) "v_fmac_f32_dpp %" #o ", %" #d ", %" #f " row_newbcast:%" #e " row_mask:0xf bank_mask:0xf\n\t"
+#define NDG_MUL32(o, d, f, e) "v_mul_f32_dpp %" #o ", %" #d ", %" #f " row_newbcast:%" #e " row_mask:0xf bank_mask:0xf\n\t"
+#define NDG_ENTRY32(i) D.v[(E + (i) * Step) / 16]
+#define NDG_LANE32(i) (E + (i) * Step) % 16
+    if constexpr (R > 4) {
+        rows32<kSet, E, Step, 4>(D, F, a);
+        rows32<kSet, E + 4 * Step, Step, R - 4>(D, F, a + 4);
+    } else if constexpr (R == 4 && kSet) {
+        asm volatile("s_nop 1\n\t" NDG_MUL32(0, 4, 8, 9) NDG_MUL32(1, 5, 8, 10) NDG_MUL32(2, 6, 8, 11)
+                         NDG_MUL32(3, 7, 8, 12)
+                     : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3])
+                     : "v"(NDG_ENTRY32(0)), "v"(NDG_ENTRY32(1)), "v"(NDG_ENTRY32(2)), "v"(NDG_ENTRY32(3)), "v"(F),
+                       "n"(NDG_LANE32(0)), "n"(NDG_LANE32(1)), "n"(NDG_LANE32(2)), "n"(NDG_LANE32(3)));
+    } else if constexpr (R == 4) {
+        asm volatile("s_nop 1\n\t" NDG_MAC32(0, 4, 8, 9) NDG_MAC32(1, 5, 8, 10) NDG_MAC32(2, 6, 8, 11)
+                         NDG_MAC32(3, 7, 8, 12)
+                     : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                     : "v"(NDG_ENTRY32(0)), "v"(NDG_ENTRY32(1)), "v"(NDG_ENTRY32(2)), "v"(NDG_ENTRY32(3)), "v"(F),
+                       "n"(NDG_LANE32(0)), "n"(NDG_LANE32(1)), "n"(NDG_LANE32(2)), "n"(NDG_LANE32(3)));
+    } else if constexpr (R > 0) {
+        if constexpr (kSet)
+            asm volatile("s_nop 1\n\t" NDG_MUL32(0, 1, 2, 3)
+                         : "=&v"(a[0])
+                         : "v"(NDG_ENTRY32(0)), "v"(F), "n"(NDG_LANE32(0)));
+        else
+            asm volatile("s_nop 1\n\t" NDG_MAC32(0, 1, 2, 3)
+                         : "+&v"(a[0])
+                         : "v"(NDG_ENTRY32(0)), "v"(F), "n"(NDG_LANE32(0)));
+        rows32<kSet, E + Step, Step, R - 1>(D, F, a + 1);
+    }
+#undef NDG_MAC32
+#undef NDG_MUL32
+#undef NDG_ENTRY32
+#undef NDG_LANE32
+}
+
+// a = D^ F, each row summed in the order of the line's nodes.
+template <int NF, int k = 0>
+__device__ __forceinline__ void contract32(const LaneTable32<NF * NF> &D, const float *F, float *a) {
+    rows32<k == 0, k, NF, NF>(D, F[k], a);
+    if constexpr (k + 1 < NF) contract32<NF, k + 1>(D, F, a);
+}
+
+// record_flux in FP32: (w_L - w_R)/2, (w_L + w_R)/2 and, for a mortar side, the three flux components.
 template <int N>
-__global__ void __launch_bounds__(192)
+__device__ __forceinline__ void record_flux32(const SideRecord &rec, const BcSide *bc, const float (&tr)[3],
+                                              const double *x64, const float *tr_in, const float *side_flux, int k,
+                                              const StageClock &clock, double cw, float &fa, float &fb, float &fc) {
+    constexpr int NF = N + 1;
+    const int kind = rec.kind;
+    if (kind == kKindMortar) {
+        const float *sfl = side_flux + bc->slot + k;
+        float f0 = sfl[0], f1 = sfl[NF], f2 = sfl[2 * NF];
+        const int n_faces = bc->n_faces;
+        for (int m = 1; m < n_faces; ++m) {
+            const float *s2 = sfl + m * 3 * NF;
+            f0 += s2[0];
+            f1 += s2[NF];
+            f2 += s2[2 * NF];
+        }
+        fa = f0;
+        fb = f1;
+        fc = f2;
+        return;
+    }
+    const float pL = tr[0], uL = tr[1], vL = tr[2];
+    const float nx = (float)rec.nx, ny = (float)rec.ny, gs = (float)rec.sf;
+    float pR = 0.f, uR = 0.f, vR = 0.f;
+    if (kind == NDG_BC_WALL || kind == NDG_BC_SYMMETRY) {
+        const float tx = (float)bc->tx, ty = (float)bc->ty;
+        pR = pL * gs;
+        const float ux = uL * gs, uy = vL * gs;
+        const float l0 = -fmaf(uy, ny, ux * nx);
+        const float l1 = fmaf(uy, ty, ux * tx);
+        uR = fmaf(tx, l1, nx * l0);
+        vR = fmaf(ty, l1, ny * l0);
+    } else if (kind == NDG_BC_OUTFLOW) {
+        pR = pL * gs;
+        uR = uL * gs;
+        vR = vL * gs;
+    } else if (kind == NDG_BC_INFLOW) {
+        const double interp = (x64[N - k] + 1) / 2;
+        const double X = bc->bx * interp + bc->ax * (1 - interp);
+        const double Y = bc->by * interp + bc->ay * (1 - interp);
+        double p64, u64, v64;
+        plane_wave(X, Y, clock.time(), cw, p64, u64, v64);
+        pR = (float)p64;
+        uR = (float)u64;
+        vR = (float)v64;
+    } else if (kind == kKindTrace) {
+        const float *nb = tr_in + bc->slot + (N - k);
+        pR = nb[0];
+        uR = nb[NF];
+        vR = nb[2 * NF];
+    }
+    const float wL = characteristic32(pL, uL, vL, nx, ny);
+    const float wR = characteristic32(pR, -uR, -vR, nx, ny);
+    fa = (wL - wR) * 0.5f;
+    fb = (wL + wR) * 0.5f;
+}
+
+// The FP32 stage: stage_kernel's phases, exchange and streaming; every sum in the order and every
+// product with the rounding of the form without them, so the results are the same bit for bit (the
+// D^ entries are therefore not folded into even and odd parts, and a mortar side keeps its three flux
+// components). gl holds the RK register and the low state word of each value, interleaved, in the
+// RK register's tile order of the shape's full tiles (the launch always uses them, so the low words
+// keep their places from one step to the next). A side with a record reads its own traces back, loaded
+// with the tile; formed again from the tile's lines they cost a wall mesh of 96 x 96, N = 8 0.4 us.
+// Bound by memory at large sizes: 384 x 384, N = 7 in 127 us a launch, 157 us with three traces
+// exchanged a point, 4-byte cached accesses and D^ in scalar registers; 512 x 512, N = 8: 297 and
+// 350 us; 256 x 256, N = 12: 169 and 182 us; 48 x 48, N = 16: 16.4 and 18.2 us. Where one round of
+// workgroups fills the chip the wait for the tile decides: 128 x 128, N = 8: 23.6 and 24.1 us, 96 x 96:
+// 14.1 and 13.9 us.
+template <int N>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 9 ? 5 : 4)))
 stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
                  const BcSide *__restrict__ bc, const double *__restrict__ tab64,
                  const float *__restrict__ tab, float *__restrict__ qh, float2 *__restrict__ gl,
-                 const float *__restrict__ tr_in, float *__restrict__ tr_out,
-                 const float *__restrict__ side_flux, int64_t K, int first, float a, float gdt,
-                 StageClock clock, int epb, int remap, double cw) {
+                 const float *__restrict__ w_in, float *__restrict__ w_out, const float *__restrict__ tr_in,
+                 float *__restrict__ tr_out, const float *__restrict__ side_flux, int64_t K, int flags, float a, float gdt,
+                 StageClock clock, int remap, double cw) {
+    const bool first = flags & kRkFirst, once = flags & kStream;
     using S = LineShape<N>;
-    constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT;
-    __shared__ float s_q[EPB * 3 * NE];
-    __shared__ float s_d[EPB * 3 * NE];
-    __shared__ float s_tr[EPB * 12 * NF];
+    constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT, NFP = NF | 1, NEP = NF * NFP;
+    constexpr int QP4 = (EPB * 3 * NE + 31 + 4 * T - 1) / (4 * T);  // 16-byte words of the tile per thread
+    constexpr int run = rk_run<N>(EPB);
+    __shared__ float s_q[EPB * 3 * NEP];
+    __shared__ float s_d[EPB * 3 * NEP];    // d_xi, then the new traces on sides 1 and 3
+    __shared__ float s_f[EPB * 12 * NF];    // fluxes, then the new traces on sides 0 and 2
     __shared__ float s_met[EPB * 4 * NF];
-    __shared__ float s_side[EPB * 4 * 3];
-    __shared__ double s_v[EPB * 8];
-    const float *Dh = tab;
+    __shared__ float s_side[EPB * 4 * 3];   // outward normal and edge Jacobian (negative: a mortar side)
     const float *lm = tab + NF * NF;
     const float *lp = lm + NF;
     const float *winv = lp + 3 * NF;
@@ -857,11 +1033,12 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
     const int tid = threadIdx.x;
     const int f = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int el = lane / NF, l = lane % NF;
     const int64_t blk = remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
-    const int64_t e0 = blk * epb;
-    const int nel = (int)min<int64_t>(epb, K - e0);
-    const bool active = el < nel;
+    const int64_t e0 = blk * EPB;
+    const int nel = (int)min<int64_t>(EPB, K - e0);
+    const int n_val = nel * 3 * NE, n_pt = nel * 4 * NF;
+    const bool active = lane < nel * NF;
+    const int el = active ? lane / NF : 0, l = active ? lane % NF : 0;
 
     clock.advance();
 
@@ -871,272 +1048,280 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
         const int item = tid + it * T;
-        code[it] = item < nel * 4 * NF ? side_nb[(e0 + item / NF / 4) * 4 + (item / NF) % 4] : INT32_MIN;
+        code[it] = item < n_pt ? side_nb[e0 * 4 + item / NF] : INT32_MIN;
     }
-    float qreg[S::QPT];
+    double P[8];  // the element's vertices; in the wave that forms the sides, from side l's first one on
+    const int side = min(l, 3);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) P[k] = verts[(e0 + el) * 8 + (f == 2 ? (2 * side + k) & 7 : k)];
+    const int32_t side_code = side_nb[(e0 + el) * 4 + side];
     const float *qg = qh + e0 * 3 * NE;
+    const int lead = (int)(((uintptr_t)qg >> 2) & 31), end = lead + n_val;
+    // words wholly inside the tile by the bounds check; the values of a last partial word one by one
+    const Buffer32 q_buf(qg - lead, end & ~3), q_all(qg - lead, end), w_buf(w_in + e0 * 4 * NF, n_pt);
+    const Buffer32 gl_buf((const float *)(gl + (blk * 3 + f) * NF * run), 2 * NF * run);
+    float4 qreg[QP4], gl_old[NF / 2];
+    float own[FPT], q_rest = 0.f;
+    float2 gl_odd = make_float2(0.f, 0.f);
+    LaneTable32<NF * NF> Dh;
+    auto load_tile = [&](auto how) {
+        constexpr int kHow = decltype(how)::value;
 #pragma unroll
-    for (int it = 0; it < S::QPT; ++it) {
-        const int r = tid + it * T;
-        qreg[it] = r < nel * 3 * NE ? qg[r] : 0.f;
-    }
-    double vreg[S::VPT];
+        for (int it = 0; it < QP4; ++it) qreg[it] = q_buf.load4<kHow>(4 * (tid + it * T));
+        q_rest = q_all.load((end & ~3) + (tid & 3));
+        Dh.load(tab);
 #pragma unroll
-    for (int it = 0; it < S::VPT; ++it) {
-        const int r = tid + it * T;
-        vreg[it] = r < nel * 8 ? verts[e0 * 8 + r] : 0.0;
-    }
-    // RK register and low words, interleaved, in the tile order [f][j][el][i] of the shape's
-    // full tiles (the launch always uses them, so the low words keep their places from one step to
-    // the next): the row owners of the tile's elements read and write one line index j with
-    // consecutive lanes on consecutive addresses, both words with one 8-byte access.
-    float g_old[NF], lo_row[NF];
-    if (active) {
-        const int64_t off = e0 * 3 * NE + ((int64_t)f * NF * nel + el) * NF + l;
+        for (int it = 0; it < FPT; ++it) own[it] = w_buf.load(tid + it * T);
 #pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            const float2 w = gl[off + j * nel * NF];
-            g_old[j] = first ? 0.f : w.x;
-            lo_row[j] = w.y;
+        for (int j = 0; j < NF / 2; ++j) gl_old[j] = gl_buf.load4<kHow>(4 * (j * run + lane));
+        if (NF % 2) gl_odd = gl_buf.load2<kHow>(2 * (NF / 2 * 2 * run + lane));
+    };
+    if (once) load_tile(std::integral_constant<int, Buffer::kNonTemporal>());
+    else load_tile(std::integral_constant<int, 0>());
+    SideRecord rec[FPT];
+    float tr[FPT][3];  // the own traces of a side with a record
+    uint64_t with_record[FPT];
+#pragma unroll
+    for (int it = 0; it < FPT; ++it) with_record[it] = __ballot(code[it] < 0 && code[it] != INT32_MIN);
+#pragma unroll
+    for (int it = 0; it < FPT; ++it)
+        if (code[it] < 0 && code[it] != INT32_MIN) {
+            const int item = tid + it * T;
+            const float *from = tr_in + (e0 * 4 + item / NF) * 3 * NF + item % NF;
+            for (int m = 0; m < 3; ++m) tr[it][m] = from[m * NF];
+            rec[it].load(bc + (-1 - code[it]));
         }
-    } else {
-#pragma unroll
-        for (int j = 0; j < NF; ++j) g_old[j] = lo_row[j] = 0.f;
-    }
-    float nbv[FPT][3];
+    float ext[FPT];
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
-        nbv[it][0] = nbv[it][1] = nbv[it][2] = 0.f;
-        const int32_t cd = code[it];
-        if (cd >= 0) {
-            const int k = (tid + it * T) % NF;
-            const float *nb = tr_in + (int64_t)(cd >> 2) * 12 * NF + (cd & 3) * 3 * NF + (N - k);
-            nbv[it][0] = nb[0];
-            nbv[it][1] = nb[NF];
-            nbv[it][2] = nb[2 * NF];
-        }
+        const int32_t cd = max(code[it], 0);  // side 0 of the group for sides with a record
+        const int k = (tid + it * T) % NF;
+        ext[it] = w_in[(int64_t)cd * NF + (N - k)];
     }
     __builtin_amdgcn_s_setprio(0);
+    auto at = [](int r) { return NFP == NF ? r : r + (int)((unsigned)r / NF); };
+    auto put_q = [&](int r, float v) {
+        if (r >= 0 && r < EPB * 3 * NE) s_q[at(r)] = v;
+    };
 #pragma unroll
-    for (int it = 0; it < S::VPT; ++it) {
-        const int r = tid + it * T;
-        if (r < nel * 8) s_v[r] = vreg[it];
+    for (int it = 0; it < QP4; ++it) {
+        const int i = 4 * (tid + it * T), r = i - lead;
+        if (i < (end & ~3)) {
+            put_q(r, qreg[it].x);
+            put_q(r + 1, qreg[it].y);
+            put_q(r + 2, qreg[it].z);
+            put_q(r + 3, qreg[it].w);
+        }
     }
+    if (tid < (end & 3)) put_q((end & ~3) + tid - lead, q_rest);
 #pragma unroll
-    for (int it = 0; it < S::QPT; ++it) {
-        const int r = tid + it * T;
-        if (r < nel * 3 * NE) s_q[r] = qreg[it];
+    for (int it = 0; it < FPT; ++it) {
+        const int item = tid + it * T;
+        if ((it + 1) * T <= EPB * 4 * NF || item < EPB * 4 * NF) s_f[item] = own[it];
     }
+    if (active && f < 2) {  // metric lines (in FP64, rounded once)
+        const double t = x64[l];
+        float *met = s_met + el * 4 * NF + 2 * f * NF;
+        // x_eta, y_eta along xi; x_xi, y_xi along eta
+        const double ax = f == 0 ? P[6] : P[2], ay = f == 0 ? P[7] : P[3], bx = f == 0 ? P[2] : P[6],
+                     by = f == 0 ? P[3] : P[7];
+        met[l] = (float)(((1 - t) * (ax - P[0]) + (1 + t) * (P[4] - bx)) / 4);
+        met[NF + l] = (float)(((1 - t) * (ay - P[1]) + (1 + t) * (P[5] - by)) / 4);
+    }
+    if (active && f == 2)  // sides l, l + N + 1, ... (N + 1 lanes cover the four)
+        for (int s = l; s < 4; s += NF) {
+            double nx, ny;
+            float sf = (float)(s == l ? side_geometry(P, 0, nx, ny) : side_geometry(verts + (e0 + el) * 8, s, nx, ny));
+            if (const int32_t cd = s == l ? side_code : side_nb[(e0 + el) * 4 + s]; cd < 0) {
+                const BcSide &r = bc[-1 - cd];
+                nx = r.nx;
+                ny = r.ny;
+                if (r.kind == kKindMortar) sf = -1.f;
+            }
+            float *sd = s_side + (el * 4 + s) * 3;
+            sd[0] = (float)nx;
+            sd[1] = (float)ny;
+            sd[2] = sf;
+        }
     __syncthreads();
 
-    // P1 (geometry in FP64, rounded once)
-    if (active) {
-        const double *P = s_v + el * 8;
-        float *met = s_met + el * 4 * NF;
-        if (f == 0) {
-            const double xi = x64[l];
-            met[l] = (float)(((1 - xi) * (P[6] - P[0]) + (1 + xi) * (P[4] - P[2])) / 4);
-            met[NF + l] = (float)(((1 - xi) * (P[7] - P[1]) + (1 + xi) * (P[5] - P[3])) / 4);
-        } else if (f == 1) {
-            const double eta = x64[l];
-            met[2 * NF + l] = (float)(((1 - eta) * (P[2] - P[0]) + (1 + eta) * (P[4] - P[6])) / 4);
-            met[3 * NF + l] = (float)(((1 - eta) * (P[3] - P[1]) + (1 + eta) * (P[5] - P[7])) / 4);
-        } else {  // sides l, l + N + 1, ... (N + 1 lanes cover the 4 sides)
-            for (int s = l; s < 4; s += NF) {
-                const int s1 = (s + 1) & 3;
-                const double ex = P[2 * s1] - P[2 * s], ey = P[2 * s1 + 1] - P[2 * s + 1];
-                const double len = sqrt(ex * ex + ey * ey);
-                float *sd = s_side + (el * 4 + s) * 3;
-                sd[0] = (float)(ey / len);
-                sd[1] = (float)(-(ex / len));
-                sd[2] = (float)side_scale(P, s, x64[0]);
-            }
-        }
-        const float *tq = s_q + el * 3 * NE + f * NE;
-        float t0 = 0.f, t1 = 0.f, t2 = 0.f, t3 = 0.f;
 #pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            const float row = tq[l * NF + j], col = tq[j * NF + l];
-            t0 += lm[j] * row;
-            t2 += lp[j] * row;
-            t1 += lp[j] * col;
-            t3 += lm[j] * col;
+    for (int it = 0; it < FPT; ++it)
+        if (with_record[it]) {  // skipped by a wave without
+            const int item = tid + it * T;
+            if (code[it] >= 0 || code[it] == INT32_MIN) continue;
+            record_flux32<N>(rec[it], bc + (-1 - code[it]), tr[it], x64, tr_in, side_flux, item % NF, clock, cw,
+                             s_f[item], s_f[EPB * 4 * NF + item], s_f[EPB * 8 * NF + item]);
         }
-        float *tr = s_tr + el * 12 * NF + f * NF;
-        tr[l] = t0;
-        tr[6 * NF + (N - l)] = t2;
-        tr[3 * NF + l] = t1;
-        tr[9 * NF + (N - l)] = t3;
+
+    // P1
+    const float *tq = s_q + el * 3 * NEP;
+    const float *met = s_met + el * 4 * NF;
+    float vx[NF], ve[NF];
+    {
+        float F[NF];
+        const float *col = tq + l, *row = tq + l * NFP;  // node (k, l) at col[k * NFP], (l, k) at row[k]
+        if (f == 0) {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) {
+                const float xeta = met[k], yeta = met[NF + k];
+                F[k] = yeta * col[NEP + k * NFP] - xeta * col[2 * NEP + k * NFP];
+            }
+        } else if (f == 1) {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) F[k] = met[NF + k] * col[k * NFP];
+        } else {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) F[k] = -(met[k] * col[k * NFP]);
+        }
+        contract32<NF>(Dh, F, vx);
+        if (f == 0) {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) {
+                const float xxi = met[2 * NF + k], yxi = met[3 * NF + k];
+                F[k] = -yxi * row[NEP + k] + xxi * row[2 * NEP + k];
+            }
+        } else if (f == 1) {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) F[k] = -met[3 * NF + k] * row[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < NF; ++k) F[k] = met[2 * NF + k] * row[k];
+        }
+        contract32<NF>(Dh, F, ve);
+    }
+    const int t1 = fresh(tid);
+#pragma unroll
+    for (int it = 0; it < FPT; ++it) {
+        const int item = t1 + it * T;
+        if (item < n_pt && !__builtin_amdgcn_inverse_ballot_w64(with_record[it])) {
+            const float w = s_f[item];
+            s_f[item] = (w - ext[it]) * 0.5f;
+            s_f[EPB * 4 * NF + item] = (w + ext[it]) * 0.5f;
+        }
     }
     __syncthreads();
 
     // P2
+    {
+        const float *side = s_side + el * 12;
+        const float *fl = s_f + el * 4 * NF;
+        auto flux = [&](int s, int k) {
+            const float sf = side[3 * s + 2];
+            const float va = fl[(f == 0 ? 0 : EPB * 4 * NF) + s * NF + k];
+            if (sf < 0.f) return fl[f * EPB * 4 * NF + s * NF + k];  // the mortar side's own component
+            return f == 0 ? va * sf : (side[3 * s + (f == 2 ? 1 : 0)] * va) * sf;
+        };
+        const float Fr = flux(1, l), Fl = flux(3, N - l), Ft = flux(2, N - l), Fb = flux(0, l);
+        float *d = s_d + el * 3 * NEP + f * NEP + l;
 #pragma unroll
-    for (int it = 0; it < FPT; ++it) {
-        const int item = tid + it * T;
-        if (item < nel * 4 * NF) {
-            const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
-            float *tr = s_tr + fe * 12 * NF + s * 3 * NF + k;
-            const float pL = tr[0], uL = tr[NF], vL = tr[2 * NF];
-            const float *sd = s_side + (fe * 4 + s) * 3;
-            float nx = sd[0], ny = sd[1];
-            const float sf = sd[2];
-            float pR, uR, vR;
-            const int32_t cd = code[it];
-            if (cd >= 0) {
-                pR = nbv[it][0];
-                uR = nbv[it][1];
-                vR = nbv[it][2];
-            } else {
-                const BcSide rec = bc[-1 - cd];
-                if (rec.kind == kKindMortar) {
-                    const float *sfl = side_flux + rec.slot + k;
-                    float f0 = sfl[0], f1 = sfl[NF], f2 = sfl[2 * NF];
-                    for (int m = 1; m < rec.n_faces; ++m) {
-                        const float *s2 = sfl + m * 3 * NF;
-                        f0 += s2[0];
-                        f1 += s2[NF];
-                        f2 += s2[2 * NF];
-                    }
-                    tr[0] = f0;
-                    tr[NF] = f1;
-                    tr[2 * NF] = f2;
-                    continue;
-                }
-                nx = (float)rec.nx;
-                ny = (float)rec.ny;
-                const float tx = (float)rec.tx, ty = (float)rec.ty, gs = (float)rec.sf;
-                if (rec.kind == kKindTrace) {
-                    const float *nb = tr_in + rec.slot + (N - k);
-                    pR = nb[0];
-                    uR = nb[NF];
-                    vR = nb[2 * NF];
-                } else if (rec.kind == NDG_BC_WALL || rec.kind == NDG_BC_SYMMETRY) {
-                    pR = pL * gs;
-                    const float ux = uL * gs, uy = vL * gs;
-                    const float l0 = -(ux * nx + uy * ny);
-                    const float l1 = ux * tx + uy * ty;
-                    uR = nx * l0 + tx * l1;
-                    vR = ny * l0 + ty * l1;
-                } else if (rec.kind == NDG_BC_OUTFLOW) {
-                    pR = pL * gs;
-                    uR = uL * gs;
-                    vR = vL * gs;
-                } else if (rec.kind == NDG_BC_INFLOW) {
-                    const double interp = (x64[N - k] + 1) / 2;
-                    const double X = rec.bx * interp + rec.ax * (1 - interp);
-                    const double Y = rec.by * interp + rec.ay * (1 - interp);
-                    double p64, u64, v64;
-                    plane_wave(X, Y, clock.time(), cw, p64, u64, v64);
-                    pR = (float)p64;
-                    uR = (float)u64;
-                    vR = (float)v64;
-                } else {
-                    pR = uR = vR = 0.f;
-                }
-            }
-            const float wL = pL + (uL * nx + vL * ny);
-            const float wR = pR - (uR * nx + vR * ny);
-            tr[0] = ((wL - wR) * 0.5f) * sf;
-            tr[NF] = (nx * (wL + wR) * 0.5f) * sf;
-            tr[2 * NF] = (ny * (wL + wR) * 0.5f) * sf;
+        for (int i = 0; i < NF; ++i) {
+            vx[i] += (Fr * lp[i] + Fl * lm[i]) * winv[i];
+            ve[i] += (Ft * lp[i] + Fb * lm[i]) * winv[i];
         }
+        if (active)
+#pragma unroll
+            for (int i = 0; i < NF; ++i) d[i * NFP] = vx[i];
     }
     __syncthreads();
 
-    const float *tq = s_q + el * 3 * NE;
-    const float *met = s_met + el * 4 * NF;
-    const float *fs = s_tr + el * 12 * NF + f * NF;
     // P3
-    if (active) {
-        const int j = l;
-        float F[NF];
+    {
+        float *d = s_d + el * 3 * NEP + f * NEP + l * NFP;
+        float *qrow = s_q + el * 3 * NEP + f * NEP + l * NFP;
+        const float xeta_i = met[l], yeta_i = met[NF + l];
 #pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            const int node = k * NF + j;
-            const float xeta = met[k], yeta = met[NF + k];
-            if (f == 0) F[k] = yeta * tq[NE + node] - xeta * tq[2 * NE + node];
-            else if (f == 1) F[k] = yeta * tq[node];
-            else F[k] = -(xeta * tq[node]);
+        for (int j = 0; j < NF; ++j) {
+            const float jac = met[2 * NF + j] * yeta_i - xeta_i * met[3 * NF + j];
+            ve[j] = (float)cw * ((-d[j] - ve[j]) / jac);
         }
-        const float Fr = fs[3 * NF + j], Fl = fs[9 * NF + (N - j)];
-        float *d = s_d + el * 3 * NE + f * NE + j;
+        float h[NF], lo[NF];
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            float acc = 0.f;
+        for (int j = 0; j < NF; ++j) {
+            const float2 w = j / 2 < NF / 2 ? (j % 2 ? make_float2(gl_old[j / 2].z, gl_old[j / 2].w)
+                                                     : make_float2(gl_old[j / 2].x, gl_old[j / 2].y))
+                                            : gl_odd;
+            ve[j] = first ? ve[j] : a * w.x + ve[j];
+            h[j] = qrow[j];
+            lo[j] = w.y;
+            two_sum_add(h[j], lo[j], gdt * ve[j]);
+        }
+        if (active) {
+            auto store_lines = [&](auto how) {
 #pragma unroll
-            for (int k = 0; k < NF; ++k) acc += Dh[i * NF + k] * F[k];
-            acc += (Fr * lp[i] + Fl * lm[i]) * winv[i];
-            d[i * NF] = acc;
+                for (int j = 0; j < NF / 2; ++j)
+                    gl_buf.store4<decltype(how)::value>(4 * (j * run + lane),
+                                                        make_float4(ve[2 * j], lo[2 * j], ve[2 * j + 1], lo[2 * j + 1]));
+                if (NF % 2) gl_buf.store2<decltype(how)::value>(2 * (NF / 2 * 2 * run + lane),
+                                                                make_float2(ve[NF - 1], lo[NF - 1]));
+            };
+            if (once) store_lines(std::integral_constant<int, Buffer::kNonTemporal>());
+            else store_lines(std::integral_constant<int, 0>());
+            float t0 = 0.f, t2 = 0.f;
+#pragma unroll
+            for (int j = 0; j < NF; ++j) {
+                qrow[j] = h[j];
+                t0 += lm[j] * h[j];
+                t2 += lp[j] * h[j];
+            }
+            float *tr = s_f + (el * 3 + f) * 2 * NF;
+            tr[l] = t0;
+            tr[NF + (N - l)] = t2;
         }
     }
     __syncthreads();
 
     // P4
-    float hn[NF];
     if (active) {
-        const int i = l;
-        float Gt[NF];
-#pragma unroll
-        for (int k = 0; k < NF; ++k) {
-            const int node = i * NF + k;
-            const float xxi = met[2 * NF + k], yxi = met[3 * NF + k];
-            if (f == 0) Gt[k] = -yxi * tq[NE + node] + xxi * tq[2 * NE + node];
-            else if (f == 1) Gt[k] = -yxi * tq[node];
-            else Gt[k] = xxi * tq[node];
-        }
-        const float Ft = fs[6 * NF + (N - i)], Fb = fs[i];
-        const float xeta_i = met[i], yeta_i = met[NF + i];
-        float *d = s_d + el * 3 * NE + f * NE + i * NF;
-        const float *qrow = tq + f * NE + i * NF;
+        const float *col = s_q + el * 3 * NEP + f * NEP + l;
+        float t1 = 0.f, t3 = 0.f;
 #pragma unroll
         for (int j = 0; j < NF; ++j) {
-            float acc = 0.f;
-#pragma unroll
-            for (int k = 0; k < NF; ++k) acc += Dh[j * NF + k] * Gt[k];
-            acc += (Ft * lp[j] + Fb * lm[j]) * winv[j];
-            const float jac = met[2 * NF + j] * yeta_i - xeta_i * met[3 * NF + j];
-            const float Gv = (float)cw * ((-d[j] - acc) / jac);
-            const float gn = first ? Gv : a * g_old[j] + Gv;
-            float h = qrow[j], lo = lo_row[j];
-            two_sum_add(h, lo, gdt * gn);
-            hn[j] = h;
-            gl[e0 * 3 * NE + ((f * NF + j) * nel + el) * NF + i] = make_float2(gn, lo);
+            const float v = col[j * NFP];
+            t1 += lp[j] * v;
+            t3 += lm[j] * v;
         }
+        float *tr = s_d + (el * 3 + f) * 2 * NF;
+        tr[l] = t1;
+        tr[NF + (N - l)] = t3;
     }
-    __syncthreads();
-    if (active) {
-        float *qw = s_q + el * 3 * NE + f * NE + l * NF;
+    {
+        // words wholly inside the tile; the values of a word that straddles an end one by one
+        const int t4 = fresh(tid);
+        auto value = [&](int r) { return s_q[min(max(at(r), 0), EPB * 3 * NEP - 1)]; };
+        auto store_tile = [&](auto how) {
 #pragma unroll
-        for (int j = 0; j < NF; ++j) qw[j] = hn[j];
+            for (int it = 0; it < QP4; ++it) {
+                const int i = 4 * (t4 + it * T), r = i - lead;
+                const float4 v = make_float4(value(r), value(r + 1), value(r + 2), value(r + 3));
+                if (it > 0 || r >= 0) q_buf.store4<decltype(how)::value>(i, v);
+            }
+        };
+        if (once) store_tile(std::integral_constant<int, Buffer::kNonTemporal>());
+        else store_tile(std::integral_constant<int, 0>());
+        const int head = min((4 - (lead & 3)) & 3, n_val), tail = lead + head <= (end & ~3) ? end & 3 : 0;
+        if (tid < head) q_all.store(lead + tid, s_q[at(tid)]);
+        if (tid >= 64 && tid < 64 + tail) q_all.store((end & ~3) + tid - 64, s_q[at((end & ~3) + tid - 64 - lead)]);
     }
     __syncthreads();
 
     // P5
-    {
-        float *qw = qh + e0 * 3 * NE;
+    const int t5 = fresh(tid);
 #pragma unroll
-        for (int it = 0; it < S::QPT; ++it) {
-            const int r = tid + it * T;
-            if (r < nel * 3 * NE) qw[r] = s_q[r];
+    for (int it = 0; it < FPT; ++it) {
+        const int item = t5 + it * T;
+        if (item >= n_pt) continue;
+        const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
+        const float *tr = ((s & 1) ? s_d : s_f) + fe * 6 * NF + (s >> 1) * NF + k;
+        const float *sd = s_side + (fe * 4 + s) * 3;
+        const float p = tr[0], u = tr[2 * NF], v = tr[4 * NF];
+        w_out[e0 * 4 * NF + item] = characteristic32(p, u, v, sd[0], sd[1]);
+        if (__builtin_amdgcn_inverse_ballot_w64(with_record[it]) || (flags & kTraceAll)) {
+            float *to = tr_out + (e0 + fe) * 12 * NF + s * 3 * NF + k;
+            to[0] = p;
+            to[NF] = u;
+            to[2 * NF] = v;
         }
-    }
-    if (active) {
-        const float *tqf = s_q + el * 3 * NE + f * NE;
-        float t0 = 0.f, t1 = 0.f, t2 = 0.f, t3 = 0.f;
-#pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            const float row = tqf[l * NF + j], col = tqf[j * NF + l];
-            t0 += lm[j] * row;
-            t2 += lp[j] * row;
-            t1 += lp[j] * col;
-            t3 += lm[j] * col;
-        }
-        float *to = tr_out + (e0 + el) * 12 * NF + f * NF;
-        to[l] = t0;
-        to[6 * NF + (N - l)] = t2;
-        to[3 * NF + l] = t1;
-        to[9 * NF + (N - l)] = t3;
     }
 }
 
@@ -1659,8 +1844,9 @@ template <int N>
 static hipError_t traces_c32_n(const DeviceMesh &m, const Group &G, hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    hipLaunchKernelGGL(traces_c32_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, G.tab32, m.qh + G.q_off,
-                       m.trace32[m.cur] + G.tr_off, G.K);
+    hipLaunchKernelGGL(traces_c32_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
+                       m.side_nb + G.e_begin * 4, m.bc, G.tab32, m.qh + G.q_off, m.trace32[m.cur] + G.tr_off,
+                       m.wave32[m.cur] + G.tr_off / 3, G.K);
     return hipGetLastError();
 }
 
@@ -1668,14 +1854,13 @@ template <int N>
 static hipError_t stage_c32_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, double dt,
                               hipStream_t s) {
     using S = LineShape<N>;
-    const int epb = S::EPB;  // the low state words are kept in the full tiles' order
-    const int64_t blocks = (G.K + epb - 1) / epb;
+    const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
+    const int flags = (stage == 0 ? kRkFirst : 0) | (m.trace_all ? kTraceAll : 0) | (12 * m.n_q > kStreamBytes ? kStream : 0);
     hipLaunchKernelGGL(stage_c32_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
-                       m.side_nb + G.e_begin * 4, m.bc, G.tab, G.tab32, m.qh + G.q_off, m.gl32 + G.q_off,
-                       m.trace32[m.cur] + G.tr_off, m.trace32[1 - m.cur] + G.tr_off,
-                       m.side_flux32, G.K, stage == 0 ? 1 : 0, (float)a, (float)gdt,
-                       stage_clock(m, G, stage, dt), epb,
-                       G.tune[NDG_PRECISION_FP32_COMPENSATED].remap, m.wave_speed);
+                       m.side_nb + G.e_begin * 4, m.bc, G.tab, G.tab32, m.qh + G.q_off, m.gl32 + G.g_off,
+                       m.wave32[m.cur] + G.tr_off / 3, m.wave32[1 - m.cur] + G.tr_off / 3, m.trace32[m.cur] + G.tr_off,
+                       m.trace32[1 - m.cur] + G.tr_off, m.side_flux32, G.K, flags, (float)a, (float)gdt,
+                       stage_clock(m, G, stage, dt), G.tune[NDG_PRECISION_FP32_COMPENSATED].remap, m.wave_speed);
     return hipGetLastError();
 }
 
@@ -1785,13 +1970,21 @@ hipError_t launch_traces_c32(const DeviceMesh &m, hipStream_t s) {
 }
 
 
+template <int N>
+static int c32_run_n() { return rk_run<N>(LineShape<N>::EPB); }
+
+static int c32_run(int N) {
+    switch (N) { CASES_1(c32_run_n) }
+    return 0;
+}
+
 // q and qh are in reference node order; gl32 in the FP32 stage's tile order (tiles of the
 // shape's EPB elements). Run per group (the order depends on N).
 hipError_t launch_to_c32(DeviceMesh &m, hipStream_t s) {
     return for_groups(m, [&](const Group &G) -> hipError_t {
         const int64_t n = G.K * 3 * (int64_t)(G.N + 1) * (G.N + 1);
         hipLaunchKernelGGL(to_c32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m.q + G.q_off,
-                           m.qh + G.q_off, m.gl32 + G.q_off, n, G.N + 1, stage_max_epb(G.N));
+                           m.qh + G.q_off, m.gl32 + G.g_off, n, G.N + 1, stage_max_epb(G.N), c32_run(G.N));
         return hipGetLastError();
     });
 }
@@ -1800,7 +1993,7 @@ hipError_t launch_from_c32(DeviceMesh &m, hipStream_t s) {
     return for_groups(m, [&](const Group &G) -> hipError_t {
         const int64_t n = G.K * 3 * (int64_t)(G.N + 1) * (G.N + 1);
         hipLaunchKernelGGL(from_c32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m.qh + G.q_off,
-                           m.gl32 + G.q_off, m.q + G.q_off, n, G.N + 1, stage_max_epb(G.N));
+                           m.gl32 + G.g_off, m.q + G.q_off, n, G.N + 1, stage_max_epb(G.N), c32_run(G.N));
         return hipGetLastError();
     });
 }

@@ -78,7 +78,8 @@ void ndg::arena_free(Arena &a) {
 
 void ndg::store_free(DeviceStore &s) {
     for (Arena *a : {&s.verts, &s.side_nb, &s.bc, &s.faces, &s.side_flux, &s.side_flux32, &s.q, &s.g, &s.tr[0],
-                     &s.tr[1], &s.wave[0], &s.wave[1], &s.rhs, &s.scratch, &s.qh, &s.gl32, &s.tr32[0], &s.tr32[1]})
+                     &s.tr[1], &s.wave[0], &s.wave[1], &s.rhs, &s.scratch, &s.qh, &s.gl32, &s.tr32[0], &s.tr32[1],
+                     &s.wave32[0], &s.wave32[1]})
         arena_free(*a);
 }
 
@@ -1395,7 +1396,10 @@ extern "C" ndg_status ndg_mesh_set_precision(ndg_mesh *mesh, int32_t precision) 
             DeviceStore &sto = mesh->store[mesh->active];
             ndg_status st;
             if ((st = fit_view(sto.qh, &d.qh, d.n_q, "hipMalloc qh")) != NDG_OK) return st;
-            if ((st = fit_view(sto.gl32, &d.gl32, d.n_q, "hipMalloc gl32")) != NDG_OK) return st;
+            if ((st = fit_view(sto.gl32, &d.gl32, d.n_g, "hipMalloc gl32")) != NDG_OK) return st;
+            for (int k = 0; k < 2; ++k)
+                if ((st = fit_view(sto.wave32[k], &d.wave32[k], d.n_tr / 3, "hipMalloc characteristics")) != NDG_OK)
+                    return st;
             if ((st = fit_view(sto.tr32[0], &d.trace32[0], d.n_tr, "hipMalloc traces32")) != NDG_OK) return st;
             if ((st = fit_view(sto.tr32[1], &d.trace32[1], d.n_tr, "hipMalloc traces32")) != NDG_OK) return st;
             d.side_flux32 = nullptr;

@@ -134,3 +134,11 @@ def test_smaller_tiles_of_the_tuner(N):
         states.append(gm.get_solution())
     for a, b in zip(*states):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,nx,ny", [(8, 1, 1), (8, 7, 1), (8, 3, 5), (7, 9, 1), (2, 21, 1), (1, 33, 1), (11, 2, 3), (16, 2, 2)])
+@pytest.mark.parametrize("bc", [nd.BC_WALL, nd.BC_INFLOW])
+def test_fp32c_tiles_and_remainders(N, nx, ny, bc):
+    """One element, exactly one tile, and tiles with a remainder, in the FP32 form."""
+    compare(grid(nx, ny, bc, jitter=0.1 if min(nx, ny) > 1 else 0.0), N, precision="fp32c")
