@@ -170,20 +170,25 @@ traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side
 // the three traces: 4 (N+1) values an element are written once and read twice (the element's own
 // from the same tile) instead of 12 (N+1) written and read, 7,200 instead of 8,290 bytes an element
 // and stage at N = 8. Sides where that is not enough carry a record (code < 0): boundary ghosts are
-// built from the element's own traces, formed from the state tile; a mortar side's flux comes from
+// built from the element's own traces, read back as the last stage wrote them; a mortar side's flux comes from
 // the mortar kernel; a periodic side whose partner does not run parallel to it reads the partner's
 // three traces. Elements write the three traces of the sides with a record (and with kTraceAll of
 // every side) for these.
 //
-// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 324 us a
-// launch, 5.8 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches 5.3 to 5.8
+// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 321 us a
+// launch, 5.9 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches 5.3 to 5.8
 // here); 421 us and 2.18 GB with the traces exchanged. 512 x 512, N = 4: 116 us (164 us before). 128 x
-// 128, N = 8 (in the last-level cache): 24.9 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
+// 128, N = 8 (in the last-level cache): 25.0 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
 // us from launch to launch, 7.0 us before. What made the difference, at N = 8:
 //  - the state and the RK register are streamed past the caches (non-temporal, in 16-byte words on
 //    whole 128-byte lines) where they are larger than these (stage_flags): 401 -> 324 us at 512 x 512;
-//  - D^ out of the scalar loads (LaneTable) and by even and odd parts (contract): 24.9 us instead of
+//  - D^ out of the scalar loads (LaneTable) and by even and odd parts (contract): 25 us instead of
 //    28 us at 128 x 128;
+//  - the entries of D^ as DPP operands (rows): 256 x 256, N = 12 in 184 us instead of 189 us, 48 x 48,
+//    N = 16 in 19.2 us instead of 20.4 us (and 35 registers fewer), 512 x 512 in 321 us instead of 325 us;
+//  - the own traces of a side with a record loaded with the tile, not formed again from its lines:
+//    23 x 23, N = 4 with walls, inflow and outflow 5.8 us instead of 6.7 us, 48 x 48, N = 16: 16.6 us
+//    instead of 19.2 us;
 //  - no branch inside the line loops and no wait among the loads (a condition on the field in a loop
 //    kept each LDS read from overlapping the next: 3,700 cycles for the update of a line, 1,700 now);
 //  - five barriers instead of six, LDS for five workgroups a CU instead of four.
@@ -248,7 +253,7 @@ struct Buffer {
 };
 
 // A table of L values held across the lanes of each row of 16 (value e in lane e mod 16 of register
-// e / 16), so that a wave-uniform entry is one cross-lane move (DPP row broadcast) away: the stage
+// e / 16), so that a wave-uniform entry is a DPP operand (row broadcast) of its multiply-add: the stage
 // kernel's D^ entries as scalar loads came a few at a time (81 doubles are more than the scalar
 // registers hold), each batch a wait of some 300 cycles that the contraction of the line could
 // not hide: 3,650 cycles for the 81 multiply-adds of a line at N = 8.
@@ -260,11 +265,6 @@ struct LaneTable {
 #pragma unroll
         for (int p = 0; p < (L + 15) / 16; ++p) v[p] = t[min(p * 16 + m, L - 1)];
     }
-    template <int E>
-    __device__ __forceinline__ double get() const {
-        const long long b = __builtin_bit_cast(long long, v[E / 16]);
-        return __builtin_bit_cast(double, (long long)__builtin_amdgcn_update_dpp(0ll, b, 0x150 + E % 16, 0xf, 0xf, true));
-    }
 };
 
 // D^ F of a line by even and odd parts: the Gauss nodes are symmetric, so D^[N-i][N-k] = -D^[i][k], and with
@@ -273,21 +273,49 @@ struct LaneTable {
 //   (D^ F)[i] = P_i + Q_i,  (D^ F)[N-i] = P_i - Q_i,  (D^ F)[m] = P_m,
 // about half the multiply-adds and entries of D^. The table holds row by row A[i][.], D^[i][m], B[i][.],
 // then B[m][.].
-template <int NF, int E = 0>
-__device__ __forceinline__ void even_odd_entries(const LaneTable<even_odd_len(NF)> &D, const double *F, double *a) {
-    constexpr int h = NF / 2, odd = NF & 1, per = 2 * h + odd;
-    constexpr bool mid = E >= h * per;
-    constexpr int i = mid ? h : E / per, c = mid ? h + odd + E - h * per : E % per;
-    // entry c of a row multiplies F[c]: s in [0, h), F[m] at h, then d
-    constexpr int out = c < h + odd ? NF - 1 - i : i;  // Q_i is summed in place N - i, P_i in place i
-    const double d = D.template get<E>();
-    a[out] = c == 0 || c == h + odd ? d * F[c] : fma(d, F[c], a[out]);
-    // finished here, a row at a time: the compiler would keep the moved entries and move the sums on
-    if constexpr (c == per - 1) {
-        asm volatile("" : "+v"(a[i]));
-        if constexpr (!mid) asm volatile("" : "+v"(a[NF - 1 - i]));
+// a[i S] += D(entry E + i Step) F for the R rows i: the entry is a DPP operand of the multiply-add (the
+// compiler moves it to a register pair first, with a wait: three issues instead of one). A block first
+// waits out the two cycles that a register written just before it takes to reach a DPP
+// instruction, and within one every row is another register.
+template <int E, int Step, int R, int S, int L>
+__device__ __forceinline__ void rows(const LaneTable<L> &D, double F, double *a) {
+#define NDG_MAC(o, d, f, e) "v_fmac_f64_dpp %" #o ", %" #d ", %" #f " row_newbcast:%" #e " row_mask:0xf bank_mask:0xf\n\t"
+#define NDG_ENTRY(i) D.v[(E + (i) * Step) / 16]
+#define NDG_LANE(i) (E + (i) * Step) % 16
+    if constexpr (R > 4) {
+        rows<E, Step, 4, S>(D, F, a);
+        rows<E + 4 * Step, Step, R - 4, S>(D, F, a + 4 * S);
+    } else if constexpr (R == 4) {
+        asm volatile("s_nop 1\n\t" NDG_MAC(0, 4, 8, 9) NDG_MAC(1, 5, 8, 10) NDG_MAC(2, 6, 8, 11) NDG_MAC(3, 7, 8, 12)
+                     : "+&v"(a[0]), "+&v"(a[S]), "+&v"(a[2 * S]), "+&v"(a[3 * S])
+                     : "v"(NDG_ENTRY(0)), "v"(NDG_ENTRY(1)), "v"(NDG_ENTRY(2)), "v"(NDG_ENTRY(3)), "v"(F),
+                       "n"(NDG_LANE(0)), "n"(NDG_LANE(1)), "n"(NDG_LANE(2)), "n"(NDG_LANE(3)));
+    } else if constexpr (R == 3) {
+        asm volatile("s_nop 1\n\t" NDG_MAC(0, 3, 6, 7) NDG_MAC(1, 4, 6, 8) NDG_MAC(2, 5, 6, 9)
+                     : "+&v"(a[0]), "+&v"(a[S]), "+&v"(a[2 * S])
+                     : "v"(NDG_ENTRY(0)), "v"(NDG_ENTRY(1)), "v"(NDG_ENTRY(2)), "v"(F), "n"(NDG_LANE(0)),
+                       "n"(NDG_LANE(1)), "n"(NDG_LANE(2)));
+    } else if constexpr (R == 2) {
+        asm volatile("s_nop 1\n\t" NDG_MAC(0, 2, 4, 5) NDG_MAC(1, 3, 4, 6)
+                     : "+&v"(a[0]), "+&v"(a[S])
+                     : "v"(NDG_ENTRY(0)), "v"(NDG_ENTRY(1)), "v"(F), "n"(NDG_LANE(0)), "n"(NDG_LANE(1)));
+    } else if constexpr (R == 1) {
+        asm volatile("s_nop 1\n\t" NDG_MAC(0, 1, 2, 3) : "+&v"(a[0]) : "v"(NDG_ENTRY(0)), "v"(F), "n"(NDG_LANE(0)));
     }
-    if constexpr (E + 1 < even_odd_len(NF)) even_odd_entries<NF, E + 1>(D, F, a);
+#undef NDG_MAC
+#undef NDG_ENTRY
+#undef NDG_LANE
+}
+
+// Q_i (summed in place N - i) and P_i (in place i) of the rows i < h, and P_m, a column at a time:
+// entry c of a row multiplies F[c], s in [0, h), F[m] at h, then d.
+template <int NF, int c = 0>
+__device__ __forceinline__ void even_odd_columns(const LaneTable<even_odd_len(NF)> &D, const double *F, double *a) {
+    constexpr int h = NF / 2, odd = NF & 1, per = 2 * h + odd;
+    if constexpr (c < h + odd) rows<c, per, h, -1>(D, F[c], a + NF - 1);
+    else rows<c, per, h, 1>(D, F[c], a);
+    if constexpr (odd && c >= h + 1) rows<h * per + c - h - 1, 1, 1, 1>(D, F[c], a + h);
+    if constexpr (c + 1 < per) even_odd_columns<NF, c + 1>(D, F, a);
 }
 
 // a = D^ F (F is overwritten).
@@ -301,7 +329,9 @@ __device__ __forceinline__ void contract(const LaneTable<even_odd_len(NF)> &D, d
         t[h + odd + k] = F[k] - F[NF - 1 - k];
     }
     if (odd) t[h] = F[h];
-    even_odd_entries<NF>(D, t, a);
+#pragma unroll
+    for (int i = 0; i < NF; ++i) a[i] = 0.0;
+    even_odd_columns<NF>(D, t, a);
 #pragma unroll
     for (int i = 0; i < h; ++i) {
         const double P = a[i], Q = a[NF - 1 - i];
@@ -341,14 +371,13 @@ struct SideRecord {
 
 // (w_L - w_R)/2 and (w_L + w_R)/2 of point k of side s with a record: a boundary ghost (Mesh2D_t.cpp:
 // 4298-4730), a mortar side (the projected flux, already times the edge Jacobian: the side's scale
-// is 1 then) or a periodic side of another direction. The normal is the record's; tq is the
-// element's state in LDS, whose traces are summed in the order of the line's nodes.
+// is 1 then) or a periodic side of another direction. The normal is the record's, tr the side's own
+// traces.
 template <int N>
-__device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide *bc, const double *tq, const double *lm,
-                                            const double *lp, const double *x, const double *tr_in,
-                                            const double *side_flux, int s, int k, const StageClock &clock, double cw,
-                                            double &fa, double &fb) {
-    constexpr int NF = N + 1, NFP = StageTile<N>::NFP, NEP = StageTile<N>::NEP;
+__device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide *bc, const double (&tr)[3],
+                                            const double *x, const double *tr_in, const double *side_flux, int k,
+                                            const StageClock &clock, double cw, double &fa, double &fb) {
+    constexpr int NF = N + 1;
     constexpr double c = kWaveSpeed;
     if (rec.kind == kKindMortar) {  // projected by the mortar kernel (already x sf)
         const double *sfl = side_flux + rec.slot + k;
@@ -363,20 +392,7 @@ __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide 
         fb = f1 * rec.nx + f2 * rec.ny;
         return;
     }
-    double pL = 0.0, uL = 0.0, vL = 0.0;
-    {
-        const bool low = s == 0 || s == 3;
-        const int m = s < 2 ? k : N - k, stride = (s & 1) ? NFP : 1;
-        const double *line = tq + ((s & 1) ? m : m * NFP);
-        constexpr int kUnroll = NF <= 6 ? NF : 3;
-#pragma unroll kUnroll
-        for (int j = 0; j < NF; ++j) {
-            const double lj = low ? lm[j] : lp[j];
-            pL += lj * line[j * stride];
-            uL += lj * line[NEP + j * stride];
-            vL += lj * line[2 * NEP + j * stride];
-        }
-    }
+    const double pL = tr[0], uL = tr[1], vL = tr[2];
     double pR = 0.0, uR = 0.0, vR = 0.0;
     if (rec.kind == NDG_BC_WALL || rec.kind == NDG_BC_SYMMETRY) {
         // ghost = sf * own trace, normal velocity reversed (Mesh2D_t.cpp:4377-4433)
@@ -454,10 +470,6 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
         const int item = tid + it * T;
         code[it] = item < n_pt ? side_nb[e0 * 4 + item / NF] : INT32_MIN;
     }
-    int32_t tile_code[(EPB * 4 + 63) / 64];  // all the tile's codes, over the lanes of each wave
-#pragma unroll
-    for (int it = 0; it < (EPB * 4 + 63) / 64; ++it)
-        tile_code[it] = side_nb[e0 * 4 + min(lane + 64 * it, nel * 4 - 1)];
     // The RK register lives only within a step (the first stage writes it without reading it), so
     // its layout is the kernel's own: within the workgroup's tile it is stored as [f][j / 2][el][i][j % 2]
     // (an odd last j by itself), so that the row owners of all the tile's elements read and write two
@@ -492,9 +504,18 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
     if (once) load_tile(std::integral_constant<int, Buffer::kNonTemporal>());
     else load_tile(std::integral_constant<int, 0>());
     SideRecord rec[FPT];
+    double tr[FPT][3];  // the own traces of a side with a record
+    uint64_t with_record[FPT];
+#pragma unroll
+    for (int it = 0; it < FPT; ++it) with_record[it] = __ballot(code[it] < 0 && code[it] != INT32_MIN);
 #pragma unroll
     for (int it = 0; it < FPT; ++it)
-        if (code[it] < 0 && code[it] != INT32_MIN) rec[it].load(bc + (-1 - code[it]));
+        if (code[it] < 0 && code[it] != INT32_MIN) {
+            const int item = tid + it * T;
+            const double *from = tr_in + (e0 * 4 + item / NF) * 3 * NF + item % NF;
+            for (int m = 0; m < 3; ++m) tr[it][m] = from[m * NF];
+            rec[it].load(bc + (-1 - code[it]));
+        }
     double ext[FPT];
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
@@ -525,22 +546,15 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
     }
     __syncthreads();
 
-    // the points of sides with a record, from the state tile (before the contractions, whose sums
-    // would be live beside it)
-    bool has_record = false;
+    // the points of sides with a record (before the contractions, whose sums would be live beside them)
 #pragma unroll
-    for (int it = 0; it < (EPB * 4 + 63) / 64; ++it) has_record = has_record || tile_code[it] < 0;
-    const bool recorded = __any(has_record);  // the same in every wave
-    if (recorded) {
-#pragma unroll
-        for (int it = 0; it < FPT; ++it) {
+    for (int it = 0; it < FPT; ++it)
+        if (with_record[it]) {  // skipped by a wave without
             const int item = tid + it * T;
             if (code[it] >= 0 || code[it] == INT32_MIN) continue;
-            const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
-            record_flux<N>(rec[it], bc + (-1 - code[it]), s_q + fe * 3 * NEP, lm, lp, x, tr_in, side_flux, s, k, clock,
-                           cw, s_f[item], s_f[EPB * 4 * NF + item]);
+            record_flux<N>(rec[it], bc + (-1 - code[it]), tr[it], x, tr_in, side_flux, item % NF, clock, cw, s_f[item],
+                           s_f[EPB * 4 * NF + item]);
         }
-    }
 
     // P1. Metric lines from the vertices (include/functions/quad_metrics.tpp:3-8): x_eta, y_eta
     // are linear in xi, x_xi, y_xi in eta.
@@ -593,7 +607,7 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
         const int item = t1 + it * T;
-        if (item < n_pt && !(recorded && side_nb[e0 * 4 + item / NF] < 0)) {
+        if (item < n_pt && !__builtin_amdgcn_inverse_ballot_w64(with_record[it])) {
             const double w = s_f[item];
             s_f[item] = c * (w - ext[it]) / 2;
             s_f[EPB * 4 * NF + item] = (w + ext[it]) / 2;
@@ -735,7 +749,7 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
         const double *sd = s_side + (fe * 4 + s) * 3;
         const double p = tr[0], u = tr[2 * NF], v = tr[4 * NF];
         w_out[e0 * 4 * NF + item] = p + c * (u * sd[0] + v * sd[1]);
-        if ((recorded && side_nb[e0 * 4 + item / NF] < 0) || (flags & kTraceAll)) {
+        if (__builtin_amdgcn_inverse_ballot_w64(with_record[it]) || (flags & kTraceAll)) {
             double *to = tr_out + (e0 + fe) * 12 * NF + s * 3 * NF + k;
             to[0] = p;
             to[NF] = u;
