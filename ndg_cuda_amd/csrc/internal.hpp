@@ -347,6 +347,9 @@ hipError_t launch_from_c32(DeviceMesh &m, hipStream_t s);
 hipError_t launch_traces_c32(const DeviceMesh &m, hipStream_t s);
 // One order group's stage kernel (of the mesh's precision); does not flip `cur`.
 hipError_t launch_group_stage(DeviceMesh &m, int group, int stage, double a, double gdt, double dt, hipStream_t s);
+// All groups' stage kernels: in one launch where stage_groups_fit, else one after another; does not flip `cur`.
+hipError_t launch_groups(DeviceMesh &m, int stage, double a, double gdt, double dt, hipStream_t s);
+bool stage_groups_fit(const DeviceMesh &m);
 // The start time of the next step (from the current trace buffer); the steps then advance it. Meshes
 // without inflow ghosts never read the time, and nothing is launched for them.
 hipError_t launch_clock_set(DeviceMesh &m, double t, hipStream_t s);

@@ -19,6 +19,7 @@
 // (read + write), and the characteristics of its sides (one value a point, read and written).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 #include <cmath>
@@ -424,23 +425,27 @@ __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide 
     fb = (wL + wR) / 2;
 }
 
+template <int N>
+constexpr int stage_lds() { return LineShape<N>::EPB * 6 * StageTile<N>::NEP + StageTile<N>::kFlux + LineShape<N>::EPB * 12; }
+
 template <int N, bool RHS_ONLY>
-__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 4 : N <= 12 ? 3 : 2)))
-stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
-             const BcSide *__restrict__ bc, const double *__restrict__ tab,
-             const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ w_in,
-             double *__restrict__ w_out, const double *__restrict__ tr_in, double *__restrict__ tr_out,
-             double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
-             double gdt, StageClock clock, int epb, int remap, double cw) {
+__device__ __forceinline__ void
+stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+           const BcSide *__restrict__ bc, const double *__restrict__ tab,
+           const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ w_in,
+           double *__restrict__ w_out, const double *__restrict__ tr_in, double *__restrict__ tr_out,
+           double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
+           double gdt, const StageClock &clock, int epb, double cw, int64_t blk,
+           double *__restrict__ s_q,     // the state tile
+           double *__restrict__ s_d,     // vertices, then d_xi, then the new traces on sides 1 and 3
+           double *__restrict__ s_f,     // fluxes, then the new traces on sides 0 and 2
+           double *__restrict__ s_side)  // outward normal and edge Jacobian per side
+{
     const bool first = flags & kRkFirst, store_g = !(flags & kRkLast), once = flags & kStream;
     using S = LineShape<N>;
     using L = StageTile<N>;
     constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT, NFP = L::NFP, NEP = L::NEP;
     constexpr double c = kWaveSpeed;
-    __shared__ double s_q[EPB * 3 * NEP];
-    __shared__ double s_d[EPB * 3 * NEP];  // vertices, then d_xi, then the new traces on sides 1 and 3
-    __shared__ double s_f[L::kFlux];       // fluxes, then the new traces on sides 0 and 2
-    __shared__ double s_side[EPB * 4 * 3]; // outward normal and edge Jacobian per side
     double *const s_v = s_d;
     static_assert(EPB * 8 <= EPB * 3 * NEP, "the vertices fit the tile they share");
     const double *lm = tab + NF * NF;
@@ -451,7 +456,6 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
     const int tid = threadIdx.x;
     const int f = __builtin_amdgcn_readfirstlane(tid >> 6);  // field of this wave
     const int lane = tid & 63;
-    const int64_t blk = remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
     const int64_t e0 = blk * epb;
     const int nel = (int)min<int64_t>(epb, K - e0);
     const int n_val = nel * 3 * NE, n_pt = nel * 4 * NF;
@@ -755,6 +759,74 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
             to[NF] = u;
             to[2 * NF] = v;
         }
+    }
+}
+
+template <int N, bool RHS_ONLY>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 4 : N <= 12 ? 3 : 2)))
+stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+             const BcSide *__restrict__ bc, const double *__restrict__ tab,
+             const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ w_in,
+             double *__restrict__ w_out, const double *__restrict__ tr_in, double *__restrict__ tr_out,
+             double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
+             double gdt, StageClock clock, int epb, int remap, double cw) {
+    using L = StageTile<N>;
+    constexpr int EPB = LineShape<N>::EPB;
+    __shared__ double s_q[EPB * 3 * L::NEP], s_d[EPB * 3 * L::NEP], s_f[L::kFlux], s_side[EPB * 12];
+    stage_tile<N, RHS_ONLY>(verts, side_nb, bc, tab, q, q_out, g, w_in, w_out, tr_in, tr_out, rhs, side_flux, K, flags, a,
+                            gdt, clock, epb, cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d,
+                            s_f, s_side);
+}
+
+// The stages of several order groups in one launch: the workgroups of group i are [first[i], first[i + 1]). Small
+// groups are bound by their launches, each as long as the latency of one workgroup: 96 x 96 elements of
+// orders 1, 3, 5, 7, 9 take 17.4 us a stage instead of 38.8 us with a launch a group (stage_groups_fit has the line).
+struct StageGroups {
+    int n;
+    int first[kMaxOrder + 2];
+    struct Part {
+        int N, epb, remap;
+        int64_t K, e_begin, q_off, tr_off, g_off;
+        const double *tab;
+    } part[kMaxOrder];
+};
+
+constexpr int max_stage_lds(int a, int b) { return a > b ? a : b; }
+template <int N>
+constexpr int most_stage_lds() {
+    if constexpr (N == 1) return stage_lds<1>();
+    else return max_stage_lds(stage_lds<N>(), most_stage_lds<N - 1>());
+}
+
+template <int Top>  // the largest order among the groups
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(Top <= 8 ? 4 : Top <= 12 ? 3 : 2)))
+stage_groups_kernel(StageGroups groups, const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+                    const BcSide *__restrict__ bc, const double *q, double *q_out, double *__restrict__ g,
+                    const double *__restrict__ w_in, double *__restrict__ w_out, const double *__restrict__ tr_in,
+                    double *__restrict__ tr_out, const double *__restrict__ side_flux, int flags, double a, double gdt,
+                    StageClock clock, double cw) {
+    __shared__ double mem[most_stage_lds<Top>()];
+    int i = 0;
+    while (i + 1 < groups.n && (int)blockIdx.x >= groups.first[i + 1]) ++i;
+    const auto &G = groups.part[i];
+    const int b = (int)blockIdx.x - groups.first[i], n_blocks = groups.first[i + 1] - groups.first[i];
+    const int64_t blk = G.remap ? xcd_block(b, n_blocks) : b;
+    auto run = [&](auto order) {
+        constexpr int N = decltype(order)::value;
+        constexpr int EPB = LineShape<N>::EPB, tile = EPB * 3 * StageTile<N>::NEP;
+        stage_tile<N, false>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, q + G.q_off, q_out + G.q_off,
+                             g + G.g_off, w_in + G.tr_off / 3, w_out + G.tr_off / 3, tr_in + G.tr_off,
+                             tr_out + G.tr_off, nullptr, side_flux, G.K, flags, a, gdt, clock, G.epb, cw, blk, mem,
+                             mem + tile, mem + 2 * tile, mem + 2 * tile + StageTile<N>::kFlux);
+    };
+    switch (G.N) {
+#define NDG_RUN(n) \
+    case n:        \
+        if constexpr (n <= Top) run(std::integral_constant<int, n>()); \
+        break;
+        NDG_RUN(1) NDG_RUN(2) NDG_RUN(3) NDG_RUN(4) NDG_RUN(5) NDG_RUN(6) NDG_RUN(7) NDG_RUN(8)
+        NDG_RUN(9) NDG_RUN(10) NDG_RUN(11) NDG_RUN(12) NDG_RUN(13) NDG_RUN(14) NDG_RUN(15) NDG_RUN(16)
+#undef NDG_RUN
     }
 }
 
@@ -1847,6 +1919,10 @@ static StageClock stage_clock(const DeviceMesh &m, const Group &G, int stage, do
     return StageClock{m.clock + begin, kB[stage] * dt, next, dt};
 }
 
+static int stage_rk_flags(const DeviceMesh &m, int stage) {
+    return (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0) | stage_flags(m);
+}
+
 template <int N>
 static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, double dt, hipStream_t s) {
     using S = LineShape<N>;
@@ -1857,8 +1933,7 @@ static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, do
                        m.g + G.g_off, m.wave[m.cur] + G.tr_off / 3, m.wave[1 - m.cur] + G.tr_off / 3,
                        m.trace[m.cur] + G.tr_off,
                        m.trace[1 - m.cur] + G.tr_off, nullptr, m.side_flux, G.K,
-                       (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0) |
-                           stage_flags(m), a, gdt,
+                       stage_rk_flags(m, stage), a, gdt,
                        stage_clock(m, G, stage, dt), epb, G.tune[NDG_PRECISION_FP64].remap, m.wave_speed);
     return hipGetLastError();
 }
@@ -1980,11 +2055,63 @@ hipError_t launch_mortar(DeviceMesh &m, hipStream_t s) {
     return mortar_m<kMaxOrder + 1>(m, s);
 }
 
+// Workgroups per group beyond the first up to which one launch takes the stages of all groups: each
+// launch that it saves is worth some 6 us, and each workgroup costs a little more there, because its
+// registers and LDS are those of the largest order compiled into the kernel (4 workgroups a CU up to order
+// 8, 3 to order 12, 2 above). Measured, us a stage with one launch and with one a group, in parallel
+// graph branches where these are the faster: orders 4, 6, 8: 4,184 workgroups 46.3 and 50.5, 7,438 69.4
+// and 68.8; orders 10, 12: 944 workgroups 23.9 and 27.8, 3,774 58.5 and 55.0; orders 4 to 12 (5 groups):
+// 549 workgroups 18.1 and 39.6, 3,421 50.1 and 58.1, 8,759 115 and 105; orders 14, 16: 693 workgroups
+// 25.9 and 28.8, 2,770 64.9 and 61.7; orders 8 to 16 (5 groups): 1,900 workgroups 48.4 and 60.0, 3,377
+// 69.9 and 67.4.
+static int64_t groups_blocks(int top) { return top <= 8 ? 2048 : top <= 12 ? 1152 : 640; }
+
+template <int Top>
+static hipError_t stage_groups_top(DeviceMesh &m, const StageGroups &P, int stage, double a, double gdt, double dt,
+                                   hipStream_t s) {
+    hipLaunchKernelGGL(stage_groups_kernel<Top>, dim3((unsigned)P.first[P.n]), dim3(192), 0, s, P, m.verts, m.side_nb,
+                       m.bc, m.q, m.q_out ? m.q_out : m.q, m.g, m.wave[m.cur], m.wave[1 - m.cur], m.trace[m.cur],
+                       m.trace[1 - m.cur], m.side_flux, stage_rk_flags(m, stage), a, gdt,
+                       stage_clock(m, m.groups[0], stage, dt), m.wave_speed);
+    return hipGetLastError();
+}
+
+bool stage_groups_fit(const DeviceMesh &m) {
+    if (m.groups.size() < 2 || m.precision != NDG_PRECISION_FP64) return false;
+    int64_t blocks = 0;
+    int top = 0;
+    for (const Group &G : m.groups) {
+        blocks += (G.K + stage_tile_epb(G) - 1) / stage_tile_epb(G);
+        top = std::max(top, G.N);
+    }
+    return blocks <= groups_blocks(top) * (int64_t)(m.groups.size() - 1);
+}
+
+hipError_t launch_groups(DeviceMesh &m, int stage, double a, double gdt, double dt, hipStream_t s) {
+    if (!stage_groups_fit(m)) {
+        for (int g = 0; g < (int)m.groups.size(); ++g)
+            if (const hipError_t e = launch_group_stage(m, g, stage, a, gdt, dt, s); e != hipSuccess) return e;
+        return hipSuccess;
+    }
+    StageGroups P;
+    P.n = (int)m.groups.size();
+    P.first[0] = 0;
+    int top = 0;
+    for (int i = 0; i < P.n; ++i) {
+        const Group &G = m.groups[i];
+        const int epb = stage_tile_epb(G);
+        P.part[i] = {G.N, epb, G.tune[NDG_PRECISION_FP64].remap, G.K, G.e_begin, G.q_off, G.tr_off, G.g_off, G.tab};
+        P.first[i + 1] = P.first[i] + (int)((G.K + epb - 1) / epb);
+        top = std::max(top, G.N);
+    }
+    if (top <= 8) return stage_groups_top<8>(m, P, stage, a, gdt, dt, s);
+    if (top <= 12) return stage_groups_top<12>(m, P, stage, a, gdt, dt, s);
+    return stage_groups_top<kMaxOrder>(m, P, stage, a, gdt, dt, s);
+}
+
 hipError_t launch_stage(DeviceMesh &m, int stage, double a, double gdt, double dt, hipStream_t s) {
     hipError_t e = launch_mortar(m, s);
-    if (e != hipSuccess) return e;
-    for (int g = 0; g < (int)m.groups.size(); ++g)
-        if ((e = launch_group_stage(m, g, stage, a, gdt, dt, s)) != hipSuccess) return e;
+    if (e != hipSuccess || (e = launch_groups(m, stage, a, gdt, dt, s)) != hipSuccess) return e;
     m.cur = 1 - m.cur;
     return hipSuccess;
 }

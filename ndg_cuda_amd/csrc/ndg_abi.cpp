@@ -1804,7 +1804,7 @@ ndg_status launch_step_body(ndg_mesh *m, double dt, bool parallel, hipStream_t s
     const int ng = (int)d.groups.size();
     for (int st = 0; st < 3; ++st) {
         HIP_TRY(launch_mortar(d, s), "mortar kernel");
-        if (parallel && ng > 1) {
+        if (parallel && ng > 1 && !stage_groups_fit(d)) {
             // one branch per group, the groups with the most bytes forked first (their launches
             // are the longest)
             std::vector<int> gorder(ng);
@@ -1822,8 +1822,7 @@ ndg_status launch_step_body(ndg_mesh *m, double dt, bool parallel, hipStream_t s
                 HIP_TRY(hipStreamWaitEvent(s, m->side_events[1 + g], 0), "join wait");
             }
         } else {
-            for (int g = 0; g < ng; ++g)
-                HIP_TRY(launch_group_stage(d, g, st, kAm[st], kGm[st] * dt, dt, s), "stage kernel");
+            HIP_TRY(launch_groups(d, st, kAm[st], kGm[st] * dt, dt, s), "stage kernel");
         }
         d.cur = 1 - d.cur;
     }

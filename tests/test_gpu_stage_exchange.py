@@ -142,3 +142,19 @@ def test_smaller_tiles_of_the_tuner(N):
 def test_fp32c_tiles_and_remainders(N, nx, ny, bc):
     """One element, exactly one tile, and tiles with a remainder, in the FP32 form."""
     compare(grid(nx, ny, bc, jitter=0.1 if min(nx, ny) > 1 else 0.0), N, precision="fp32c")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bc", [nd.BC_WALL, nd.BC_INFLOW])
+@pytest.mark.parametrize("orders", [(1, 2), (1, 8), (3, 4, 8), (1, 9), (5, 8, 12), (2, 13), (1, 7, 12, 16), tuple(range(1, 17))])
+def test_groups_in_one_launch(orders, bc):
+    """Few elements of each order: partial tiles, every kernel of the one-launch form (up to 8, 12, 16)."""
+    rng = np.random.default_rng(len(orders))
+    compare(grid(6, 5, bc), min(orders), orders=rng.permutation(np.resize(orders, 30)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(260, 170), (260, 260)])
+def test_groups_on_both_sides_of_the_line(nx, ny):
+    """1,744 and 2,667 workgroups of two groups: one launch for both, one launch each."""
+    compare(grid(nx, ny), 1, orders=np.where(np.arange(nx * ny) % nx < nx // 2, 1, 2), steps=1)
