@@ -19,7 +19,8 @@
 //   rho_0[i] = sum_j lm[j] nu[i][j] / w[j],  rho_2[N-i] = sum_j lp[j] nu[i][j] / w[j]
 // (rho_s is the adjoint of the side flux F*_s); per side point omega_L = sf (rho_p + n.rho_uv)/2,
 // omega_R = sf (-rho_p + n.rho_uv)/2; the own trace adjoint is (omega_L, n omega_L) plus what the
-// neighbour exports for this point, chi = (omega_R, -n omega_R) computed on its side; finally the
+// neighbour exports for this point, chi = (omega_R, -n omega_R) computed on its side (only omega_R is
+// stored: -n is the receiver's own normal, or for an oblique periodic side found from the partner); finally the
 // traces' and fluxes' transposes scatter into lambda:
 //   dl_p += y_eta Fbar_u - x_eta Fbar_v - y_xi Gbar_u + x_xi Gbar_v,
 //   dl_u += y_eta Fbar_p - y_xi Gbar_p,  dl_v += -x_eta Fbar_p + x_xi Gbar_p,
@@ -51,6 +52,10 @@ constexpr int kAdjExport = 4;   // export chi for the next reverse stage
 constexpr int kAdjApply = 8;    // do the transpose (off: export only)
 constexpr int kAdjSource = 16;  // add the receivers' misfit source to lambda' before the export
 
+// Bound by the phases' latency and, at large sizes, by the state's traffic (lambda and mu read and
+// written, q_s read). 128 x 128, N = 8: 41 us a launch, 50 us before the contractions took D^T from the lanes
+// of registers by even and odd parts (scalar loads a row at a time), one value a side point was
+// exchanged instead of three and the branch on the field left P5's loop.
 template <int N>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 10 ? 3 : 2)))
 adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
@@ -71,35 +76,36 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
     const double *lm = tab + NF * NF;
     const double *lp = lm + NF;
     const double *x = lp + 2 * NF;
-    const double *winv = x + NF;
-    const double *DhT = tab + 2 * NF * NF + 5 * NF;  // DhT[a][i] = Dh[i][a]
+    const double *lpw = tab + table_stage_offset(N);  // l(+1) / w; that of l(-1) is its reverse
 
     const int tid = threadIdx.x;
     const int f = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int el = lane / NF, l = lane % NF;
     const int64_t e0 = (int64_t)blockIdx.x * EPB;
     const int nel = (int)min<int64_t>(EPB, K - e0);
-    const bool active = el < nel;
+    const bool active = lane < nel * NF;
+    // lanes past the tile's lines work on line 0 of its first element, so that every lane takes part
+    // in the D^ broadcasts, and store nothing
+    const int el = active ? lane / NF : 0, l = active ? lane % NF : 0;
     const bool apply = flags & kAdjApply;
 
     // P0: connectivity and neighbour exports of the thread's flux points, lambda and mu tiles,
     // vertices.
-    double nbv[FPT][3];
+    int32_t code[FPT];
+    double ext[FPT];
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
-        nbv[it][0] = nbv[it][1] = nbv[it][2] = 0.0;
         const int item = tid + it * T;
-        if (apply && item < nel * 4 * NF) {
-            int32_t cd = side_nb[(e0 + item / NF / 4) * 4 + (item / NF) % 4];
-            const int k = item % NF;
-            // the host admits interior and periodic sides only: a record is an oblique periodic side's
-            if (cd < 0) cd = (int32_t)bc[-1 - cd].partner;
-            const double *nb = chi_in + (int64_t)(cd >> 2) * 12 * NF + (cd & 3) * 3 * NF + (N - k);
-            nbv[it][0] = nb[0];
-            nbv[it][1] = nb[NF];
-            nbv[it][2] = nb[2 * NF];
-        }
+        code[it] = item < nel * 4 * NF ? side_nb[e0 * 4 + item / NF] : 0;
+    }
+    LaneTable<even_odd_len(NF)> Dt;
+    Dt.load(tab + table_adjoint_offset(N));
+#pragma unroll
+    for (int it = 0; it < FPT; ++it) {
+        int32_t cd = code[it];
+        // the host admits interior and periodic sides only: a record is an oblique periodic side's
+        if (cd < 0) cd = (int32_t)bc[-1 - cd].partner;
+        ext[it] = apply ? chi_in[(int64_t)cd * NF + (N - (tid + it * T) % NF)] : 0.0;
     }
     double mreg[QPT], lreg[QPT], qreg[QPT];
     const double *lg = lam + e0 * 3 * NE;
@@ -173,8 +179,8 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
         // P3 (same phase as P1, which writes only the metric and side arrays): per field f, the lift transposes rho of the four sides and the volume transpose
         // Fbar_f[a][l] = sum_i Dh[i][a] nu_f[i][l] (column l, into s_a); row l of nu_f stays in
         // registers for P4. One contraction per field and direction: the same work in each wave.
-        double row[NF];
-        if (active) {
+        double row[NF], t[NF];
+        {
             const double *nb = s_n + el * 3 * NE + f * NE;
             double col[NF];
 #pragma unroll
@@ -185,39 +191,33 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
             double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
 #pragma unroll
             for (int m = 0; m < NF; ++m) {
-                r1 += lp[m] * winv[m] * col[m];
-                r3 += lm[m] * winv[m] * col[m];
-                r0 += lm[m] * winv[m] * row[m];
-                r2 += lp[m] * winv[m] * row[m];
+                r1 += lpw[m] * col[m];
+                r3 += lpw[N - m] * col[m];
+                r0 += lpw[N - m] * row[m];
+                r2 += lpw[m] * row[m];
             }
-            double *rho = s_rho + el * 12 * NF + f * NF;
-            rho[l] = r0;
-            rho[3 * NF + l] = r1;
-            rho[6 * NF + (N - l)] = r2;
-            rho[9 * NF + (N - l)] = r3;
-            double *fb = s_a + el * 3 * NE + f * NE + l;
-#pragma unroll 1
-            for (int a = 0; a < NF; ++a) {
-                double F = 0.0;
+            contract<NF>(Dt, col, t);
+            if (active) {
+                double *rho = s_rho + el * 12 * NF + f * NF;
+                rho[l] = r0;
+                rho[3 * NF + l] = r1;
+                rho[6 * NF + (N - l)] = r2;
+                rho[9 * NF + (N - l)] = r3;
+                double *fb = s_a + el * 3 * NE + f * NE + l;
 #pragma unroll
-                for (int i = 0; i < NF; ++i) F += DhT[a * NF + i] * col[i];
-                fb[a * NF] = F;
+                for (int a = 0; a < NF; ++a) fb[a * NF] = t[a];
             }
         }
         __syncthreads();
 
         // P4: Gbar_f[l][b] = sum_j Dh[j][b] nu_f[l][j] in place of row l of nu_f (only this
         // thread reads that row from here on); flux transpose at the side points: own trace
-        // adjoint tau = (omega_L, n omega_L) plus the neighbour's export for this point.
+        // adjoint tau = (omega_L, n omega_L) plus the neighbour's (omega_R, -n' omega_R) for this point.
+        contract<NF>(Dt, row, t);
         if (active) {
             double *gs_ = s_n + el * 3 * NE + f * NE + l * NF;
-#pragma unroll 1
-            for (int b = 0; b < NF; ++b) {
-                double G = 0.0;
 #pragma unroll
-                for (int j = 0; j < NF; ++j) G += DhT[b * NF + j] * row[j];
-                gs_[b] = G;
-            }
+            for (int b = 0; b < NF; ++b) gs_[b] = t[b];
         }
 #pragma unroll
         for (int it = 0; it < FPT; ++it) {
@@ -226,11 +226,18 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
                 const int fe = item / (4 * NF), s = (item / NF) % 4, k = item % NF;
                 double *rho = s_rho + fe * 12 * NF + s * 3 * NF + k;
                 const double *sd = s_side + (fe * 4 + s) * 3;
-                const double nx = sd[0], ny = sd[1], sf = sd[2];
+                const double nx = sd[0], ny = sd[1], sf = sd[2], wr = ext[it];
                 const double wl = sf * ((rho[0] + nx * rho[NF] + ny * rho[2 * NF]) / 2);
-                rho[0] = wl + nbv[it][0];
-                rho[NF] = nx * wl + nbv[it][1];
-                rho[2 * NF] = ny * wl + nbv[it][2];
+                double mx = nx, my = ny;  // -n': the own normal on a side shared by two elements
+                if (code[it] < 0) {
+                    const int64_t cd = bc[-1 - code[it]].partner;
+                    side_geometry(verts + (cd >> 2) * 8, (int)(cd & 3), mx, my);
+                    mx = -mx;
+                    my = -my;
+                }
+                rho[0] = wl + wr;
+                rho[NF] = nx * wl + mx * wr;
+                rho[2 * NF] = ny * wl + my * wr;
             }
         }
         __syncthreads();
@@ -250,18 +257,22 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
             const double *tau = s_rho + el * 12 * NF + f * NF;
             const double t0 = tau[i], t2 = tau[6 * NF + (N - i)];
             const double ye = met[NF + i], xe = met[i], lpi = lp[i], lmi = lm[i];
+            // (a branch on the field inside the loop would keep each LDS read from overlapping the next)
+            if (f == 0) {
 #pragma unroll
-            for (int b = 0; b < NF; ++b) {
-                const double yx = met[3 * NF + b], xx = met[2 * NF + b];
-                double v;
-                if (f == 0)
-                    v = ye * Fb[NE + b] - xe * Fb[2 * NE + b] - yx * Gb[NE + b] + xx * Gb[2 * NE + b];
-                else if (f == 1)
-                    v = ye * Fb[b] - yx * Gb[b];
-                else
-                    v = -(xe * Fb[b]) + xx * Gb[b];
-                da[b] = v + lm[b] * t0 + lp[b] * t2 + lpi * tau[3 * NF + b] + lmi * tau[9 * NF + (N - b)];
+                for (int b = 0; b < NF; ++b)
+                    da[b] = ye * Fb[NE + b] - xe * Fb[2 * NE + b] - met[3 * NF + b] * Gb[NE + b] +
+                            met[2 * NF + b] * Gb[2 * NE + b];
+            } else if (f == 1) {
+#pragma unroll
+                for (int b = 0; b < NF; ++b) da[b] = ye * Fb[b] - met[3 * NF + b] * Gb[b];
+            } else {
+#pragma unroll
+                for (int b = 0; b < NF; ++b) da[b] = -(xe * Fb[b]) + met[2 * NF + b] * Gb[b];
             }
+#pragma unroll
+            for (int b = 0; b < NF; ++b)
+                da[b] += lm[b] * t0 + lp[b] * t2 + lpi * tau[3 * NF + b] + lmi * tau[9 * NF + (N - b)];
         }
         __syncthreads();
         if (active) {
@@ -335,10 +346,10 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
 #pragma unroll
         for (int m = 0; m < NF; ++m) {
             const double col = nf_[m * NF + l], row = nf_[l * NF + m];
-            r1 += lp[m] * winv[m] * col;
-            r3 += lm[m] * winv[m] * col;
-            r0 += lm[m] * winv[m] * row;
-            r2 += lp[m] * winv[m] * row;
+            r1 += lpw[m] * col;
+            r3 += lpw[N - m] * col;
+            r0 += lpw[N - m] * row;
+            r2 += lpw[m] * row;
         }
         double *rho = s_rho + el * 12 * NF + f * NF;
         rho[l] = r0;
@@ -347,7 +358,7 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
         rho[9 * NF + (N - l)] = r3;
     }
     __syncthreads();
-    // P9: the export chi = (omega_R, -n omega_R) of every side point.
+    // P9: the export chi = omega_R of every side point.
 #pragma unroll
     for (int it = 0; it < FPT; ++it) {
         const int item = tid + it * T;
@@ -356,11 +367,7 @@ adjoint_stage_kernel(const double *__restrict__ verts, const int32_t *__restrict
             const double *rho = s_rho + fe * 12 * NF + s * 3 * NF + k;
             const double *sd = s_side + (fe * 4 + s) * 3;
             const double nx = sd[0], ny = sd[1], sf = sd[2];
-            const double wr = sf * ((-rho[0] + nx * rho[NF] + ny * rho[2 * NF]) / 2);
-            double *co = chi_out + (e0 + fe) * 12 * NF + s * 3 * NF + k;
-            co[0] = wr;
-            co[NF] = -(nx * wr);
-            co[2 * NF] = -(ny * wr);
+            chi_out[e0 * 4 * NF + item] = sf * ((-rho[0] + nx * rho[NF] + ny * rho[2 * NF]) / 2);
         }
     }
 }

@@ -113,22 +113,21 @@ __host__ __device__ inline int64_t mortar_matrix_key(int Ne, int Nf, int side, i
 constexpr int64_t kMortarMatrixKeys = (int64_t)(kMaxOrder + 1) * (kMaxOrder + 1) * 4 * kMortarClasses;
 
 // Per-order constant tables in device memory, packed as Dhat[Nf*Nf], l(-1)[Nf], l(+1)[Nf], w[Nf],
-// x[Nf], 1/w[Nf], then the modal matrix poly[Nf*Nf] used by the estimator, the transpose
-// Dhat^T[Nf*Nf] used by the adjoint (its columns as contiguous rows), and for the stage kernel
-// l(+1)/w[Nf] and the even and odd parts of Dhat (see contract in kernels.hip).
+// x[Nf], 1/w[Nf], then the modal matrix poly[Nf*Nf] used by the estimator, the even and odd parts of
+// Dhat^T (see contract in device.hpp) used by the adjoint, and for both stage kernels l(+1)/w[Nf] and
+// the even and odd parts of Dhat.
 __host__ __device__ constexpr int even_odd_len(int nf) {
     return (nf / 2) * (2 * (nf / 2) + nf % 2) + (nf % 2) * (nf / 2);
 }
 inline int64_t table_pack_len(int N) {
     const int nf = N + 1;
-    return (int64_t)nf * nf * 3 + 6 * nf + even_odd_len(nf);
+    return (int64_t)nf * nf * 2 + 6 * nf + 2 * even_odd_len(nf);
+}
+__host__ __device__ constexpr int64_t table_adjoint_offset(int N) {
+    return (int64_t)(N + 1) * (N + 1) * 2 + 5 * (N + 1);
 }
 __host__ __device__ constexpr int64_t table_stage_offset(int N) {
-    return (int64_t)(N + 1) * (N + 1) * 3 + 5 * (N + 1);
-}
-inline int64_t table_dhat_t_offset(int N) {
-    const int nf = N + 1;
-    return (int64_t)nf * nf * 2 + 5 * nf;
+    return table_adjoint_offset(N) + even_odd_len(N + 1);
 }
 inline int64_t table_poly_offset(int N) {
     const int nf = N + 1;

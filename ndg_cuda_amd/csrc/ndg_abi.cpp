@@ -3021,7 +3021,7 @@ extern "C" ndg_status ndg_apply_rhs_transpose(ndg_mesh *mesh, const double *mp, 
     DevBuf lam, muv, chi;
     if ((st = dev_alloc(lam, sizeof(double) * d.n_q, "hipMalloc adjoint")) != NDG_OK) return st;
     if ((st = dev_alloc(muv, sizeof(double) * d.n_q, "hipMalloc adjoint")) != NDG_OK) return st;
-    if ((st = dev_alloc(chi, sizeof(double) * d.n_tr, "hipMalloc adjoint")) != NDG_OK) return st;
+    if ((st = dev_alloc(chi, sizeof(double) * d.n_tr / 3, "hipMalloc adjoint")) != NDG_OK) return st;
     HIP_TRY(hipStreamSynchronize(mesh->stream), "ndg_apply_rhs_transpose sync");
     double *const ins[3] = {const_cast<double *>(mp), const_cast<double *>(mu), const_cast<double *>(mv)};
     if ((st = copy_state(mesh, muv.as<double>(), ins, false, "upload adjoint")) != NDG_OK) return st;
@@ -3097,8 +3097,8 @@ extern "C" ndg_status ndg_adjoint_gradient(ndg_mesh *mesh, const ndg_receivers *
     double *const rbuf[2] = {n_kept >= 1 ? block(0) : nullptr, n_kept >= 2 ? block(1) : (n_blocks > 1 ? block(1) : nullptr)};
     if ((st = dev_alloc(lam, qb, "hipMalloc adjoint")) != NDG_OK) return st;
     if ((st = dev_alloc(mu, qb, "hipMalloc adjoint")) != NDG_OK) return st;
-    if ((st = dev_alloc(chi0, sizeof(double) * d.n_tr, "hipMalloc adjoint")) != NDG_OK) return st;
-    if ((st = dev_alloc(chi1, sizeof(double) * d.n_tr, "hipMalloc adjoint")) != NDG_OK) return st;
+    if ((st = dev_alloc(chi0, sizeof(double) * d.n_tr / 3, "hipMalloc adjoint")) != NDG_OK) return st;
+    if ((st = dev_alloc(chi1, sizeof(double) * d.n_tr / 3, "hipMalloc adjoint")) != NDG_OK) return st;
     const int64_t nblk = adjoint_blocks(d);
     if ((st = dev_alloc(cpart, sizeof(double) * nblk, "hipMalloc adjoint")) != NDG_OK) return st;
     if ((st = dev_alloc(recs, sizeof(double) * R.n * n_steps, "hipMalloc records")) != NDG_OK) return st;

@@ -169,18 +169,21 @@ std::vector<double> pack_tables(const Tables &t, int N) {
     for (int i = 0; i < nf; ++i) out.push_back(1.0 / t.tab[NDG_TABLE_WEIGHTS][N][i]);
     const auto &M = t.tab[NDG_TABLE_POLYNOMIALS][N];
     out.insert(out.end(), M.begin(), M.end());
-    for (int a = 0; a < nf; ++a)
-        for (int i = 0; i < nf; ++i) out.push_back(Dh[i * nf + a]);
-    for (int i = 0; i < nf; ++i) out.push_back(t.tab[NDG_TABLE_LAGRANGE_RIGHT][N][i] / t.tab[NDG_TABLE_WEIGHTS][N][i]);
-    const int h = nf / 2;
-    for (int i = 0; i < h + nf % 2; ++i) {
-        const double *row = Dh.data() + i * nf;
-        if (i < h) {
-            for (int k = 0; k < h; ++k) out.push_back((row[k] + row[N - k]) / 2);
-            if (nf % 2) out.push_back(row[h]);
+    // even and odd parts of D^ (transposed: of its transpose)
+    auto even_odd = [&](bool transposed) {
+        auto D = [&](int i, int k) { return transposed ? Dh[k * nf + i] : Dh[i * nf + k]; };
+        const int h = nf / 2;
+        for (int i = 0; i < h + nf % 2; ++i) {
+            if (i < h) {
+                for (int k = 0; k < h; ++k) out.push_back((D(i, k) + D(i, N - k)) / 2);
+                if (nf % 2) out.push_back(D(i, h));
+            }
+            for (int k = 0; k < h; ++k) out.push_back((D(i, k) - D(i, N - k)) / 2);
         }
-        for (int k = 0; k < h; ++k) out.push_back((row[k] - row[N - k]) / 2);
-    }
+    };
+    even_odd(true);
+    for (int i = 0; i < nf; ++i) out.push_back(t.tab[NDG_TABLE_LAGRANGE_RIGHT][N][i] / t.tab[NDG_TABLE_WEIGHTS][N][i]);
+    even_odd(false);
     return out;
 }
 
