@@ -689,8 +689,28 @@ struct StageGroups {
         int N, epb, remap;
         int64_t K, e_begin, q_off, tr_off, g_off;
         const double *tab;
+        const float *tab32;
     } part[kMaxOrder];
 };
+
+// Calls run(order, part, tile) for the workgroup's group.
+template <int Top, class Run>
+__device__ __forceinline__ void run_group(const StageGroups &groups, Run &&run) {
+    int i = 0;
+    while (i + 1 < groups.n && (int)blockIdx.x >= groups.first[i + 1]) ++i;
+    const StageGroups::Part &G = groups.part[i];
+    const int b = (int)blockIdx.x - groups.first[i], n_blocks = groups.first[i + 1] - groups.first[i];
+    const int64_t blk = G.remap ? xcd_block(b, n_blocks) : b;
+    switch (G.N) {
+#define NDG_RUN(n) \
+    case n:        \
+        if constexpr (n <= Top) run(std::integral_constant<int, n>(), G, blk); \
+        break;
+        NDG_RUN(1) NDG_RUN(2) NDG_RUN(3) NDG_RUN(4) NDG_RUN(5) NDG_RUN(6) NDG_RUN(7) NDG_RUN(8)
+        NDG_RUN(9) NDG_RUN(10) NDG_RUN(11) NDG_RUN(12) NDG_RUN(13) NDG_RUN(14) NDG_RUN(15) NDG_RUN(16)
+#undef NDG_RUN
+    }
+}
 
 constexpr int max_stage_lds(int a, int b) { return a > b ? a : b; }
 template <int N>
@@ -707,28 +727,14 @@ stage_groups_kernel(StageGroups groups, const double *__restrict__ verts, const 
                     double *__restrict__ tr_out, const double *__restrict__ side_flux, int flags, double a, double gdt,
                     StageClock clock, double cw) {
     __shared__ double mem[most_stage_lds<Top>()];
-    int i = 0;
-    while (i + 1 < groups.n && (int)blockIdx.x >= groups.first[i + 1]) ++i;
-    const auto &G = groups.part[i];
-    const int b = (int)blockIdx.x - groups.first[i], n_blocks = groups.first[i + 1] - groups.first[i];
-    const int64_t blk = G.remap ? xcd_block(b, n_blocks) : b;
-    auto run = [&](auto order) {
+    run_group<Top>(groups, [&](auto order, const StageGroups::Part &G, int64_t blk) {
         constexpr int N = decltype(order)::value;
         constexpr int EPB = LineShape<N>::EPB, tile = EPB * 3 * StageTile<N>::NEP;
         stage_tile<N, false>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, q + G.q_off, q_out + G.q_off,
                              g + G.g_off, w_in + G.tr_off / 3, w_out + G.tr_off / 3, tr_in + G.tr_off,
                              tr_out + G.tr_off, nullptr, side_flux, G.K, flags, a, gdt, clock, G.epb, cw, blk, mem,
                              mem + tile, mem + 2 * tile, mem + 2 * tile + StageTile<N>::kFlux);
-    };
-    switch (G.N) {
-#define NDG_RUN(n) \
-    case n:        \
-        if constexpr (n <= Top) run(std::integral_constant<int, n>()); \
-        break;
-        NDG_RUN(1) NDG_RUN(2) NDG_RUN(3) NDG_RUN(4) NDG_RUN(5) NDG_RUN(6) NDG_RUN(7) NDG_RUN(8)
-        NDG_RUN(9) NDG_RUN(10) NDG_RUN(11) NDG_RUN(12) NDG_RUN(13) NDG_RUN(14) NDG_RUN(15) NDG_RUN(16)
-#undef NDG_RUN
-    }
+    });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -995,23 +1001,24 @@ __device__ __forceinline__ void record_flux32(const SideRecord &rec, const BcSid
 // workgroups fills the chip the wait for the tile decides: 128 x 128, N = 8: 23.6 and 24.1 us, 96 x 96:
 // 14.1 and 13.9 us.
 template <int N>
-__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 9 ? 5 : 4)))
-stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
-                 const BcSide *__restrict__ bc, const double *__restrict__ tab64,
-                 const float *__restrict__ tab, float *__restrict__ qh, float2 *__restrict__ gl,
-                 const float *__restrict__ w_in, float *__restrict__ w_out, const float *__restrict__ tr_in,
-                 float *__restrict__ tr_out, const float *__restrict__ side_flux, int64_t K, int flags, float a, float gdt,
-                 StageClock clock, int remap, double cw) {
+__device__ __forceinline__ void
+stage_c32_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+               const BcSide *__restrict__ bc, const double *__restrict__ tab64,
+               const float *__restrict__ tab, float *__restrict__ qh, float2 *__restrict__ gl,
+               const float *__restrict__ w_in, float *__restrict__ w_out, const float *__restrict__ tr_in,
+               float *__restrict__ tr_out, const float *__restrict__ side_flux, int64_t K, int flags, float a, float gdt,
+               const StageClock &clock, double cw, int64_t blk,
+               float *__restrict__ s_q,     // the state tile
+               float *__restrict__ s_d,     // d_xi, then the new traces on sides 1 and 3
+               float *__restrict__ s_f,     // fluxes, then the new traces on sides 0 and 2
+               float *__restrict__ s_met,   // metric lines
+               float *__restrict__ s_side)  // outward normal and edge Jacobian (negative: a mortar side)
+{
     const bool first = flags & kRkFirst, once = flags & kStream;
     using S = LineShape<N>;
     constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT, NFP = NF | 1, NEP = NF * NFP;
     constexpr int QP4 = (EPB * 3 * NE + 31 + 4 * T - 1) / (4 * T);  // 16-byte words of the tile per thread
     constexpr int run = rk_run<N>(EPB);
-    __shared__ float s_q[EPB * 3 * NEP];
-    __shared__ float s_d[EPB * 3 * NEP];    // d_xi, then the new traces on sides 1 and 3
-    __shared__ float s_f[EPB * 12 * NF];    // fluxes, then the new traces on sides 0 and 2
-    __shared__ float s_met[EPB * 4 * NF];
-    __shared__ float s_side[EPB * 4 * 3];   // outward normal and edge Jacobian (negative: a mortar side)
     const float *lm = tab + NF * NF;
     const float *lp = lm + NF;
     const float *winv = lp + 3 * NF;
@@ -1020,7 +1027,6 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
     const int tid = threadIdx.x;
     const int f = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int64_t blk = remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
     const int64_t e0 = blk * EPB;
     const int nel = (int)min<int64_t>(EPB, K - e0);
     const int n_val = nel * 3 * NE, n_pt = nel * 4 * NF;
@@ -1310,6 +1316,51 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
             to[2 * NF] = v;
         }
     }
+}
+
+template <int N>
+struct StageTile32 {
+    static constexpr int EPB = LineShape<N>::EPB, NF = N + 1, tile = EPB * 3 * NF * (NF | 1), flux = EPB * 12 * NF,
+                         met = EPB * 4 * NF, side = EPB * 12, lds = 2 * tile + flux + met + side;
+};
+
+template <int N>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 9 ? 5 : 4)))
+stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+                 const BcSide *__restrict__ bc, const double *__restrict__ tab64,
+                 const float *__restrict__ tab, float *__restrict__ qh, float2 *__restrict__ gl,
+                 const float *__restrict__ w_in, float *__restrict__ w_out, const float *__restrict__ tr_in,
+                 float *__restrict__ tr_out, const float *__restrict__ side_flux, int64_t K, int flags, float a, float gdt,
+                 StageClock clock, int remap, double cw) {
+    using L = StageTile32<N>;
+    __shared__ float s_q[L::tile], s_d[L::tile], s_f[L::flux], s_met[L::met], s_side[L::side];
+    stage_c32_tile<N>(verts, side_nb, bc, tab64, tab, qh, gl, w_in, w_out, tr_in, tr_out, side_flux, K, flags, a, gdt, clock,
+                      cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d, s_f, s_met, s_side);
+}
+
+template <int N>
+constexpr int most_stage_lds32() {
+    if constexpr (N == 1) return StageTile32<1>::lds;
+    else return max_stage_lds(StageTile32<N>::lds, most_stage_lds32<N - 1>());
+}
+
+// stage_groups_kernel for the FP32 form.
+template <int Top>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(Top <= 8 ? 5 : Top <= 12 ? 4 : 3)))
+stage_c32_groups_kernel(StageGroups groups, const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+                        const BcSide *__restrict__ bc, float *__restrict__ qh, float2 *__restrict__ gl,
+                        const float *__restrict__ w_in, float *__restrict__ w_out, const float *__restrict__ tr_in,
+                        float *__restrict__ tr_out, const float *__restrict__ side_flux, int flags, float a, float gdt,
+                        StageClock clock, double cw) {
+    __shared__ float mem[most_stage_lds32<Top>()];
+    run_group<Top>(groups, [&](auto order, const StageGroups::Part &G, int64_t blk) {
+        constexpr int N = decltype(order)::value;
+        using L = StageTile32<N>;
+        float *s_f = mem + 2 * L::tile, *s_met = s_f + L::flux;
+        stage_c32_tile<N>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, G.tab32, qh + G.q_off, gl + G.g_off,
+                          w_in + G.tr_off / 3, w_out + G.tr_off / 3, tr_in + G.tr_off, tr_out + G.tr_off, side_flux,
+                          G.K, flags, a, gdt, clock, cw, blk, mem, mem + L::tile, s_f, s_met, s_met + L::met);
+    });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1879,16 +1930,19 @@ static hipError_t traces_c32_n(const DeviceMesh &m, const Group &G, hipStream_t 
     return hipGetLastError();
 }
 
+static int stage_c32_flags(const DeviceMesh &m, int stage) {
+    return (stage == 0 ? kRkFirst : 0) | (m.trace_all ? kTraceAll : 0) | (12 * m.n_q > kStreamBytes ? kStream : 0);
+}
+
 template <int N>
 static hipError_t stage_c32_n(DeviceMesh &m, const Group &G, int stage, double a, double gdt, double dt,
                               hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    const int flags = (stage == 0 ? kRkFirst : 0) | (m.trace_all ? kTraceAll : 0) | (12 * m.n_q > kStreamBytes ? kStream : 0);
     hipLaunchKernelGGL(stage_c32_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, G.tab32, m.qh + G.q_off, m.gl32 + G.g_off,
                        m.wave32[m.cur] + G.tr_off / 3, m.wave32[1 - m.cur] + G.tr_off / 3, m.trace32[m.cur] + G.tr_off,
-                       m.trace32[1 - m.cur] + G.tr_off, m.side_flux32, G.K, flags, (float)a, (float)gdt,
+                       m.trace32[1 - m.cur] + G.tr_off, m.side_flux32, G.K, stage_c32_flags(m, stage), (float)a, (float)gdt,
                        stage_clock(m, G, stage, dt), G.tune[NDG_PRECISION_FP32_COMPENSATED].remap, m.wave_speed);
     return hipGetLastError();
 }
@@ -1964,25 +2018,37 @@ hipError_t launch_mortar(DeviceMesh &m, hipStream_t s) {
 // and 68.8; orders 10, 12: 944 workgroups 23.9 and 27.8, 3,774 58.5 and 55.0; orders 4 to 12 (5 groups):
 // 549 workgroups 18.1 and 39.6, 3,421 50.1 and 58.1, 8,759 115 and 105; orders 14, 16: 693 workgroups
 // 25.9 and 28.8, 2,770 64.9 and 61.7; orders 8 to 16 (5 groups): 1,900 workgroups 48.4 and 60.0, 3,377
-// 69.9 and 67.4.
+// 69.9 and 67.4. The FP32 form, whose kernels lose less occupancy there, takes the same line: orders 4 to 12:
+// 549 workgroups 18.1 and 39.3, 3,421 43.1 and 57.0; orders 10, 12: 944 workgroups 20.2 and 28.2.
 static int64_t groups_blocks(int top) { return top <= 8 ? 2048 : top <= 12 ? 1152 : 640; }
+
+static int stage_epb(const DeviceMesh &m, const Group &G) {
+    return m.precision == NDG_PRECISION_FP32_COMPENSATED ? stage_max_epb(G.N) : stage_tile_epb(G);
+}
 
 template <int Top>
 static hipError_t stage_groups_top(DeviceMesh &m, const StageGroups &P, int stage, double a, double gdt, double dt,
                                    hipStream_t s) {
-    hipLaunchKernelGGL(stage_groups_kernel<Top>, dim3((unsigned)P.first[P.n]), dim3(192), 0, s, P, m.verts, m.side_nb,
-                       m.bc, m.q, m.q_out ? m.q_out : m.q, m.g, m.wave[m.cur], m.wave[1 - m.cur], m.trace[m.cur],
-                       m.trace[1 - m.cur], m.side_flux, stage_rk_flags(m, stage), a, gdt,
-                       stage_clock(m, m.groups[0], stage, dt), m.wave_speed);
+    if (m.precision == NDG_PRECISION_FP32_COMPENSATED)
+        hipLaunchKernelGGL(stage_c32_groups_kernel<Top>, dim3((unsigned)P.first[P.n]), dim3(192), 0, s, P, m.verts,
+                           m.side_nb, m.bc, m.qh, m.gl32, m.wave32[m.cur], m.wave32[1 - m.cur], m.trace32[m.cur],
+                           m.trace32[1 - m.cur], m.side_flux32, stage_c32_flags(m, stage), (float)a, (float)gdt,
+                           stage_clock(m, m.groups[0], stage, dt), m.wave_speed);
+    else
+        hipLaunchKernelGGL(stage_groups_kernel<Top>, dim3((unsigned)P.first[P.n]), dim3(192), 0, s, P, m.verts, m.side_nb,
+                           m.bc, m.q, m.q_out ? m.q_out : m.q, m.g, m.wave[m.cur], m.wave[1 - m.cur], m.trace[m.cur],
+                           m.trace[1 - m.cur], m.side_flux, stage_rk_flags(m, stage), a, gdt,
+                           stage_clock(m, m.groups[0], stage, dt), m.wave_speed);
     return hipGetLastError();
 }
 
 bool stage_groups_fit(const DeviceMesh &m) {
-    if (m.groups.size() < 2 || m.precision != NDG_PRECISION_FP64) return false;
+    if (m.groups.size() < 2) return false;
     int64_t blocks = 0;
     int top = 0;
     for (const Group &G : m.groups) {
-        blocks += (G.K + stage_tile_epb(G) - 1) / stage_tile_epb(G);
+        const int epb = stage_epb(m, G);
+        blocks += (G.K + epb - 1) / epb;
         top = std::max(top, G.N);
     }
     return blocks <= groups_blocks(top) * (int64_t)(m.groups.size() - 1);
@@ -2000,8 +2066,8 @@ hipError_t launch_groups(DeviceMesh &m, int stage, double a, double gdt, double 
     int top = 0;
     for (int i = 0; i < P.n; ++i) {
         const Group &G = m.groups[i];
-        const int epb = stage_tile_epb(G);
-        P.part[i] = {G.N, epb, G.tune[NDG_PRECISION_FP64].remap, G.K, G.e_begin, G.q_off, G.tr_off, G.g_off, G.tab};
+        const int epb = stage_epb(m, G);
+        P.part[i] = {G.N, epb, G.tune[m.precision].remap, G.K, G.e_begin, G.q_off, G.tr_off, G.g_off, G.tab, G.tab32};
         P.first[i + 1] = P.first[i] + (int)((G.K + epb - 1) / epb);
         top = std::max(top, G.N);
     }

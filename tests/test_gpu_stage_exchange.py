@@ -158,3 +158,10 @@ def test_groups_in_one_launch(orders, bc):
 def test_groups_on_both_sides_of_the_line(nx, ny):
     """1,744 and 2,667 workgroups of two groups: one launch for both, one launch each."""
     compare(grid(nx, ny), 1, orders=np.where(np.arange(nx * ny) % nx < nx // 2, 1, 2), steps=1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("orders", [(1, 8), (3, 4, 8), (5, 8, 12), (2, 13), tuple(range(1, 17))])
+def test_fp32c_groups_in_one_launch(orders):
+    rng = np.random.default_rng(len(orders))
+    compare(grid(6, 5, nd.BC_INFLOW), min(orders), orders=rng.permutation(np.resize(orders, 30)), precision="fp32c")
