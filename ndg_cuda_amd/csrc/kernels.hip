@@ -165,10 +165,10 @@ traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side
 // three traces. Elements write the three traces of the sides with a record (and with kTraceAll of
 // every side) for these.
 //
-// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 321 us a
-// launch, 5.9 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches 5.3 to 5.8
+// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 317 us a
+// launch, 5.95 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches 5.3 to 5.8
 // here); 421 us and 2.18 GB with the traces exchanged. 512 x 512, N = 4: 116 us (164 us before). 128 x
-// 128, N = 8 (in the last-level cache): 25.0 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
+// 128, N = 8 (in the last-level cache): 24.8 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
 // us from launch to launch, 7.0 us before. What made the difference, at N = 8:
 //  - the state and the RK register are streamed past the caches (non-temporal, in 16-byte words on
 //    whole 128-byte lines) where they are larger than these (stage_flags): 401 -> 324 us at 512 x 512;
@@ -179,6 +179,8 @@ traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side
 //  - the own traces of a side with a record loaded with the tile, not formed again from its lines:
 //    23 x 23, N = 4 with walls, inflow and outflow 5.8 us instead of 6.7 us, 48 x 48, N = 16: 16.6 us
 //    instead of 19.2 us;
+//  - what the geometry reads after the contractions (side codes, the line's coordinate) loaded with the
+//    tile: 256 x 256, N = 12 in 182 us instead of 188 us, 512 x 512 in 317 us instead of 320 us;
 //  - no branch inside the line loops and no wait among the loads (a condition on the field in a loop
 //    kept each LDS read from overlapping the next: 3,700 cycles for the update of a line, 1,700 now);
 //  - five barriers instead of six, LDS for five workgroups a CU instead of four.
@@ -375,6 +377,8 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
         const int item = tid + it * T;
         code[it] = item < n_pt ? side_nb[e0 * 4 + item / NF] : INT32_MIN;
     }
+    const int32_t side_code = side_nb[(e0 + el) * 4 + min(l, 3)];  // of the side this thread forms in wave 2
+    const double x_l = x[l];
     // The RK register lives only within a step (the first stage writes it without reading it), so
     // its layout is the kernel's own: within the workgroup's tile it is stored as [f][j / 2][el][i][j % 2]
     // (an odd last j by itself), so that the row owners of all the tile's elements read and write two
@@ -501,7 +505,6 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
     // the Jacobian of a bilinear element is linear in eta along the thread's eta line: jac_m + jac_d eta
     double jac_m, jac_d;
     {
-        const double x_l = x[fresh(l)];
         const double xeta = ((P[6] - P[0]) + (P[4] - P[2]) + ((P[4] - P[2]) - (P[6] - P[0])) * x_l) / 4;
         const double yeta = ((P[7] - P[1]) + (P[5] - P[3]) + ((P[5] - P[3]) - (P[7] - P[1])) * x_l) / 4;
         jac_m = (((P[4] - P[6]) + (P[2] - P[0])) * yeta - xeta * ((P[5] - P[7]) + (P[3] - P[1]))) / 4;
@@ -522,7 +525,7 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
         for (int s = l; s < 4; s += NF) {
             double *sd = s_side + (el * 4 + s) * 3;
             sd[2] = side_geometry(P, s, sd[0], sd[1]);
-            if (const int32_t cd = side_nb[(e0 + el) * 4 + s]; cd < 0) {
+            if (const int32_t cd = s == l ? side_code : side_nb[(e0 + el) * 4 + s]; cd < 0) {
                 const BcSide &rec = bc[-1 - cd];
                 sd[0] = rec.nx;
                 sd[1] = rec.ny;
