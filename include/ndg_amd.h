@@ -325,6 +325,10 @@ ndg_status ndg_mesh_set_graph(ndg_mesh *mesh, int32_t mode);
  * No reference counterpart (the reference launches every element kernel with 32 threads per
  * block, include/solvers/Solver2D_t.tcu:45-52). */
 ndg_status ndg_mesh_autotune(ndg_mesh *mesh, int32_t repeats);
+/* Sets the launch shape of one order group for the current precision: elements per workgroup (1 to the
+ * order's maximum; the FP32 form takes the maximum only) and the block order flag, as ndg_mesh_tuning
+ * reports them. The results do not depend on it. No reference counterpart. */
+ndg_status ndg_mesh_set_tuning(ndg_mesh *mesh, int32_t order, int32_t epb, int32_t remap);
 /* The launch shape in use per order group (ascending N): orders, elements per workgroup, block
  * order flag. Any output may be NULL; *n_groups receives the group count. */
 ndg_status ndg_mesh_tuning(const ndg_mesh *mesh, int32_t *orders, int32_t *epb, int32_t *remap,

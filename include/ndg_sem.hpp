@@ -376,6 +376,8 @@ class Mesh2D_t {
     void set_graph(int32_t mode) { check(ndg_mesh_set_graph(handle_, mode)); }
     // Times the launch shapes of each order group's stage kernel and keeps the fastest.
     void autotune(int32_t repeats = 5) { check(ndg_mesh_autotune(handle_, repeats)); }
+    // Launch shape of one order group: elements per workgroup and the XCD-contiguous block order.
+    void set_tuning(int32_t order, int32_t epb, bool remap) { check(ndg_mesh_set_tuning(handle_, order, epb, remap)); }
     void estimate_error(std::vector<double> &error, std::vector<double> &sigma, std::vector<int32_t> &refine,
                         std::vector<int32_t> &coarsen) {
         error.resize(n_elements_);

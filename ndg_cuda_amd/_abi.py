@@ -39,7 +39,7 @@ EXPORTED = ["ndg_last_error", "ndg_device_count", "ndg_tables_create", "ndg_tabl
             "ndg_mesh_destroy", "ndg_mesh_set_stream", "ndg_mesh_info", "ndg_mesh_set_precision", "ndg_set_ic",
             "ndg_set_state", "ndg_get_state", "ndg_get_solution", "ndg_get_complete_solution", "ndg_get_traces", "ndg_compute_rhs",
             "ndg_get_delta_t", "ndg_step", "ndg_solve", "ndg_solve_output", "ndg_run_steps", "ndg_pre_condition", "ndg_synchronize",
-            "ndg_estimate_error", "ndg_mesh_set_graph", "ndg_mesh_autotune", "ndg_mesh_tuning",
+            "ndg_estimate_error", "ndg_mesh_set_graph", "ndg_mesh_autotune", "ndg_mesh_set_tuning", "ndg_mesh_tuning",
             "ndg_mesh_set_wave_speed", "ndg_record_receivers", "ndg_adjoint_set_store_budget", "ndg_adjoint_set_c_derivative", "ndg_adjoint_gradient", "ndg_apply_rhs_transpose",
             "ndg_adapt", "ndg_mesh_set_adaptivity", "ndg_mesh_orders", "ndg_hilbert_child_order",
             "ndg_hilbert_element_status", "ndg_record_receivers_noalloc", "ndg_mesh_set_adapt_mode",
@@ -143,6 +143,7 @@ def lib():
             "ndg_estimate_error": [vp, vp, vp, vp, vp],
             "ndg_mesh_set_graph": [vp, i32],
             "ndg_mesh_autotune": [vp, i32],
+            "ndg_mesh_set_tuning": [vp, i32, i32, i32],
             "ndg_mesh_tuning": [vp, vp, vp, vp, i32, vp],
             "ndg_mesh_set_wave_speed": [vp, f64],
             "ndg_record_receivers": [vp, vp, f64, i64, vp],

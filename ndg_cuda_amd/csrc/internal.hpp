@@ -399,9 +399,11 @@ hipError_t launch_record(const DeviceMesh &m, const int64_t *elem, const double 
 hipError_t launch_record_rk(const DeviceMesh &m, const int64_t *elem, const double *w_t, int n, double *out,
                             hipStream_t s);
 // Elements per workgroup tile of the FP64 stage kernel for group G (the RK register's tile order),
-// the values of one (field, line index) run of a tile, and the register's size for K elements.
+// the values of one (field, line index) run of a tile (of epb elements: stage_run), and the register's
+// size for K elements, which holds them in tiles of any size.
 int stage_tile_epb(const Group &G);
 int stage_tile_run(const Group &G);
+int stage_run(int N, int epb);
 int64_t stage_rk_values(int N, int64_t K);
 hipError_t launch_source(double *lam, const DeviceMesh &m, const int64_t *elem, const double *w,
                          const double *res, int n, hipStream_t s);

@@ -1840,16 +1840,20 @@ int stage_tile_epb(const Group &G) {
 template <int N>
 static int stage_run_n(int epb) { return rk_run<N>(epb); }
 
-int stage_tile_run(const Group &G) {
-    const int epb = stage_tile_epb(G);
-    switch (G.N) { CASES_1(stage_run_n, epb) }
+int stage_run(int N, int epb) {
+    switch (N) { CASES_1(stage_run_n, epb) }
     return 0;
 }
 
+int stage_tile_run(const Group &G) { return stage_run(G.N, stage_tile_epb(G)); }
+
+// Enough for every tile size a launch may take: a last tile with few elements is as long as a full one,
+// so that for few elements neither the largest size nor the smallest needs the most.
 template <int N>
 static int64_t rk_values_n(int64_t K) {
-    constexpr int EPB = LineShape<N>::EPB;
-    return 3 * (N + 1) * std::max((K + EPB - 1) / EPB * rk_run<N>(EPB), K * (N + 2));
+    int64_t most = 0;
+    for (int epb = 1; epb <= LineShape<N>::EPB; ++epb) most = std::max(most, (K + epb - 1) / epb * rk_run<N>(epb));
+    return 3 * (N + 1) * most;
 }
 
 int64_t stage_rk_values(int N, int64_t K) {

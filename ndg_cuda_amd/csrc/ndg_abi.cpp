@@ -1966,6 +1966,23 @@ extern "C" ndg_status ndg_mesh_autotune(ndg_mesh *mesh, int32_t repeats) {
     return status;
 }
 
+extern "C" ndg_status ndg_mesh_set_tuning(ndg_mesh *mesh, int32_t order, int32_t epb, int32_t remap) {
+    if (!mesh) return fail(NDG_ERR_INVALID, "ndg_mesh_set_tuning: null mesh");
+    DeviceMesh &d = mesh->d;
+    for (Group &G : d.groups) {
+        if (G.N != order) continue;
+        const int emax = stage_max_epb(G.N);
+        if (epb < 1 || epb > emax || (d.precision == NDG_PRECISION_FP32_COMPENSATED && epb != emax))
+            return fail(NDG_ERR_INVALID, "ndg_mesh_set_tuning: elements per workgroup outside the order's range");
+        HIP_TRY(hipStreamSynchronize(mesh->stream), "ndg_mesh_set_tuning sync");
+        drop_graphs(mesh);
+        G.tune[d.precision].epb = epb;
+        G.tune[d.precision].remap = remap != 0;
+        return NDG_OK;
+    }
+    return fail(NDG_ERR_INVALID, "ndg_mesh_set_tuning: no elements of this order");
+}
+
 extern "C" ndg_status ndg_mesh_tuning(const ndg_mesh *mesh, int32_t *orders, int32_t *epb, int32_t *remap,
                                       int32_t capacity, int32_t *n_groups) {
     if (!mesh) return fail(NDG_ERR_INVALID, "ndg_mesh_tuning: null mesh");

@@ -244,6 +244,10 @@ class Mesh2D_t:
         check(lib().ndg_mesh_autotune(self._h, int(repeats)))
         return self.tuning()
 
+    def set_tuning(self, order: int, epb: int, remap: bool):
+        """Sets one order group's launch shape as tuning() reports it (results do not depend on it)."""
+        check(lib().ndg_mesh_set_tuning(self._h, int(order), int(epb), int(remap)))
+
     def tuning(self):
         n = ctypes.c_int32()
         check(lib().ndg_mesh_tuning(self._h, None, None, None, 0, ctypes.byref(n)))
