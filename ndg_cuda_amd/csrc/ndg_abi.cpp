@@ -1741,10 +1741,13 @@ extern "C" ndg_status ndg_get_traces(ndg_mesh *mesh, double *out) {
     ndg_status st = refresh_fp64(mesh);
     if (st != NDG_OK) return st;
     const DeviceMesh &d = mesh->d;
-    // the steps keep the three traces of the sides that need them only
-    if (d.precision == NDG_PRECISION_FP64) HIP_TRY(launch_traces(d, mesh->stream), "traces kernel");
+    // The steps keep the three traces of the sides that need them only. They are formed in the buffer that the
+    // next stage writes, so that the one it reads stays as the last stage left it.
+    DeviceMesh spare = d;
+    spare.cur = 1 - d.cur;
+    HIP_TRY(launch_traces(spare, mesh->stream), "traces kernel");
     mesh->staging.resize((size_t)d.n_tr);
-    HIP_TRY(hipMemcpyAsync(mesh->staging.data(), d.trace[d.cur], sizeof(double) * d.n_tr, hipMemcpyDeviceToHost,
+    HIP_TRY(hipMemcpyAsync(mesh->staging.data(), d.trace[spare.cur], sizeof(double) * d.n_tr, hipMemcpyDeviceToHost,
                            mesh->stream), "download traces");
     HIP_TRY(hipStreamSynchronize(mesh->stream), "ndg_get_traces sync");
     int64_t o = 0;
