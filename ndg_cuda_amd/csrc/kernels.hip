@@ -185,7 +185,9 @@ traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side
 //    kept each LDS read from overlapping the next: 3,700 cycles for the update of a line, 1,700 now);
 //  - five barriers instead of six, LDS for five workgroups a CU instead of four.
 //
-// RHS_ONLY writes G (the compute_dg_wave_derivative output) and leaves the state alone. flags:
+// RHS_ONLY writes G (the compute_dg_wave_derivative output) and leaves the state alone. MORTAR: the mesh may
+// have mortar sides, whose own flux components P2 takes. Meshes without have a kernel without: 128 x 128,
+// N = 8 in 24.3 us instead of 25.3 us, 256 x 256, N = 7 in 68.8 us instead of 69.3 us. flags:
 // kRkFirst, the step's first stage (a = 0: the RK register is not read); kRkLast, the step's last
 // stage, whose RK register no one reads (the next step's first stage overwrites it), so it is not
 // stored.
@@ -274,16 +276,17 @@ struct SideRecord {
 };
 
 // (w_L - w_R)/2 and (w_L + w_R)/2 of point k of side s with a record: a boundary ghost (Mesh2D_t.cpp:
-// 4298-4730), a mortar side (the projected flux, already times the edge Jacobian: the side's scale
-// is 1 then) or a periodic side of another direction. The normal is the record's, tr the side's own
-// traces.
-template <int N>
+// 4298-4730), a periodic side of another direction, or a mortar side, which has the three components of
+// its projected flux instead, already times the edge Jacobian: its faces may lie off the side's line by
+// what the topology allows. The normal is the record's, tr the side's own traces.
+template <int N, bool MORTAR>
 __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide *bc, const double (&tr)[3],
                                             const double *x, const double *tr_in, const double *side_flux, int k,
-                                            const StageClock &clock, double cw, double &fa, double &fb) {
+                                            const StageClock &clock, double cw, double &fa, double &fb,
+                                            double &fc) {
     constexpr int NF = N + 1;
     constexpr double c = kWaveSpeed;
-    if (rec.kind == kKindMortar) {  // projected by the mortar kernel (already x sf)
+    if (MORTAR && rec.kind == kKindMortar) {  // projected by the mortar kernel (already x sf)
         const double *sfl = side_flux + rec.slot + k;
         double f0 = sfl[0], f1 = sfl[NF], f2 = sfl[2 * NF];
         for (int m = 1; m < rec.n_faces; ++m) {  // a side covered by several faces
@@ -293,7 +296,8 @@ __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide 
             f2 += s2[2 * NF];
         }
         fa = f0;
-        fb = f1 * rec.nx + f2 * rec.ny;
+        fb = f1;
+        fc = f2;
         return;
     }
     const double pL = tr[0], uL = tr[1], vL = tr[2];
@@ -328,10 +332,20 @@ __device__ __forceinline__ void record_flux(const SideRecord &rec, const BcSide 
     fb = (wL + wR) / 2;
 }
 
+// The mortar sides' third flux component has a place of its own in LDS, but at N = 7, 8, where it would leave
+// room for four workgroups a CU instead of five: there it lies in the d_xi tile, at the price of a barrier
+// (160 x 160 of orders 4 to 12: 50.3 us a stage, 51.1 us with the barrier at every order).
 template <int N>
-constexpr int stage_lds() { return LineShape<N>::EPB * 6 * StageTile<N>::NEP + StageTile<N>::kFlux + LineShape<N>::EPB * 12; }
+constexpr bool kOwnFluxPlace = N != 7 && N != 8;
+template <int N>
+constexpr int flux_place() { return kOwnFluxPlace<N> ? LineShape<N>::EPB * 4 * (N + 1) : 0; }
 
-template <int N, bool RHS_ONLY>
+template <int N>
+constexpr int stage_lds() {
+    return LineShape<N>::EPB * 6 * StageTile<N>::NEP + StageTile<N>::kFlux + LineShape<N>::EPB * 12 + flux_place<N>();
+}
+
+template <int N, bool RHS_ONLY, bool MORTAR>
 __device__ __forceinline__ void
 stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
            const BcSide *__restrict__ bc, const double *__restrict__ tab,
@@ -342,15 +356,16 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
            double *__restrict__ s_q,     // the state tile
            double *__restrict__ s_d,     // vertices, then d_xi, then the new traces on sides 1 and 3
            double *__restrict__ s_f,     // fluxes, then the new traces on sides 0 and 2
-           double *__restrict__ s_side)  // outward normal and edge Jacobian per side
+           double *__restrict__ s_side,  // outward normal and edge Jacobian (negative: a mortar side) per side
+           double *__restrict__ s_place) // flux_place values
 {
     const bool first = flags & kRkFirst, store_g = !(flags & kRkLast), once = flags & kStream;
     using S = LineShape<N>;
     using L = StageTile<N>;
     constexpr int NF = S::NF, NE = S::NE, EPB = S::EPB, T = S::T, FPT = S::FPT, NFP = L::NFP, NEP = L::NEP;
     constexpr double c = kWaveSpeed;
-    double *const s_v = s_d;
-    static_assert(EPB * 8 <= EPB * 3 * NEP, "the vertices fit the tile they share");
+    double *const s_v = s_d, *const s_fc = kOwnFluxPlace<N> ? s_place : s_d + EPB * 8;
+    static_assert(EPB * (kOwnFluxPlace<N> ? 8 : 8 + 4 * NF) <= EPB * 3 * NEP, "what shares the tile fits it");
     const double *lm = tab + NF * NF;
     const double *lp = lm + NF;
     const double *x = lp + 2 * NF;
@@ -461,8 +476,8 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
         if (with_record[it]) {  // skipped by a wave without
             const int item = tid + it * T;
             if (code[it] >= 0 || code[it] == INT32_MIN) continue;
-            record_flux<N>(rec[it], bc + (-1 - code[it]), tr[it], x, tr_in, side_flux, item % NF, clock, cw, s_f[item],
-                           s_f[EPB * 4 * NF + item]);
+            record_flux<N, MORTAR>(rec[it], bc + (-1 - code[it]), tr[it], x, tr_in, side_flux, item % NF, clock, cw, s_f[item],
+                           s_f[EPB * 4 * NF + item], s_fc[item]);
         }
 
     // P1. Metric lines from the vertices (include/functions/quad_metrics.tpp:3-8): x_eta, y_eta
@@ -529,22 +544,37 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
                 const BcSide &rec = bc[-1 - cd];
                 sd[0] = rec.nx;
                 sd[1] = rec.ny;
-                if (rec.kind == kKindMortar) sd[2] = 1.0;
+                if (MORTAR && rec.kind == kKindMortar) sd[2] = -1.0;
             }
         }
     __syncthreads();
 
     // P2. Lifts: the thread's column j = l of d_xi and row i = l of d_eta. The flux of field f at a
     // side point is (w_L - w_R)/2 (p) or the normal's component times (w_L + w_R)/2 (u, v), times
-    // the edge Jacobian.
+    // the edge Jacobian, and the field's own component on a mortar side.
     {
         const double *side = s_side + el * 12;
         const double *fl = s_f + (f == 0 ? 0 : EPB * 4 * NF) + el * 4 * NF;
         const double v1 = fl[NF + l], v3 = fl[3 * NF + N - l], v2 = fl[2 * NF + N - l], v0 = fl[l];
         const double *n = side + (f == 2 ? 1 : 0);
         const double n0 = f ? n[0] : 1.0, n1 = f ? n[3] : 1.0, n2 = f ? n[6] : 1.0, n3 = f ? n[9] : 1.0;
-        const double Fr = (n1 * v1) * side[5], Fl = (n3 * v3) * side[11], Ft = (n2 * v2) * side[8],
-                     Fb = (n0 * v0) * side[2];
+        double Fr = (n1 * v1) * side[5], Fl = (n3 * v3) * side[11], Ft = (n2 * v2) * side[8], Fb = (n0 * v0) * side[2];
+        if (MORTAR) {
+            const double *own = f == 2 ? s_fc + el * 4 * NF : fl;
+            if (kOwnFluxPlace<N>) {
+                const double o1 = own[NF + l], o3 = own[3 * NF + N - l], o2 = own[2 * NF + N - l], o0 = own[l];
+                Fr = side[5] < 0.0 ? o1 : Fr;
+                Fl = side[11] < 0.0 ? o3 : Fl;
+                Ft = side[8] < 0.0 ? o2 : Ft;
+                Fb = side[2] < 0.0 ? o0 : Fb;
+            } else {  // (these reads all at once would spill)
+                if (side[5] < 0.0) Fr = own[NF + l];
+                if (side[11] < 0.0) Fl = own[3 * NF + N - l];
+                if (side[8] < 0.0) Ft = own[2 * NF + N - l];
+                if (side[2] < 0.0) Fb = own[l];
+                __syncthreads();  // d_xi replaces the third components
+            }
+        }
         double *d = s_d + el * 3 * NEP + f * NEP + l;
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
@@ -666,7 +696,7 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
     }
 }
 
-template <int N, bool RHS_ONLY>
+template <int N, bool RHS_ONLY, bool MORTAR>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 4 : N <= 12 ? 3 : 2)))
 stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
              const BcSide *__restrict__ bc, const double *__restrict__ tab,
@@ -676,10 +706,11 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
              double gdt, StageClock clock, int epb, int remap, double cw) {
     using L = StageTile<N>;
     constexpr int EPB = LineShape<N>::EPB;
-    __shared__ double s_q[EPB * 3 * L::NEP], s_d[EPB * 3 * L::NEP], s_f[L::kFlux], s_side[EPB * 12];
-    stage_tile<N, RHS_ONLY>(verts, side_nb, bc, tab, q, q_out, g, w_in, w_out, tr_in, tr_out, rhs, side_flux, K, flags, a,
+    constexpr int place = MORTAR ? flux_place<N>() : 0;
+    __shared__ double s_q[EPB * 3 * L::NEP], s_d[EPB * 3 * L::NEP], s_f[L::kFlux], s_side[EPB * 12], s_place[place ? place : 1];
+    stage_tile<N, RHS_ONLY, MORTAR>(verts, side_nb, bc, tab, q, q_out, g, w_in, w_out, tr_in, tr_out, rhs, side_flux, K, flags, a,
                             gdt, clock, epb, cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d,
-                            s_f, s_side);
+                            s_f, s_side, s_place);
 }
 
 // The stages of several order groups in one launch: the workgroups of group i are [first[i], first[i + 1]). Small
@@ -733,10 +764,11 @@ stage_groups_kernel(StageGroups groups, const double *__restrict__ verts, const 
     run_group<Top>(groups, [&](auto order, const StageGroups::Part &G, int64_t blk) {
         constexpr int N = decltype(order)::value;
         constexpr int EPB = LineShape<N>::EPB, tile = EPB * 3 * StageTile<N>::NEP;
-        stage_tile<N, false>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, q + G.q_off, q_out + G.q_off,
+        stage_tile<N, false, true>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, q + G.q_off, q_out + G.q_off,
                              g + G.g_off, w_in + G.tr_off / 3, w_out + G.tr_off / 3, tr_in + G.tr_off,
                              tr_out + G.tr_off, nullptr, side_flux, G.K, flags, a, gdt, clock, G.epb, cw, blk, mem,
-                             mem + tile, mem + 2 * tile, mem + 2 * tile + StageTile<N>::kFlux);
+                             mem + tile, mem + 2 * tile, mem + 2 * tile + StageTile<N>::kFlux,
+                             mem + 2 * tile + StageTile<N>::kFlux + EPB * 12);
     });
 }
 
@@ -1887,7 +1919,8 @@ static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, do
     using S = LineShape<N>;
     const int epb = group_epb<N>(G, NDG_PRECISION_FP64);
     const int64_t blocks = (G.K + epb - 1) / epb;
-    hipLaunchKernelGGL((stage_kernel<N, false>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
+    auto *const kernel = m.n_faces ? stage_kernel<N, false, true> : stage_kernel<N, false, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, (m.q_out ? m.q_out : m.q) + G.q_off,
                        m.g + G.g_off, m.wave[m.cur] + G.tr_off / 3, m.wave[1 - m.cur] + G.tr_off / 3,
                        m.trace[m.cur] + G.tr_off,
@@ -1901,7 +1934,7 @@ template <int N>
 static hipError_t rhs_n(DeviceMesh &m, const Group &G, hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    hipLaunchKernelGGL((stage_kernel<N, true>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
+    hipLaunchKernelGGL((stage_kernel<N, true, true>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.q + G.q_off, nullptr,
                        m.wave[m.cur] + G.tr_off / 3, nullptr, m.trace[m.cur] + G.tr_off, nullptr, m.rhs + G.q_off, m.side_flux,
                        G.K, stage_flags(m), 0.0, 0.0,
