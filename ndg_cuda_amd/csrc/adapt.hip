@@ -644,7 +644,12 @@ __device__ void side_roles(const LogicalMesh &L, int64_t t, bool &mortar, bool &
     const int hk = L.hang[t];
     const bool other = l >= 0 && L.order[l / 4] != L.order[k];
     mortar = hk != 0 || other;
-    oblique = !mortar && L.periodic[t] == kPeriodicOblique;
+    oblique = false;
+    if (!mortar && L.periodic[t]) {
+        const v2 a0 = corner(L, k, (int)(t % 4)), a1 = corner(L, k, (int)(t % 4) + 1);
+        const v2 b0 = corner(L, l / 4, (int)(l % 4)), b1 = corner(L, l / 4, (int)(l % 4) + 1);
+        oblique = !opposite_sides(a1.x - a0.x, a1.y - a0.y, b1.x - b0.x, b1.y - b0.y);
+    }
     if (L.periodic[t]) owned = mortar ? (hk == 2 ? chain_length(L, t) : 1) : 0;
     else owned = hk == 1 || (hk == 0 && other && l / 4 > k);
 }

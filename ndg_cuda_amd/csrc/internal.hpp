@@ -49,14 +49,13 @@ constexpr int32_t kKindMortar = 100;
 // characteristic is not this side's incoming one, so its three traces are read (`slot`: their
 // offset in the group's slice of the trace buffer).
 constexpr int32_t kKindTrace = 101;
-// Values of LogicalMesh::periodic (and the host topology's): no, yes, and such a side.
-constexpr int8_t kPeriodic = 1, kPeriodicOblique = 2;
-// Whether the side a0 -> a1 runs against the side b0 -> b1 (their normals are opposite) to rounding:
-// coordinates of size X carry errors of about 1e-16 X, so an edge of length len has a direction
-// good to 1e-16 X / len.
+// Whether the outward normals of the sides along a and b, run in the same sense around their elements, are
+// opposite to the last bit or two (2^-51). Sides further from parallel exchange their traces: a
+// characteristic is formed with its element's normal, so what the receiver's differs by is lost.
 __host__ __device__ inline bool opposite_sides(double ax, double ay, double bx, double by) {
+#pragma clang fp contract(off)
     const double la = sqrt(ax * ax + ay * ay), lb = sqrt(bx * bx + by * by);
-    return fabs(ax / la + bx / lb) <= 1e-12 && fabs(ay / la + by / lb) <= 1e-12;
+    return fabs(ax / la + bx / lb) <= 4.5e-16 && fabs(ay / la + by / lb) <= 4.5e-16;
 }
 
 // One non-conforming face (src/meshes/Mesh2D_t.cpp:3803-4006). L is the element

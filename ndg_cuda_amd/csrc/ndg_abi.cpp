@@ -607,6 +607,13 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
     std::vector<int64_t> mortar_rec((size_t)(4 * K), -1);
     std::vector<int64_t> partners;  // sides whose three traces are read
     int64_t n_slot = 0;
+    auto oblique = [&](int64_t es) {
+        if (!periodic_link[es]) return false;
+        const int64_t l = link[es];
+        const v2 a0 = corner(es / 4, (int)(es % 4)), a1 = corner(es / 4, (int)(es % 4) + 1);
+        const v2 b0 = corner(l / 4, (int)(l % 4)), b1 = corner(l / 4, (int)(l % 4) + 1);
+        return !opposite_sides(a1.x - a0.x, a1.y - a0.y, b1.x - b0.x, b1.y - b0.y);
+    };
     auto add_record = [&](int64_t es, int32_t kind) -> BcSide & {
         BcSide rec{};
         rec.kind = kind;
@@ -672,7 +679,7 @@ ndg_status build_device(ndg_mesh *m, const std::vector<int32_t> &order, DeviceMe
                 continue;
             }
             if (hk == 2) continue;  // built from its small sides
-            if (l >= 0 && hk == 0 && order[l / 4] == order[e] && periodic_link[es] == kPeriodicOblique) {
+            if (l >= 0 && hk == 0 && order[l / 4] == order[e] && oblique(es)) {
                 BcSide &rec = add_record(es, kKindTrace);
                 rec.slot = trace_at(l / 4, (int)(l % 4)) - group_of(l / 4).tr_off;
                 rec.partner = local_of(l / 4) * 4 + l % 4;
@@ -1076,7 +1083,7 @@ ndg_status build_topology(const HostMesh &h, Topology &t) {
             // unchanged (and takes the donor element's order), so the side couples to the donor
             // element side directly.
             link[es] = bar_side[d];
-            periodic_link[es] = kPeriodic;
+            periodic_link[es] = 1;
             continue;
         }
         if (kind < NDG_BC_NONE || kind > NDG_BC_OUTFLOW) return fail(NDG_ERR_INVALID, "mesh topology: unknown boundary kind");
@@ -1232,11 +1239,6 @@ ndg_status build_topology(const HostMesh &h, Topology &t) {
     for (int64_t es = 0; es < 4 * K; ++es)
         if (link[es] == INT64_MIN)
             return fail(NDG_ERR_INVALID, "mesh topology: element side has neither a neighbour nor a boundary bar");
-    for (int64_t es = 0; es < 4 * K; ++es) {
-        if (!periodic_link[es]) continue;
-        const v2 a0 = P(h.quads[es]), a1 = P(end_node(es)), b0 = P(h.quads[link[es]]), b1 = P(end_node(link[es]));
-        if (!opposite_sides(a1.x - a0.x, a1.y - a0.y, b1.x - b0.x, b1.y - b0.y)) periodic_link[es] = kPeriodicOblique;
-    }
     return NDG_OK;
 }
 
@@ -2669,7 +2671,7 @@ extern "C" ndg_status ndg_mesh_sides(ndg_mesh *mesh, int64_t *link, int8_t *hang
         if (link) link[i] = mesh->link[i];
         if (hang) hang[i] = (int8_t)mesh->hang_kind[i];
         if (next_small) next_small[i] = mesh->hang_second[i];
-        if (periodic) periodic[i] = (int8_t)(mesh->periodic_link[i] != 0);
+        if (periodic) periodic[i] = (int8_t)mesh->periodic_link[i];
         if (span) span[i] = mesh->span[i];
     }
     return NDG_OK;

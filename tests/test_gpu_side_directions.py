@@ -9,7 +9,7 @@ import pytest
 import ndg_cuda_amd as nd
 from meshes import split_elements
 from oracle import oracle as O
-from test_gpu_stage_exchange import grid
+from test_gpu_stage_exchange import PULSES, grid
 
 
 def rhs_of(desc, N, top):
@@ -56,3 +56,43 @@ def test_hanging_faces_off_the_side(N, more):
     gm, got, want = rhs_of(desc, N, N + max(more, default=0))
     for name, g, r in zip("puv", got, want):
         assert np.max(np.abs(g - r)) <= 4e-14 * np.max(np.abs(r)), name
+
+
+def nearly_periodic(n, turn, seed):
+    """An n x n mesh of translated periodic pairs; the inner nodes of the bottom and left boundary moved off it so
+    that the pairs are out of parallel by about `turn`."""
+    d = grid(n, n, nd.BC_PERIODIC, 0.1)
+    k = np.arange(n)
+    for s in range(4):
+        d.bar_donor[n * s + k] = n * ((s + 2) % 4) + k
+    rng = np.random.default_rng(seed)
+    for axis in (0, 1):  # across the side at coordinate -1 of the axis
+        on = np.flatnonzero((d.xy[:, axis] == -1) & (np.abs(d.xy[:, 1 - axis]) < 0.99))
+        d.xy[on, axis] += rng.choice([-0.5, 0.5], len(on)) * turn * 2 / n
+    return d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("turn", [0.8e-12, 1e-13, 0.0])
+@pytest.mark.parametrize("N", [1, 2, 5, 8])
+def test_periodic_pairs_out_of_parallel(N, turn):
+    gm, got, want = rhs_of(nearly_periodic(6, turn, 3), N, N)
+    for name, g, r in zip("puv", got, want):
+        assert np.max(np.abs(g - r)) <= 4e-14 * np.max(np.abs(r)), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["device", "host"])
+def test_periodic_pairs_out_of_parallel_through_an_adaptation(mode):
+    """Both rebuilds judge the new sides by their own vertices, as a mesh made of them does."""
+    desc = nearly_periodic(4, 0.8e-12, 4)
+    ndg = nd.NDG_t(8, 5)
+    gm = nd.Mesh2D_t(desc, 4, 8, 5, 0, 0, 0, 1e-3, 1e-14, 0.0, ndg)
+    gm.initial_conditions(PULSES)
+    gm.set_adapt_mode(mode)
+    assert gm.adapt(8, 0) > 0
+    desc.quad_N = gm.orders_.copy()
+    ref = nd.Mesh2D_t(desc, 4, 8, 5, 0, 0, 0, 1e-3, 1e-14, 0.0, ndg)
+    ref.set_solution(*gm.get_solution())
+    for g, r in zip(gm.compute_rhs(0.0), ref.compute_rhs(0.0)):
+        assert np.array_equal(g, r)
