@@ -36,10 +36,10 @@ struct BcSide {
 
 // Stage kernel flags: the step's first stage (the RK register is not read), its last stage, the
 // three traces written for every side (see DeviceMesh::trace_all), and the state and RK register
-// streamed past the caches (where together they have more than kStreamBytes).
+// streamed past the caches (where a stage has more bytes than kStreamBytes).
 constexpr int kRkFirst = 1, kRkLast = 2, kTraceAll = 4, kStream = 8;
 constexpr int kRhsClock = 2;
-constexpr int64_t kStreamBytes = int64_t(160) << 20;
+constexpr int64_t kStreamBytes[2] = {232000000, 242000000};  // NDG_PRECISION_*
 
 // Element side whose face is non-conforming: its element flux trace is produced by the mortar
 // kernel (interpolation to the face, flux, L2 projection back) before the stage kernels run.

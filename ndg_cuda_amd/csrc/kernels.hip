@@ -1893,12 +1893,21 @@ int64_t stage_rk_values(int N, int64_t K) {
     return 0;
 }
 
-// The state and the RK register go past the caches when they are far larger than these (the
-// last-level cache holds 256 MB), so that they leave room for what is read again. At N = 8, past and
-// through the caches: 512 x 512 (1 GB) 324 and 401 us a launch, 256 x 256 (255 MB) 85.8 and 91.1,
-// 192 x 192 (143 MB) 51.2 and 45.2, 160 x 160 (100 MB) 37.3 and 33.8.
-static int stage_flags(const DeviceMesh &m) {
-    return (m.trace_all ? kTraceAll : 0) | (16 * m.n_q > kStreamBytes ? kStream : 0);
+// The state and the RK register go past the caches when a stage's bytes (these, both buffers of
+// characteristics, vertices and codes) no longer fit the last-level cache of 256 MB from one stage to the
+// next, so that they leave room for what is read again. Measured, us a stage past and through the caches,
+// FP64: N = 8: 200 x 200 (182 MB) 55.4 and 48.8, 216 x 216 (212 MB) 60.9 and 55.4, 232 x 232 (245 MB) 71.6
+// and 64.3, 248 x 248 (279 MB) 79.5 and 78.2, 264 x 264 (317 MB) 92.0 and 92.7, 512 x 512 (1.2 GB) 324 and
+// 401; N = 12: 160 x 160 (231 MB) 76.1 and 67.9; N = 4: 360 x 360 (207 MB) 60.4 and 55.7, 384 x 384 (236 MB)
+// 67.6 and 74.4, 400 x 400 (256 MB) 74.1 and 80.5; N = 2: 580 x 580 (237 MB) 73.0 and 66.8; N = 6: 288 x 288
+// (239 MB) 68.1 and 71.0. The FP32 form: N = 8: 224 x 224 (165 MB) 58.1 and 52.5, 256 x 256 (215 MB) 80.4 and
+// 65.7, 264 x 264 (229 MB) 87.5 and 70.7, 272 x 272 (243 MB) 89.1 and 91.7, 288 x 288 (272 MB) 99.7 and 108,
+// 512 x 512 (861 MB) 271 and 287; N = 12: 184 x 184 (223 MB) 84.8 and 76.9, 192 x 192 (243 MB) 96.8 and 95.4;
+// N = 4: 460 x 460 (241 MB) 84.7 and 72.9, 480 x 480 (263 MB) 89.6 and 98.4.
+static int stage_flags(const DeviceMesh &m, int precision) {
+    const bool c32 = precision == NDG_PRECISION_FP32_COMPENSATED;
+    const int64_t bytes = (c32 ? 12 : 16) * m.n_q + (c32 ? 8 : 16) * (m.n_tr / 3) + 80 * m.K;
+    return (m.trace_all ? kTraceAll : 0) | (bytes > kStreamBytes[precision] ? kStream : 0);
 }
 
 // The clock has a start time for each trace buffer that a step can begin with: three stages flip it
@@ -1911,7 +1920,7 @@ static StageClock stage_clock(const DeviceMesh &m, const Group &G, int stage, do
 }
 
 static int stage_rk_flags(const DeviceMesh &m, int stage) {
-    return (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0) | stage_flags(m);
+    return (stage == 0 ? kRkFirst : 0) | (stage == 2 && !m.keep_last_rk ? kRkLast : 0) | stage_flags(m, NDG_PRECISION_FP64);
 }
 
 template <int N>
@@ -1937,7 +1946,7 @@ static hipError_t rhs_n(DeviceMesh &m, const Group &G, hipStream_t s) {
     hipLaunchKernelGGL((stage_kernel<N, true, true>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.q + G.q_off, nullptr,
                        m.wave[m.cur] + G.tr_off / 3, nullptr, m.trace[m.cur] + G.tr_off, nullptr, m.rhs + G.q_off, m.side_flux,
-                       G.K, stage_flags(m), 0.0, 0.0,
+                       G.K, stage_flags(m, NDG_PRECISION_FP64), 0.0, 0.0,
                        StageClock{m.clock + kRhsClock, 0.0, nullptr, 0.0}, S::EPB, 1, m.wave_speed);
     return hipGetLastError();
 }
@@ -1971,7 +1980,7 @@ static hipError_t traces_c32_n(const DeviceMesh &m, const Group &G, hipStream_t 
 }
 
 static int stage_c32_flags(const DeviceMesh &m, int stage) {
-    return (stage == 0 ? kRkFirst : 0) | (m.trace_all ? kTraceAll : 0) | (12 * m.n_q > kStreamBytes ? kStream : 0);
+    return (stage == 0 ? kRkFirst : 0) | stage_flags(m, NDG_PRECISION_FP32_COMPENSATED);
 }
 
 template <int N>
