@@ -966,13 +966,13 @@ __device__ __forceinline__ void contract32(const LaneTable32<NF * NF> &D, const 
 }
 
 // record_flux in FP32: (w_L - w_R)/2, (w_L + w_R)/2 and, for a mortar side, the three flux components.
-template <int N>
+template <int N, bool MORTAR>
 __device__ __forceinline__ void record_flux32(const SideRecord &rec, const BcSide *bc, const float (&tr)[3],
                                               const double *x64, const float *tr_in, const float *side_flux, int k,
                                               const StageClock &clock, double cw, float &fa, float &fb, float &fc) {
     constexpr int NF = N + 1;
     const int kind = rec.kind;
-    if (kind == kKindMortar) {
+    if (MORTAR && kind == kKindMortar) {
         const float *sfl = side_flux + bc->slot + k;
         float f0 = sfl[0], f1 = sfl[NF], f2 = sfl[2 * NF];
         const int n_faces = bc->n_faces;
@@ -1030,12 +1030,13 @@ __device__ __forceinline__ void record_flux32(const SideRecord &rec, const BcSid
 // RK register's tile order of the shape's full tiles (the launch always uses them, so the low words
 // keep their places from one step to the next). A side with a record reads its own traces back, loaded
 // with the tile; formed again from the tile's lines they cost a wall mesh of 96 x 96, N = 8 0.4 us.
-// Bound by memory at large sizes: 384 x 384, N = 7 in 127 us a launch, 157 us with three traces
-// exchanged a point, 4-byte cached accesses and D^ in scalar registers; 512 x 512, N = 8: 297 and
-// 350 us; 256 x 256, N = 12: 169 and 182 us; 48 x 48, N = 16: 16.4 and 18.2 us. Where one round of
-// workgroups fills the chip the wait for the tile decides: 128 x 128, N = 8: 23.6 and 24.1 us, 96 x 96:
-// 14.1 and 13.9 us.
-template <int N>
+// Bound by memory at large sizes: 384 x 384, N = 7 in 126 us a launch, 157 us with three traces
+// exchanged a point, 4-byte cached accesses and D^ in scalar registers; 512 x 512, N = 8: 293 and
+// 350 us; 256 x 256, N = 12: 170 and 186 us; 48 x 48, N = 16: 16.1 and 18.1 us. Where one round of
+// workgroups fills the chip the wait for the tile decides: 128 x 128, N = 8: 22.7 and 24.2 us, 96 x 96:
+// 13.6 and 13.7 us. There the vertices in 16-byte words and no code for mortar sides on meshes without
+// (MORTAR) count: 14.3 us with eight loads of a coordinate and one kernel for all meshes.
+template <int N, bool MORTAR>
 __device__ __forceinline__ void
 stage_c32_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
                const BcSide *__restrict__ bc, const double *__restrict__ tab64,
@@ -1081,7 +1082,11 @@ stage_c32_tile(const double *__restrict__ verts, const int32_t *__restrict__ sid
     double P[8];  // the element's vertices; in the wave that forms the sides, from side l's first one on
     const int side = min(l, 3);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) P[k] = verts[(e0 + el) * 8 + (f == 2 ? (2 * side + k) & 7 : k)];
+    for (int k = 0; k < 4; ++k) {
+        const double2 v = ((const double2 *)verts)[(e0 + el) * 4 + (f == 2 ? (side + k) & 3 : k)];
+        P[2 * k] = v.x;
+        P[2 * k + 1] = v.y;
+    }
     const int32_t side_code = side_nb[(e0 + el) * 4 + side];
     const float *qg = qh + e0 * 3 * NE;
     const int lead = (int)(((uintptr_t)qg >> 2) & 31), end = lead + n_val;
@@ -1164,7 +1169,7 @@ stage_c32_tile(const double *__restrict__ verts, const int32_t *__restrict__ sid
                 const BcSide &r = bc[-1 - cd];
                 nx = r.nx;
                 ny = r.ny;
-                if (r.kind == kKindMortar) sf = -1.f;
+                if (MORTAR && r.kind == kKindMortar) sf = -1.f;
             }
             float *sd = s_side + (el * 4 + s) * 3;
             sd[0] = (float)nx;
@@ -1178,7 +1183,7 @@ stage_c32_tile(const double *__restrict__ verts, const int32_t *__restrict__ sid
         if (with_record[it]) {  // skipped by a wave without
             const int item = tid + it * T;
             if (code[it] >= 0 || code[it] == INT32_MIN) continue;
-            record_flux32<N>(rec[it], bc + (-1 - code[it]), tr[it], x64, tr_in, side_flux, item % NF, clock, cw,
+            record_flux32<N, MORTAR>(rec[it], bc + (-1 - code[it]), tr[it], x64, tr_in, side_flux, item % NF, clock, cw,
                              s_f[item], s_f[EPB * 4 * NF + item], s_f[EPB * 8 * NF + item]);
         }
 
@@ -1237,7 +1242,7 @@ stage_c32_tile(const double *__restrict__ verts, const int32_t *__restrict__ sid
         auto flux = [&](int s, int k) {
             const float sf = side[3 * s + 2];
             const float va = fl[(f == 0 ? 0 : EPB * 4 * NF) + s * NF + k];
-            if (sf < 0.f) return fl[f * EPB * 4 * NF + s * NF + k];  // the mortar side's own component
+            if (MORTAR && sf < 0.f) return fl[f * EPB * 4 * NF + s * NF + k];  // the mortar side's own component
             return f == 0 ? va * sf : (side[3 * s + (f == 2 ? 1 : 0)] * va) * sf;
         };
         const float Fr = flux(1, l), Fl = flux(3, N - l), Ft = flux(2, N - l), Fb = flux(0, l);
@@ -1359,7 +1364,7 @@ struct StageTile32 {
                          met = EPB * 4 * NF, side = EPB * 12, lds = 2 * tile + flux + met + side;
 };
 
-template <int N>
+template <int N, bool MORTAR>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 9 ? 5 : 4)))
 stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
                  const BcSide *__restrict__ bc, const double *__restrict__ tab64,
@@ -1369,7 +1374,7 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
                  StageClock clock, int remap, double cw) {
     using L = StageTile32<N>;
     __shared__ float s_q[L::tile], s_d[L::tile], s_f[L::flux], s_met[L::met], s_side[L::side];
-    stage_c32_tile<N>(verts, side_nb, bc, tab64, tab, qh, gl, w_in, w_out, tr_in, tr_out, side_flux, K, flags, a, gdt, clock,
+    stage_c32_tile<N, MORTAR>(verts, side_nb, bc, tab64, tab, qh, gl, w_in, w_out, tr_in, tr_out, side_flux, K, flags, a, gdt, clock,
                       cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d, s_f, s_met, s_side);
 }
 
@@ -1392,7 +1397,7 @@ stage_c32_groups_kernel(StageGroups groups, const double *__restrict__ verts, co
         constexpr int N = decltype(order)::value;
         using L = StageTile32<N>;
         float *s_f = mem + 2 * L::tile, *s_met = s_f + L::flux;
-        stage_c32_tile<N>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, G.tab32, qh + G.q_off, gl + G.g_off,
+        stage_c32_tile<N, true>(verts + G.e_begin * 8, side_nb + G.e_begin * 4, bc, G.tab, G.tab32, qh + G.q_off, gl + G.g_off,
                           w_in + G.tr_off / 3, w_out + G.tr_off / 3, tr_in + G.tr_off, tr_out + G.tr_off, side_flux,
                           G.K, flags, a, gdt, clock, cw, blk, mem, mem + L::tile, s_f, s_met, s_met + L::met);
     });
@@ -1988,7 +1993,8 @@ static hipError_t stage_c32_n(DeviceMesh &m, const Group &G, int stage, double a
                               hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    hipLaunchKernelGGL(stage_c32_kernel<N>, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
+    auto *const kernel = m.n_faces ? stage_c32_kernel<N, true> : stage_c32_kernel<N, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, G.tab32, m.qh + G.q_off, m.gl32 + G.g_off,
                        m.wave32[m.cur] + G.tr_off / 3, m.wave32[1 - m.cur] + G.tr_off / 3, m.trace32[m.cur] + G.tr_off,
                        m.trace32[1 - m.cur] + G.tr_off, m.side_flux32, G.K, stage_c32_flags(m, stage), (float)a, (float)gdt,
