@@ -77,12 +77,6 @@ struct LaneTable {
     }
 };
 
-// D^ F of a line by even and odd parts: the Gauss nodes are symmetric, so D^[N-i][N-k] = -D^[i][k], and with
-// s_k = F[k] + F[N-k], d_k = F[k] - F[N-k] (k < h = (N+1)/2) and the middle node m of an even order
-//   Q_i = sum_k A[i][k] s_k + D^[i][m] F[m],  P_i = sum_k B[i][k] d_k,  A, B = (D^[i][k] +- D^[i][N-k])/2,
-//   (D^ F)[i] = P_i + Q_i,  (D^ F)[N-i] = P_i - Q_i,  (D^ F)[m] = P_m,
-// about half the multiply-adds and entries of D^. The table holds row by row A[i][.], D^[i][m], B[i][.],
-// then B[m][.].
 // a[i S] += D(entry E + i Step) F for the R rows i: the entry is a DPP operand of the multiply-add (the
 // compiler moves it to a register pair first, with a wait: three issues instead of one). A block first
 // waits out the two cycles that a register written just before it takes to reach a DPP
@@ -117,6 +111,13 @@ __device__ __forceinline__ void rows(const LaneTable<L> &D, double F, double *a)
 #undef NDG_LANE
 }
 
+// D^ F of a line by even and odd parts: the Gauss nodes are symmetric, so D^[N-i][N-k] = -D^[i][k], and with
+// s_k = F[k] + F[N-k], d_k = F[k] - F[N-k] (k < h = (N+1)/2) and the middle node m of an even order
+//   Q_i = sum_k A[i][k] s_k + D^[i][m] F[m],  P_i = sum_k B[i][k] d_k,  A, B = (D^[i][k] +- D^[i][N-k])/2,
+//   (D^ F)[i] = P_i + Q_i,  (D^ F)[N-i] = P_i - Q_i,  (D^ F)[m] = P_m,
+// about half the multiply-adds and entries of D^. The table holds row by row A[i][.], D^[i][m], B[i][.],
+// then B[m][.].
+
 // Q_i (summed in place N - i) and P_i (in place i) of the rows i < h, and P_m, a column at a time:
 // entry c of a row multiplies F[c], s in [0, h), F[m] at h, then d.
 template <int NF, int c = 0>
@@ -128,9 +129,9 @@ __device__ __forceinline__ void even_odd_columns(const LaneTable<even_odd_len(NF
     if constexpr (c + 1 < per) even_odd_columns<NF, c + 1>(D, F, a);
 }
 
-// a = D^ F (F is overwritten).
+// a = D^ F.
 template <int NF>
-__device__ __forceinline__ void contract(const LaneTable<even_odd_len(NF)> &D, double *F, double *a) {
+__device__ __forceinline__ void contract(const LaneTable<even_odd_len(NF)> &D, const double *F, double *a) {
     constexpr int h = NF / 2, odd = NF & 1;
     double t[NF];
 #pragma unroll

@@ -801,8 +801,8 @@ __device__ __forceinline__ int64_t c32_tile_index(int64_t e, int f, int i, int j
 }
 
 // q and qh are in reference node order; gl32 (RK register in x, low state word in y) is in the
-// FP32 stage kernel's tile order. Thread r writes one float2. The RK register carries no value
-// from one step to the next, so g is copied word for word whatever its order.
+// FP32 stage kernel's tile order. Thread r writes one float2. The register's word starts at zero: it
+// carries no value from one step to the next, and a step's first stage does not use what it loads there.
 __global__ void to_c32_kernel(const double *__restrict__ q, float *__restrict__ qh, float2 *__restrict__ gl32,
                               int64_t n, int nf, int epb, int run) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
