@@ -696,7 +696,7 @@ stage_tile(const double *__restrict__ verts, const int32_t *__restrict__ side_nb
     }
 }
 
-template <int N, bool RHS_ONLY, bool MORTAR>
+template <int N, bool RHS_ONLY>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 4 : N <= 12 ? 3 : 2)))
 stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
              const BcSide *__restrict__ bc, const double *__restrict__ tab,
@@ -705,12 +705,29 @@ stage_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_
              double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
              double gdt, StageClock clock, int epb, int remap, double cw) {
     using L = StageTile<N>;
-    constexpr int EPB = LineShape<N>::EPB;
-    constexpr int place = MORTAR ? flux_place<N>() : 0;
+    constexpr int EPB = LineShape<N>::EPB, place = RHS_ONLY ? flux_place<N>() : 0;
     __shared__ double s_q[EPB * 3 * L::NEP], s_d[EPB * 3 * L::NEP], s_f[L::kFlux], s_side[EPB * 12], s_place[place ? place : 1];
-    stage_tile<N, RHS_ONLY, MORTAR>(verts, side_nb, bc, tab, q, q_out, g, w_in, w_out, tr_in, tr_out, rhs, side_flux, K, flags, a,
-                            gdt, clock, epb, cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d,
-                            s_f, s_side, s_place);
+    stage_tile<N, RHS_ONLY, RHS_ONLY>(verts, side_nb, bc, tab, q, q_out, g, w_in, w_out, tr_in, tr_out, rhs, side_flux, K,
+                                      flags, a, gdt, clock, epb, cw,
+                                      remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d, s_f, s_side,
+                                      s_place);
+}
+
+// The stage of a mesh with mortar faces.
+template <int N>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 4 : N <= 12 ? 3 : 2)))
+stage_mortar_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+                    const BcSide *__restrict__ bc, const double *__restrict__ tab,
+                    const double *q, double *q_out, double *__restrict__ g, const double *__restrict__ w_in,
+                    double *__restrict__ w_out, const double *__restrict__ tr_in, double *__restrict__ tr_out,
+                    double *__restrict__ rhs, const double *__restrict__ side_flux, int64_t K, int flags, double a,
+                    double gdt, StageClock clock, int epb, int remap, double cw) {
+    using L = StageTile<N>;
+    constexpr int EPB = LineShape<N>::EPB, place = flux_place<N>();
+    __shared__ double s_q[EPB * 3 * L::NEP], s_d[EPB * 3 * L::NEP], s_f[L::kFlux], s_side[EPB * 12], s_place[place ? place : 1];
+    stage_tile<N, false, true>(verts, side_nb, bc, tab, q, q_out, g, w_in, w_out, tr_in, tr_out, rhs, side_flux, K, flags, a,
+                               gdt, clock, epb, cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d,
+                               s_f, s_side, s_place);
 }
 
 // The stages of several order groups in one launch: the workgroups of group i are [first[i], first[i + 1]). Small
@@ -1364,7 +1381,7 @@ struct StageTile32 {
                          met = EPB * 4 * NF, side = EPB * 12, lds = 2 * tile + flux + met + side;
 };
 
-template <int N, bool MORTAR>
+template <int N>
 __global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 9 ? 5 : 4)))
 stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
                  const BcSide *__restrict__ bc, const double *__restrict__ tab64,
@@ -1374,7 +1391,22 @@ stage_c32_kernel(const double *__restrict__ verts, const int32_t *__restrict__ s
                  StageClock clock, int remap, double cw) {
     using L = StageTile32<N>;
     __shared__ float s_q[L::tile], s_d[L::tile], s_f[L::flux], s_met[L::met], s_side[L::side];
-    stage_c32_tile<N, MORTAR>(verts, side_nb, bc, tab64, tab, qh, gl, w_in, w_out, tr_in, tr_out, side_flux, K, flags, a, gdt, clock,
+    stage_c32_tile<N, false>(verts, side_nb, bc, tab64, tab, qh, gl, w_in, w_out, tr_in, tr_out, side_flux, K, flags, a, gdt, clock,
+                      cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d, s_f, s_met, s_side);
+}
+
+// The stage of a mesh with mortar faces.
+template <int N>
+__global__ void __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(N <= 9 ? 5 : 4)))
+stage_c32_mortar_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side_nb,
+                        const BcSide *__restrict__ bc, const double *__restrict__ tab64,
+                        const float *__restrict__ tab, float *__restrict__ qh, float2 *__restrict__ gl,
+                        const float *__restrict__ w_in, float *__restrict__ w_out, const float *__restrict__ tr_in,
+                        float *__restrict__ tr_out, const float *__restrict__ side_flux, int64_t K, int flags, float a, float gdt,
+                        StageClock clock, int remap, double cw) {
+    using L = StageTile32<N>;
+    __shared__ float s_q[L::tile], s_d[L::tile], s_f[L::flux], s_met[L::met], s_side[L::side];
+    stage_c32_tile<N, true>(verts, side_nb, bc, tab64, tab, qh, gl, w_in, w_out, tr_in, tr_out, side_flux, K, flags, a, gdt, clock,
                       cw, remap ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x, s_q, s_d, s_f, s_met, s_side);
 }
 
@@ -1933,7 +1965,7 @@ static hipError_t stage_n(DeviceMesh &m, const Group &G, int stage, double a, do
     using S = LineShape<N>;
     const int epb = group_epb<N>(G, NDG_PRECISION_FP64);
     const int64_t blocks = (G.K + epb - 1) / epb;
-    auto *const kernel = m.n_faces ? stage_kernel<N, false, true> : stage_kernel<N, false, false>;
+    auto *const kernel = m.n_faces ? stage_mortar_kernel<N> : stage_kernel<N, false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, (m.q_out ? m.q_out : m.q) + G.q_off,
                        m.g + G.g_off, m.wave[m.cur] + G.tr_off / 3, m.wave[1 - m.cur] + G.tr_off / 3,
@@ -1948,7 +1980,7 @@ template <int N>
 static hipError_t rhs_n(DeviceMesh &m, const Group &G, hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    hipLaunchKernelGGL((stage_kernel<N, true, true>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
+    hipLaunchKernelGGL((stage_kernel<N, true>), dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, m.q + G.q_off, m.q + G.q_off, nullptr,
                        m.wave[m.cur] + G.tr_off / 3, nullptr, m.trace[m.cur] + G.tr_off, nullptr, m.rhs + G.q_off, m.side_flux,
                        G.K, stage_flags(m, NDG_PRECISION_FP64), 0.0, 0.0,
@@ -1993,7 +2025,7 @@ static hipError_t stage_c32_n(DeviceMesh &m, const Group &G, int stage, double a
                               hipStream_t s) {
     using S = LineShape<N>;
     const int64_t blocks = (G.K + S::EPB - 1) / S::EPB;
-    auto *const kernel = m.n_faces ? stage_c32_kernel<N, true> : stage_c32_kernel<N, false>;
+    auto *const kernel = m.n_faces ? stage_c32_mortar_kernel<N> : stage_c32_kernel<N>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(S::T), 0, s, m.verts + G.e_begin * 8,
                        m.side_nb + G.e_begin * 4, m.bc, G.tab, G.tab32, m.qh + G.q_off, m.gl32 + G.g_off,
                        m.wave32[m.cur] + G.tr_off / 3, m.wave32[1 - m.cur] + G.tr_off / 3, m.trace32[m.cur] + G.tr_off,
