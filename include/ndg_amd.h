@@ -319,8 +319,9 @@ ndg_status ndg_synchronize(ndg_mesh *mesh);
  * clock that the graph advances, so one graph serves every step of size dt; it is recaptured when
  * dt or the precision changes. No reference counterpart for the mode switch itself. */
 ndg_status ndg_mesh_set_graph(ndg_mesh *mesh, int32_t mode);
-/* Times every candidate launch shape of each order group's stage kernel (elements per workgroup
- * from the shape's maximum down to 1, XCD-contiguous block order on or off) on this mesh, `repeats`
+/* Times the candidate launch shapes of each order group's stage kernel (elements per workgroup: the
+ * shape's maximum, about a half and a quarter of it, and 1; the FP32 form the maximum only;
+ * XCD-contiguous block order on or off) on this mesh, `repeats`
  * launches each, and keeps the fastest for the current precision. The state is left unchanged.
  * No reference counterpart (the reference launches every element kernel with 32 threads per
  * block, include/solvers/Solver2D_t.tcu:45-52). */

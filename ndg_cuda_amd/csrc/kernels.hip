@@ -165,10 +165,10 @@ traces_kernel(const double *__restrict__ verts, const int32_t *__restrict__ side
 // three traces. Elements write the three traces of the sides with a record (and with kTraceAll of
 // every side) for these.
 //
-// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 317 us a
-// launch, 5.95 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches 5.3 to 5.8
-// here); 421 us and 2.18 GB with the traces exchanged. 512 x 512, N = 4: 116 us (164 us before). 128 x
-// 128, N = 8 (in the last-level cache): 24.8 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
+// What bounds it: HBM at large sizes, the phases' latency at small ones. 512 x 512, N = 8: 316 to 323 us a
+// launch over runs, 5.84 to 5.97 TB/s of the 1.89 GB it moves (a plain in-place copy of two streams reaches
+// 5.3 to 5.8 here); 421 us and 2.18 GB with the traces exchanged. 512 x 512, N = 4: 116 us (164 us before). 128 x
+// 128, N = 8 (in the last-level cache): 24.3 us, 33.2 us before; 16 x 16, N = 6 (29 workgroups): 5.7
 // us from launch to launch, 7.0 us before. What made the difference, at N = 8:
 //  - the state and the RK register are streamed past the caches (non-temporal, in 16-byte words on
 //    whole 128-byte lines) where they are larger than these (stage_flags): 401 -> 324 us at 512 x 512;

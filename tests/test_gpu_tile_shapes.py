@@ -39,6 +39,16 @@ def test_one_group(N, K, epb, remap):
     same(run(desc, N, [(N, epb, remap)]), run(desc, N, []))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [1, 3, 8, 11, 16])
+def test_tile_sizes_on_two_and_a_part(N):
+    most = 64 // (N + 1)
+    desc = grid(2 * most + 3, 1, nd.BC_OUTFLOW, jitter=0.0)
+    ref = run(desc, N, [])
+    for epb in sorted({1, 2, (most + 3) // 4, (most + 1) // 2, most - 1, most} - {0}):
+        same(run(desc, N, [(N, epb, epb % 2)]), ref)
+
+
 def mixed(N, K, ones):
     """`ones` elements of order 1, K of order N and, up to the largest order, 3 of order N + 1, whose register lies
     behind that of the K."""
